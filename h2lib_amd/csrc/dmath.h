@@ -2,52 +2,67 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stdint.h>
 
 namespace h2hip {
 
+// sin and cos of |r| <= 0.80: r + r^3 S(r^2) and 1 - r^2/2 + r^4 C(r^2) with
+// S and C of degree 5, the best approximations in the maximum norm on
+// |r| <= 1.02 pi/4 (exchange algorithm of Remez in 60 digits; they miss
+// sin and cos by 2.1e-18 and 6.4e-20 before the coefficients are rounded).
+// Absolute errors 0.35 and 0.43 times 2^-52 (4e6 arguments against
+// long-double sinl / cosl, the same operations in C).
+__device__ __forceinline__ void sincos_poly(double r, double &s, double &c) {
+  const double r2 = r * r;
+  double ps = 1.5881735738984916e-10;
+  ps = fma(ps, r2, -2.5050476368259563e-08);
+  ps = fma(ps, r2, 2.755731170446063e-06);
+  ps = fma(ps, r2, -0.00019841269823307647);
+  ps = fma(ps, r2, 0.0083333333333128);
+  ps = fma(ps, r2, -0.16666666666666582);
+  s = fma(r * r2, ps, r);
+  double pc = -1.1355204972150358e-11;
+  pc = fma(pc, r2, 2.087563880745057e-09);
+  pc = fma(pc, r2, -2.7557313742707853e-07);
+  pc = fma(pc, r2, 2.4801587287420472e-05);
+  pc = fma(pc, r2, -0.0013888888888870916);
+  pc = fma(pc, r2, 0.04166666666666658);
+  pc = fma(pc, r2, -0.5);
+  c = fma(r2, pc, 1.0);
+}
+
 // sin and cos of x: Cody and Waite's reduction by pi/2 in three parts
-// (n = rint(2x / pi), r = x - n pi/2 with fused products) to |r| <= pi/4,
-// then the Taylor polynomials of sin r and cos r to degree 17 and 16 in
-// Horner form (coefficients (-1)^k / k!; the first terms left out are
-// 8.4e-20 and 2.0e-18 at most, at |r| = pi/4).  Absolute error below
-// 0.59 * 2^-52 for |x| < 2^45 (the same operations in C with fma, against
-// long-double sinl / cosl on 4e6 arguments, a quarter of them next to
-// multiples of pi/2); beyond, where k r of a coupling never comes, the
-// error grows with the rounding of 2x / pi; NaN and infinities give NaN.
+// (n the integer next to 2x / pi, r = x - n pi/2 with fused products) to |r| <= pi/4,
+// then sincos_poly (Taylor polynomials of degree 17 and 16, which the code
+// had before, took three operations more for the same error).  Absolute
+// error below 0.59 * 2^-52 for |x| < 2^45 (the same operations in C with
+// fma, against long-double sinl / cosl on 4e6 arguments, a quarter of them
+// next to multiples of pi/2); beyond, where k r of a coupling never comes,
+// the error grows with the rounding of 2x / pi; NaN and infinities give NaN.
 // No branches, so the evaluations of the coupling kernels stay branch-free
 // (the library's sincos carries a large-argument path).
 __device__ __forceinline__ void sincos_cw(double x, double &s, double &c) {
   constexpr double TWO_OVER_PI = 0.6366197723675814;
   constexpr double P1 = 1.5707963267948966, P2 = 6.123233995736766e-17,
                    P3 = -1.4973849048591698e-33;
-  const double n = rint(x * TWO_OVER_PI);
+  // adding 1.5 * 2^52 rounds to an integer and leaves its low bits in the
+  // low mantissa bits (the conversion to a 64-bit integer took eight
+  // operations)
+  constexpr double MAGIC = 6755399441055744.0;
+  const double m = fma(x, TWO_OVER_PI, MAGIC);
+  const double n = m - MAGIC;
   double r = fma(-n, P1, x);
   r = fma(-n, P2, r);
   r = fma(-n, P3, r);
-  const double r2 = r * r;
-  double ps = 1.0 / 355687428096000.0;  // 1 / 17!
-  ps = fma(ps, r2, -1.0 / 1307674368000.0);
-  ps = fma(ps, r2, 1.0 / 6227020800.0);
-  ps = fma(ps, r2, -1.0 / 39916800.0);
-  ps = fma(ps, r2, 1.0 / 362880.0);
-  ps = fma(ps, r2, -1.0 / 5040.0);
-  ps = fma(ps, r2, 1.0 / 120.0);
-  ps = fma(ps, r2, -1.0 / 6.0);
-  const double sr = fma(r * r2, ps, r);
-  double pc = 1.0 / 20922789888000.0;  // 1 / 16!
-  pc = fma(pc, r2, -1.0 / 87178291200.0);
-  pc = fma(pc, r2, 1.0 / 479001600.0);
-  pc = fma(pc, r2, -1.0 / 3628800.0);
-  pc = fma(pc, r2, 1.0 / 40320.0);
-  pc = fma(pc, r2, -1.0 / 720.0);
-  pc = fma(pc, r2, 1.0 / 24.0);
-  pc = fma(pc, r2, -0.5);
-  const double cr = fma(r2, pc, 1.0);
+  double sr, cr;
+  sincos_poly(r, sr, cr);
   // quadrant n mod 4: (sin, cos) = (sr, cr), (cr, -sr), (-sr, -cr), (-cr, sr)
-  const int q = (int)(long long)n & 3;
-  const double s0 = (q & 1) ? cr : sr, c0 = (q & 1) ? sr : cr;
-  s = (q & 2) ? -s0 : s0;
-  c = ((q + 1) & 2) ? -c0 : c0;
+  const uint32_t q = (uint32_t)__builtin_bit_cast(uint64_t, m);
+  const double s0 = (q & 1u) ? cr : sr, c0 = (q & 1u) ? sr : cr;
+  const uint64_t ss = (uint64_t)(q & 2u) << 62,
+                 cs = (uint64_t)((q + 1u) & 2u) << 62;
+  s = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, s0) ^ ss);
+  c = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, c0) ^ cs);
 }
 
 }  // namespace h2hip

@@ -122,7 +122,11 @@ struct Tile {
   // from sbeg, ns[0] identical, then ns[1] edge, then ns[2] vertex pairs
   uint32_t sbeg;
   uint16_t ns[3];
+  // the tile whose rows are this tile's columns and whose columns are its
+  // rows (a diagonal tile: itself), NO_MIRROR if there is none
+  uint32_t mirror;
 };
+constexpr uint32_t NO_MIRROR = 0xffffffffu;
 
 struct Fixup {  // identity term of the cc double layer at (t, t), t != s
   uint64_t pos;
@@ -165,6 +169,11 @@ struct KArgs {
   // grouped by tile, evaluated by the tile's workgroup (nullptr: separate
   // launches per rule class over the class-sorted list)
   const SPair *tlist;
+  // mirrored tiles (nmir != 0): the tiles to run, one of each mirrored pair,
+  // and how many identical and vertex pairs are to be evaluated (they come
+  // first in their class's list)
+  const uint32_t *mirlist;
+  uint32_t nmir, nmain3, nmain1;
 };
 
 // Launches the regular tile kernel over `ntiles` tiles and then (unless
@@ -174,9 +183,18 @@ struct KArgs {
 int launch_laplace(int layer, int rb, int cb, uint32_t q, const KArgs &a,
                    uint32_t ntiles, const SPair *sp, const uint32_t *ncls,
                    hipStream_t stream);
-int launch_helmholtz(int layer, int rb, int cb, uint32_t q, const KArgs &a,
-                     uint32_t ntiles, const SPair *sp, const uint32_t *ncls,
-                     hipStream_t stream);
+int launch_helmholtz_slp(int rb, int cb, uint32_t q, const KArgs &a,
+                         uint32_t ntiles, const SPair *sp,
+                         const uint32_t *ncls, hipStream_t stream);
+int launch_helmholtz_dlp(int rb, int cb, uint32_t q, const KArgs &a,
+                         uint32_t ntiles, const SPair *sp,
+                         const uint32_t *ncls, hipStream_t stream);
+int launch_helmholtz_slp_sp(int rb, int cb, uint32_t q, const KArgs &a,
+                            uint32_t ntiles, const SPair *sp,
+                            const uint32_t *ncls, hipStream_t stream);
+int launch_helmholtz_dlp_sp(int rb, int cb, uint32_t q, const KArgs &a,
+                            uint32_t ntiles, const SPair *sp,
+                            const uint32_t *ncls, hipStream_t stream);
 
 }  // namespace nf
 }  // namespace h2hip
@@ -187,6 +205,7 @@ struct h2hip_surface {
   std::vector<double> x, n, g;
   std::vector<uint32_t> t;
   std::vector<uint32_t> v2t_ptr, v2t;  // triangles of each vertex
+  double hmax = 0.0;                   // longest edge
   h2hip::DevBuf<double> d_x, d_n, d_g;
   h2hip::DevBuf<uint32_t> d_t;
   // data of the L2 projection onto the linear basis, built on first use:
@@ -263,6 +282,11 @@ struct h2hip_nfplan {
   std::vector<h2hip::SPair> spairs;  // sorted by class, identical first
   std::vector<h2hip::SPair> tpairs;  // grouped by tile (Tile::sbeg, ns)
   uint64_t pairs[4] = {0, 0, 0, 0};  // support pairs per class
+  // mirrored tiles (nf::KArgs::mirlist), empty unless every tile has its
+  // mirror
+  std::vector<uint32_t> mirlist;
+  uint32_t nmain[4] = {0, 0, 0, 0};
+  h2hip::DevBuf<uint32_t> d_mirlist;
   h2hip::DevBuf<h2hip::Tile> d_tiles;
   h2hip::DevBuf<h2hip::Supp> d_supp;
   h2hip::DevBuf<h2hip::Fixup> d_fix;

@@ -1,6 +1,6 @@
 // Near-field Galerkin quadrature on gfx950: planning, execution and the
 // C ABI.  The kernels live in nf_device.h (instantiated per kernel family
-// in nf_laplace.hip and nf_helmholtz.hip).
+// in nf_laplace.hip and nf_helmholtz_*.hip).
 //
 // Planning cuts every requested block into tiles of at most 64 x 64 DOFs.
 // A tile lists the support triangles of its rows and of its columns (for
@@ -247,6 +247,48 @@ unsigned plan_threads(uint64_t work) {
   return std::min(16u, hw);
 }
 
+// Sets Tile::mirror and lists one tile of each mirrored pair (in tile order)
+// if every tile has its mirror; otherwise leaves both unset.  key[i]: the
+// positions of the tile's first row and column in the index arrays (~0: no
+// mirror), which with the sizes name its rows and columns.  A tile that
+// occurs more than once, or whose mirror lies at another place in its block
+// (the identity terms depend on it), has no mirror.
+void set_mirrors(std::vector<Tile> &tiles, const std::vector<uint64_t> &key,
+                 std::vector<uint32_t> &list) {
+  const uint32_t n = (uint32_t)tiles.size();
+  uint64_t cap = 16;
+  while (cap < 2 * (uint64_t)n) cap *= 2;
+  std::vector<uint32_t> slot(cap, NO_MIRROR);
+  // open addressing; the first tile of a key keeps the slot
+  auto find = [&](uint64_t k, uint8_t nr, uint8_t nc) -> uint32_t & {
+    uint64_t h = (k + nr * 257u + nc) * 0x9e3779b97f4a7c15ull;
+    for (h = (h ^ h >> 32) & (cap - 1);; h = (h + 1) & (cap - 1)) {
+      uint32_t &s = slot[h];
+      if (s == NO_MIRROR ||
+          (key[s] == k && tiles[s].nr == nr && tiles[s].nc == nc))
+        return s;
+    }
+  };
+  for (uint32_t i = 0; i < n; i++) {
+    if (key[i] == ~0ull) return;
+    uint32_t &s = find(key[i], tiles[i].nr, tiles[i].nc);
+    if (s != NO_MIRROR) return;
+    s = i;
+  }
+  std::vector<uint32_t> mir(n);
+  for (uint32_t i = 0; i < n; i++) {
+    const Tile &T = tiles[i];
+    const uint32_t m = find(key[i] << 32 | key[i] >> 32, T.nc, T.nr);
+    if (m == NO_MIRROR || tiles[m].row0 != T.col0 || tiles[m].col0 != T.row0)
+      return;
+    mir[i] = m;
+  }
+  for (uint32_t i = 0; i < n; i++) {
+    tiles[i].mirror = mir[i];
+    if (i <= mir[i]) list.push_back(i);
+  }
+}
+
 // ntr: per-block ntrans flags (nullptr: ntrans for every block); st: the
 // uploads keep large enough device buffers of P and are ordered on st
 // (otherwise new buffers, complete on return).
@@ -272,6 +314,8 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
   P->d_tiles_f.release();
   P->d_tpairs.release();
   for (auto &c : P->pairs) c = 0;
+  for (auto &c : P->nmain) c = 0;
+  P->mirlist.clear();
   P->s = s;
   P->rb = rb;
   P->cb = cb;
@@ -297,9 +341,16 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
   }
   P->entries = total;
 
+  // Mirrored tiles need one index array (and basis) on both sides
+  const bool mirrors =
+      rb == cb && nridx == ncidx && !ntr && !ntrans &&
+      (ridx_all == cidx_all ||
+       std::memcmp(ridx_all, cidx_all, sizeof(uint32_t) * nridx) == 0);
+
   // ---- tiles and support lists, per range of blocks ----
   struct Part {
     std::vector<Tile> tiles;
+    std::vector<uint64_t> key;  // per tile, see set_mirrors
     std::vector<Supp> supp;
     std::vector<Fixup> fix;
     std::string err;
@@ -402,7 +453,11 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
           // most three columns (Library/bem3d.c:2533 tests a loop variable
           // that equals 3 there).
           T.flags = (cols > 3) ? 1 : 0;
+          T.mirror = NO_MIRROR;
           W.tiles.push_back(T);
+          W.key.push_back(mirrors && !rrep && !crep
+                              ? (uint64_t)(roff + r0) << 32 | (coff + c0)
+                              : ~0ull);
         }
       }
       // cc identity terms the reference leaves at (t, t) with t != s
@@ -450,6 +505,7 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
     }
   });
   std::vector<Tile> tiles;
+  std::vector<uint64_t> tkey;
   for (auto &W : parts) {
     if (!W.err.empty()) {
       set_error(W.err);
@@ -461,6 +517,7 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
       T.csup += base;
     }
     tiles.insert(tiles.end(), W.tiles.begin(), W.tiles.end());
+    tkey.insert(tkey.end(), W.key.begin(), W.key.end());
     P->supp.insert(P->supp.end(), W.supp.begin(), W.supp.end());
     P->fix.insert(P->fix.end(), W.fix.begin(), W.fix.end());
   }
@@ -476,16 +533,32 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
   P->tiles.resize(tiles.size());
   for (size_t i = 0; i < order.size(); i++) P->tiles[i] = tiles[order[i]];
   tiles.clear();
+  if (mirrors) {
+    std::vector<uint64_t> key(order.size());
+    for (size_t i = 0; i < order.size(); i++) key[i] = tkey[order[i]];
+    set_mirrors(P->tiles, key, P->mirlist);
+  }
 
   // ---- pairs with common vertices, found through the vertex-to-triangle
   // map, per range of tiles ----
   struct SPart {
     std::vector<SPair> by_cls[4];
+    size_t nmain[4] = {0, 0, 0, 0};  // pairs to evaluate (mirrored tiles)
     std::vector<SPair> tp;  // grouped by tile
     uint64_t pairs0 = 0;
     std::string err;
   };
   const uint32_t ntiles = (uint32_t)P->tiles.size();
+  const bool mir = !P->mirlist.empty();
+  // whether a pair of mirrored tiles' lists is evaluated for both entries
+  // in this tile: the edge rule is not symmetric, and a constant-basis
+  // triangle meets itself only where its index is repeated or on the
+  // diagonal
+  auto is_main = [&](const SPair &q) {
+    if (q.cls == CLS_EDGE || (q.cls == CLS_IDENTICAL && !rb)) return true;
+    const uint32_t m = P->tiles[q.tile].mirror;
+    return m == q.tile ? (q.cls == CLS_IDENTICAL || q.r < q.c) : q.tile < m;
+  };
   std::vector<SPart> sparts(
       std::max(1u, std::min<unsigned>(plan_threads(P->supp.size()), ntiles)));
   parallel_ranges(ntiles, (unsigned)sparts.size(),
@@ -527,6 +600,7 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
               q.cls =
                   (uint16_t)classify(sr.v, P->supp[T.csup + c].v, q.perm);
               W.by_cls[q.cls].push_back(q);
+              if (mir && is_main(q)) W.nmain[q.cls]++;
             }
           }
         }
@@ -557,7 +631,7 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
   // class lists (identical, edge, vertex) one after the other, each in part
   // order; then the parts copy their pieces at the same time
   const unsigned np = (unsigned)sparts.size();
-  std::vector<size_t> tdst(np), cdst(4 * (size_t)np);
+  std::vector<size_t> tdst(np), cdst(4 * (size_t)np), odst(4 * (size_t)np);
   size_t ntp = 0, nsp = 0;
   for (unsigned part = 0; part < np; part++) {
     tdst[part] = ntp;
@@ -565,11 +639,23 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
     P->pairs[0] += sparts[part].pairs0;
   }
   for (int c = 3; c >= 1; c--) {
-    for (unsigned part = 0; part < np; part++) {
-      cdst[4 * part + c] = nsp;
-      nsp += sparts[part].by_cls[c].size();
-      P->pairs[c] += sparts[part].by_cls[c].size();
+    // mirrored tiles: the pairs to evaluate first, then the others
+    size_t nmain = 0;
+    for (auto &W : sparts) {
+      if (!mir) W.nmain[c] = W.by_cls[c].size();
+      nmain += W.nmain[c];
+      P->pairs[c] += W.by_cls[c].size();
     }
+    size_t other = nsp + nmain;
+    for (unsigned part = 0; part < np; part++) {
+      const SPart &W = sparts[part];
+      cdst[4 * part + c] = nsp;
+      odst[4 * part + c] = other;
+      nsp += W.nmain[c];
+      other += W.by_cls[c].size() - W.nmain[c];
+    }
+    nsp = other;
+    P->nmain[c] = (uint32_t)nmain;
     P->pairs[0] -= P->pairs[c];
   }
   if (ntp > 0xffffffffull) {
@@ -586,9 +672,15 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
       for (uint32_t ti = t0; ti < t1; ti++)
         P->tiles[ti].sbeg += (uint32_t)tdst[part];
       std::copy(W.tp.begin(), W.tp.end(), P->tpairs.begin() + tdst[part]);
-      for (int c = 1; c < 4; c++)
-        std::copy(W.by_cls[c].begin(), W.by_cls[c].end(),
-                  P->spairs.begin() + cdst[4 * part + c]);
+      for (int c = 1; c < 4; c++) {
+        auto first = P->spairs.begin() + cdst[4 * part + c],
+             rest = P->spairs.begin() + odst[4 * part + c];
+        if (W.nmain[c] == W.by_cls[c].size())
+          std::copy(W.by_cls[c].begin(), W.by_cls[c].end(), first);
+        else
+          std::partition_copy(W.by_cls[c].begin(), W.by_cls[c].end(), first,
+                              rest, is_main);
+      }
       W = SPart();
     }
   });
@@ -599,12 +691,15 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
     H2HIP_CHECK(P->d_fix.upload_grow(P->fix.data(), P->fix.size(), st));
     H2HIP_CHECK(
         P->d_spairs.upload_grow(P->spairs.data(), P->spairs.size(), st));
+    H2HIP_CHECK(
+        P->d_mirlist.upload_grow(P->mirlist.data(), P->mirlist.size(), st));
     return H2HIP_OK;
   }
   H2HIP_CHECK(P->d_tiles.upload(P->tiles.data(), P->tiles.size()));
   H2HIP_CHECK(P->d_supp.upload(P->supp.data(), P->supp.size()));
   H2HIP_CHECK(P->d_fix.upload(P->fix.data(), P->fix.size()));
   H2HIP_CHECK(P->d_spairs.upload(P->spairs.data(), P->spairs.size()));
+  H2HIP_CHECK(P->d_mirlist.upload(P->mirlist.data(), P->mirlist.size()));
   return H2HIP_OK;
 }
 
@@ -643,6 +738,13 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
   a.out = (double *)d_out;
   a.counter = P->persistent ? P->d_counter.p : nullptr;
   a.tlist = nullptr;
+  // mirrored tiles in the launches per rule class of the plan's own order
+  const bool mir = !P->mirlist.empty() && !P->sorted && !P->persistent &&
+                   !P->fused && !far;
+  a.mirlist = P->d_mirlist.p;
+  a.nmir = mir ? (uint32_t)P->mirlist.size() : 0;
+  a.nmain3 = P->nmain[CLS_IDENTICAL];
+  a.nmain1 = P->nmain[CLS_VERTEX];
   if (P->fused && !far && op->q == 2 && op->q2 == 4) {
     a.tiles = P->d_tiles_f.p;
     a.tlist = P->d_tpairs.p;
@@ -650,12 +752,22 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
   const uint32_t ntiles = (uint32_t)P->tiles.size();
   uint32_t ncls[4];
   for (int c = 0; c < 4; c++) ncls[c] = (uint32_t)P->pairs[c];
+  // FP64 Helmholtz kernels without argument reduction: real k, and the phase
+  // varies by at most pi/4 over two edges (|r - r0| <= 2 h within a pair of
+  // triangles, r <= 2 h in a pair with common vertices)
+  const bool small = a.mp == 0 && a.ki == 0.0 &&
+                     std::fabs(a.kr) * 2.0 * s->hmax <= 0.25 * M_PI;
+  auto launch = op->kernel != H2HIP_HELMHOLTZ ? nullptr
+                : op->layer == H2HIP_SLP
+                    ? (small ? nf::launch_helmholtz_slp_sp
+                             : nf::launch_helmholtz_slp)
+                    : (small ? nf::launch_helmholtz_dlp_sp
+                             : nf::launch_helmholtz_dlp);
   const int rc =
-      op->kernel == H2HIP_HELMHOLTZ
-          ? nf::launch_helmholtz(op->layer, op->rb, op->cb, op->q, a, ntiles,
-                                 P->d_spairs.p, ncls, stream)
-          : nf::launch_laplace(op->layer, op->rb, op->cb, op->q, a, ntiles,
-                               P->d_spairs.p, ncls, stream);
+      launch ? launch(op->rb, op->cb, op->q, a, ntiles, P->d_spairs.p, ncls,
+                      stream)
+             : nf::launch_laplace(op->layer, op->rb, op->cb, op->q, a, ntiles,
+                                  P->d_spairs.p, ncls, stream);
   if (rc != H2HIP_OK) {
     set_error("unsupported regular quadrature order (1..4 supported)");
     return rc;
@@ -896,6 +1008,15 @@ int h2hip_surface_create(h2hip_surface **out, uint32_t vertices,
       for (int d = 0; d < 3; d++) s->n[3 * i + d] = c[d] / len;
     }
   }
+  double h2 = 0.0;
+  for (uint32_t i = 0; i < triangles; i++)
+    for (int l = 0; l < 3; l++) {
+      const double *p = &s->x[3 * s->t[3 * i + l]];
+      const double *q = &s->x[3 * s->t[3 * i + (l + 1) % 3]];
+      const double d0 = p[0] - q[0], d1 = p[1] - q[1], d2 = p[2] - q[2];
+      h2 = std::max(h2, d0 * d0 + d1 * d1 + d2 * d2);
+    }
+  s->hmax = std::sqrt(h2);
   // triangles of each vertex, in decreasing triangle order as the
   // reference's prepend-built lists
   s->v2t_ptr.assign(vertices + 1, 0);
@@ -1245,6 +1366,8 @@ int h2hip_nfplan_set_schedule(h2hip_nfplan *p, int sorted, int persistent) {
       p->tiles[i] = p->tiles0[perm[i]];
       pos[perm[i]] = (uint32_t)i;
     }
+    for (auto &T : p->tiles)
+      if (T.mirror != NO_MIRROR) T.mirror = pos[T.mirror];
     for (auto &sp : p->spairs) sp.tile = pos[sp.tile];
   } else {
     p->tiles = p->tiles0;

@@ -1,5 +1,5 @@
 // Device code of the near-field quadrature (included by the per-family
-// translation units nf_laplace.hip and nf_helmholtz.hip).
+// translation units nf_laplace.hip and nf_helmholtz_*.hip).
 //
 // Two kernels per operator, run in this order on one stream:
 //
@@ -33,7 +33,23 @@ namespace nf {
 constexpr int NTHREADS = 256;
 constexpr int NWAVES = NTHREADS / 64;
 
-enum { K_LAP_SLP = 0, K_LAP_DLP = 1, K_HELM_SLP = 2, K_HELM_DLP = 3 };
+// K_HELM_*_SP: the Helmholtz kernels for surfaces on which the phase varies
+// by less than pi/4 within a pair of triangles with common vertices and
+// around a reference distance within any other pair (real k, 2 |k| h <= pi/4
+// with the longest edge h): no argument reduction per evaluation, and no
+// damping, whose exponential breaks up the evaluations of a pair.
+enum {
+  K_LAP_SLP = 0,
+  K_LAP_DLP = 1,
+  K_HELM_SLP = 2,
+  K_HELM_DLP = 3,
+  K_HELM_SLP_SP = 4,
+  K_HELM_DLP_SP = 5
+};
+constexpr bool is_dlp(int ker) {
+  return ker == K_LAP_DLP || ker == K_HELM_DLP || ker == K_HELM_DLP_SP;
+}
+constexpr bool small_phase(int ker) { return ker >= K_HELM_SLP_SP; }
 
 // 1/sqrt(x): hardware estimate and one third-order correction
 // y (1 + e/2 + 3 e^2/8), e = 1 - x y^2.  Positive finite x only (x = 0
@@ -44,42 +60,71 @@ __device__ __forceinline__ double rsqrt_fast(double x) {
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
+// x^(-3/2): y^3 (1 + 3e/2 + 15e^2/8) with y and e as above (two roundings
+// and one operation less than the cube of rsqrt_fast).
+__device__ __forceinline__ double rsqrt3_fast(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double y2 = y * y;
+  const double e = fma(-x, y2, 1.0);
+  const double t = y * y2;
+  return fma(t * e, fma(e, 1.875, 1.5), t);
+}
+
 // Kernel function values without the 1/(4 pi) factor.
 // Laplace SLP 1/r, DLP <d, n_y>/r^3 (Library/laplacebem3d.c:35-108);
 // Helmholtz SLP e^{ikr}/r, DLP e^{ikr} (1 - ikr) <d, n_y>/r^3
 // (Library/helmholtzbem3d.c:26-170), d = x - y, r = |d|,
 // k = kr + i ki' with ki = -ki' (damping e^{ki r}).
+//
+// kcore: the part that does not depend on the normal, g (fr + i fi) with
+// real g; the double layers multiply g by <d, n>.  The phase is k r - ph0
+// (ph0 = 0: the kernel itself); the small-phase kernels take it without
+// argument reduction.
+template <int KER>
+__device__ __forceinline__ void kcore(double r2, double kr, double ki,
+                                      double ph0, double &g, double &fr,
+                                      double &fi) {
+  if constexpr (KER == K_LAP_SLP) {
+    g = rsqrt_fast(r2);
+    fr = 1.0;
+    fi = 0.0;
+  } else if constexpr (KER == K_LAP_DLP) {
+    g = rsqrt3_fast(r2);
+    fr = 1.0;
+    fi = 0.0;
+  } else {
+    const double rs = rsqrt_fast(r2);
+    const double r = r2 * rs;
+    g = is_dlp(KER) ? rs * rs * rs : rs;
+    double s, c;
+    if constexpr (small_phase(KER)) {
+      h2hip::sincos_poly(fma(kr, r, -ph0), s, c);
+    } else {
+      if (ki != 0.0) g *= exp(ki * r);
+      h2hip::sincos_cw(kr * r, s, c);
+    }
+    if constexpr (is_dlp(KER)) {
+      const double kr_r = kr * r;
+      fr = fma(kr_r, s, c);
+      fi = fma(-c, kr_r, s);
+    } else {
+      fr = c;
+      fi = s;
+    }
+  }
+}
+
 template <int KER>
 __device__ __forceinline__ void kval(double dx, double dy, double dz,
                                      double nx, double ny, double nz,
                                      double kr, double ki, double &re,
                                      double &im) {
   const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-  const double rs = rsqrt_fast(r2);
-  if constexpr (KER == K_LAP_SLP) {
-    re = rs;
-    im = 0.0;
-  } else if constexpr (KER == K_LAP_DLP) {
-    re = fma(dx, nx, fma(dy, ny, dz * nz)) * (rs * rs * rs);
-    im = 0.0;
-  } else if constexpr (KER == K_HELM_SLP) {
-    const double r = r2 * rs;
-    double amp = rs;
-    if (ki != 0.0) amp *= exp(ki * r);
-    double s, c;
-    h2hip::sincos_cw(kr * r, s, c);
-    re = amp * c;
-    im = amp * s;
-  } else {
-    const double r = r2 * rs;
-    double amp = fma(dx, nx, fma(dy, ny, dz * nz)) * (rs * rs * rs);
-    if (ki != 0.0) amp *= exp(ki * r);
-    const double kr_r = kr * r;
-    double s, c;
-    h2hip::sincos_cw(kr_r, s, c);
-    re = fma(kr_r, s, c) * amp;
-    im = fma(-c, kr_r, s) * amp;
-  }
+  double g, fr, fi;
+  kcore<KER>(r2, kr, ki, 0.0, g, fr, fi);
+  if constexpr (is_dlp(KER)) g *= fma(dx, nx, fma(dy, ny, dz * nz));
+  re = KER >= K_HELM_SLP ? fr * g : g;
+  im = KER >= K_HELM_SLP ? fi * g : 0.0;
 }
 
 // The same kernel values in FP32 (mixed precision), from a difference
@@ -89,40 +134,44 @@ __device__ __forceinline__ void kval(double dx, double dy, double dz,
 // [-1/2, 1/2] revolutions before the hardware sine and cosine, so their
 // argument is always small; the damping e^{ki r} is the hardware 2^x of
 // ki log2(e) r.
+// kcore32, kval32: as kcore and kval.
 template <int KER>
-__device__ __forceinline__ void kval32(float dx, float dy, float dz, float nx,
-                                       float ny, float nz, float krf,
-                                       float krev, float kil2, float &re,
-                                       float &im) {
-  const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+__device__ __forceinline__ void kcore32(float r2, float krf, float krev,
+                                        float kil2, float &g, float &fr,
+                                        float &fi) {
   const float rs = __builtin_amdgcn_rsqf(r2);
-  if constexpr (KER == K_LAP_SLP) {
-    re = rs;
-    im = 0.0f;
-  } else if constexpr (KER == K_LAP_DLP) {
-    re = fmaf(dx, nx, fmaf(dy, ny, dz * nz)) * (rs * rs * rs);
-    im = 0.0f;
-  } else {
+  g = is_dlp(KER) ? rs * rs * rs : rs;
+  fr = 1.0f;
+  fi = 0.0f;
+  if constexpr (KER >= K_HELM_SLP) {
     const float r = r2 * rs;
     float rev = r * krev;
     rev -= __builtin_rintf(rev);
     const float s = __builtin_amdgcn_sinf(rev);
     const float c = __builtin_amdgcn_cosf(rev);
-    float amp;
-    if constexpr (KER == K_HELM_SLP)
-      amp = rs;
-    else
-      amp = fmaf(dx, nx, fmaf(dy, ny, dz * nz)) * (rs * rs * rs);
-    if (kil2 != 0.0f) amp *= __builtin_amdgcn_exp2f(kil2 * r);
-    if constexpr (KER == K_HELM_SLP) {
-      re = amp * c;
-      im = amp * s;
-    } else {
+    if (kil2 != 0.0f) g *= __builtin_amdgcn_exp2f(kil2 * r);
+    if constexpr (is_dlp(KER)) {
       const float kr_r = krf * r;
-      re = fmaf(kr_r, s, c) * amp;
-      im = fmaf(-c, kr_r, s) * amp;
+      fr = fmaf(kr_r, s, c);
+      fi = fmaf(-c, kr_r, s);
+    } else {
+      fr = c;
+      fi = s;
     }
   }
+}
+
+template <int KER>
+__device__ __forceinline__ void kval32(float dx, float dy, float dz, float nx,
+                                       float ny, float nz, float krf,
+                                       float krev, float kil2, float &re,
+                                       float &im) {
+  float g, fr, fi;
+  kcore32<KER>(fmaf(dx, dx, fmaf(dy, dy, dz * dz)), krf, krev, kil2, g, fr,
+               fi);
+  if constexpr (is_dlp(KER)) g *= fmaf(dx, nx, fmaf(dy, ny, dz * nz));
+  re = KER >= K_HELM_SLP ? fr * g : g;
+  im = KER >= K_HELM_SLP ? fi * g : 0.0f;
 }
 
 // Normal vector of the double layer kernels for the pair (row triangle
@@ -137,6 +186,15 @@ __device__ __forceinline__ void layer_normal(const KArgs &a, uint32_t rt,
   const double sg = a.adj ? -1.0 : 1.0;
 #pragma unroll
   for (int d = 0; d < 3; d++) nv[d] = sg * a.n[3 * t + d];
+}
+
+// kernel constant and Gram determinants of a pair of triangles (constant
+// basis: in the order of the triangle numbers, as entry_sums)
+template <bool CC>
+__device__ __forceinline__ double pair_factor(const KArgs &a, uint32_t rt,
+                                              uint32_t ct) {
+  const uint32_t lo = CC && rt > ct ? ct : rt, hi = CC && rt > ct ? rt : ct;
+  return a.kc * a.g[lo] * a.g[hi];
 }
 
 static __global__ void zero_counter(uint32_t *c) { *c = 0u; }
@@ -161,15 +219,249 @@ __device__ __forceinline__ void kahan_add(float &s, float &c, float x) {
   s = t;
 }
 
-// One tile of the regular kernel, run by all NTHREADS threads of a
-// workgroup.  MP: 0 FP64; 1 mixed (FP32 kernel values and inner sums, FP64
+// Element matrices of a pair of triangles without common vertices by the
+// tensor-product rule: S1[l][k] sums the kernel over the row triangle's
+// local function l and the column triangle's k (1 or 3 each); TWO: S2[l][k]
+// the kernel of the exchanged pair (column triangle as the row, the mirror
+// block's entry), which shares the difference, its length and the phase and
+// costs one product with the other normal n2 more.  n1, n2 multiply
+// d = x - y.  MP: 0 FP64; 1 mixed (FP32 kernel values and inner sums, FP64
 // outer sums); 2 mixed with FP32 accumulation throughout, the outer sums
-// compensated (Kahan).
+// compensated (Kahan); TWO is for MP 0 and 1.
+template <int KER, int BR, int BC, int Q, int MP, bool TWO>
+__device__ __forceinline__ void pair_sums(
+    const KArgs &a, uint32_t tt, uint32_t ts, const double (&n1)[3],
+    const double (&n2)[3], double (&S1re)[BR ? 3 : 1][BC ? 3 : 1],
+    double (&S1im)[BR ? 3 : 1][BC ? 3 : 1],
+    double (&S2re)[BR ? 3 : 1][BC ? 3 : 1],
+    double (&S2im)[BR ? 3 : 1][BC ? 3 : 1]) {
+  constexpr bool CPLX = KER >= K_HELM_SLP;
+  constexpr bool DLP = is_dlp(KER);
+  constexpr int NR = BR ? 3 : 1;
+  constexpr int NC = BC ? 3 : 1;
+  constexpr int QQ = Q * Q;
+  const double *__restrict__ W = a.regw;  // w | phi0 w | phi1 w | phi2 w
+  const double *__restrict__ Pt = a.regpts + (size_t)tt * (3 * QQ);
+  const double *__restrict__ Ps = a.regpts + (size_t)ts * (3 * QQ);
+#pragma unroll
+  for (int l = 0; l < NR; l++)
+#pragma unroll
+    for (int k = 0; k < NC; k++)
+      S1re[l][k] = S1im[l][k] = S2re[l][k] = S2im[l][k] = 0.0;
+  if constexpr (MP != 0) {
+    static_assert(!(TWO && MP == 2), "both orders: FP64 outer sums");
+    // x_i - y_b = (P_t,i - P_s,0) - (P_s,b - P_s,0), the first difference in
+    // FP64 (then rounded), the offsets of the column points in FP32
+    const float *__restrict__ Os = a.regoff + (size_t)ts * (3 * QQ);
+    const float *__restrict__ WF = a.regwf;
+    const double sx0 = Ps[0], sy0 = Ps[1], sz0 = Ps[2];
+    float ptx[QQ], pty[QQ], ptz[QQ];
+#pragma unroll
+    for (int i = 0; i < QQ; i++) {
+      ptx[i] = (float)(Pt[3 * i] - sx0);
+      pty[i] = (float)(Pt[3 * i + 1] - sy0);
+      ptz[i] = (float)(Pt[3 * i + 2] - sz0);
+    }
+    const float n1x = (float)n1[0], n1y = (float)n1[1], n1z = (float)n1[2];
+    const float n2x = (float)n2[0], n2y = (float)n2[1], n2z = (float)n2[2];
+    // MP 2: the outer sums in FP32 with their compensations
+    float Fre[NR][NC], Fim[NR][NC], Cre[NR][NC], Cim[NR][NC];
+#pragma unroll
+    for (int l = 0; l < NR; l++)
+#pragma unroll
+      for (int k = 0; k < NC; k++)
+        Fre[l][k] = Fim[l][k] = Cre[l][k] = Cim[l][k] = 0.0f;
+#pragma unroll
+    for (int b = 0; b < QQ; b++) {
+      const float qx = Os[3 * b], qy = Os[3 * b + 1], qz = Os[3 * b + 2];
+      float Ure[NR], Uim[NR], Vre[NR], Vim[NR];
+#pragma unroll
+      for (int l = 0; l < NR; l++) Ure[l] = Uim[l] = Vre[l] = Vim[l] = 0.0f;
+#pragma unroll
+      for (int i = 0; i < QQ; i++) {
+        const float dx = ptx[i] - qx, dy = pty[i] - qy, dz = ptz[i] - qz;
+        float g, fr, fi;
+        kcore32<KER>(fmaf(dx, dx, fmaf(dy, dy, dz * dz)), a.krf, a.krev,
+                     a.kil2, g, fr, fi);
+        float g1 = g, g2 = g;
+        if constexpr (DLP) {
+          g1 = fmaf(dx, n1x, fmaf(dy, n1y, dz * n1z)) * g;
+          if constexpr (TWO) g2 = fmaf(dx, n2x, fmaf(dy, n2y, dz * n2z)) * g;
+        }
+#pragma unroll
+        for (int l = 0; l < NR; l++) {
+          const float wr = BR ? WF[QQ * (1 + l) + i] : WF[i];
+          Ure[l] = fmaf(wr, CPLX ? g1 * fr : g1, Ure[l]);
+          if constexpr (CPLX) Uim[l] = fmaf(wr, g1 * fi, Uim[l]);
+          if constexpr (TWO) {
+            Vre[l] = fmaf(wr, CPLX ? g2 * fr : g2, Vre[l]);
+            if constexpr (CPLX) Vim[l] = fmaf(wr, g2 * fi, Vim[l]);
+          }
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < NC; k++) {
+        if constexpr (MP == 2) {
+          const float wc = BC ? WF[QQ * (1 + k) + b] : WF[b];
+#pragma unroll
+          for (int l = 0; l < NR; l++) {
+            kahan_add(Fre[l][k], Cre[l][k], wc * Ure[l]);
+            if constexpr (CPLX) kahan_add(Fim[l][k], Cim[l][k], wc * Uim[l]);
+          }
+        } else {
+          const double wc = BC ? W[QQ * (1 + k) + b] : W[b];
+#pragma unroll
+          for (int l = 0; l < NR; l++) {
+            S1re[l][k] = fma(wc, (double)Ure[l], S1re[l][k]);
+            if constexpr (CPLX)
+              S1im[l][k] = fma(wc, (double)Uim[l], S1im[l][k]);
+            if constexpr (TWO) {
+              S2re[l][k] = fma(wc, (double)Vre[l], S2re[l][k]);
+              if constexpr (CPLX)
+                S2im[l][k] = fma(wc, (double)Vim[l], S2im[l][k]);
+            }
+          }
+        }
+      }
+    }
+    if constexpr (MP == 2) {
+#pragma unroll
+      for (int l = 0; l < NR; l++)
+#pragma unroll
+        for (int k = 0; k < NC; k++) {
+          S1re[l][k] = (double)Fre[l][k] - (double)Cre[l][k];
+          S1im[l][k] = (double)Fim[l][k] - (double)Cim[l][k];
+        }
+    }
+  } else {
+    double ptx[QQ], pty[QQ], ptz[QQ];
+#pragma unroll
+    for (int i = 0; i < QQ; i++) {
+      ptx[i] = Pt[3 * i];
+      pty[i] = Pt[3 * i + 1];
+      ptz[i] = Pt[3 * i + 2];
+    }
+    // small phase: k r is taken relative to that of the first points, the
+    // sums are turned by it at the end
+    double ph0 = 0.0;
+    if constexpr (small_phase(KER)) {
+      const double dx = ptx[0] - Ps[0], dy = pty[0] - Ps[1],
+                   dz = ptz[0] - Ps[2];
+      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+      ph0 = a.kr * (r2 * rsqrt_fast(r2));
+    }
+#pragma unroll
+    for (int b = 0; b < QQ; b++) {
+      const double qx = Ps[3 * b], qy = Ps[3 * b + 1], qz = Ps[3 * b + 2];
+      double Ure[NR], Uim[NR], Vre[NR], Vim[NR];
+#pragma unroll
+      for (int l = 0; l < NR; l++) Ure[l] = Uim[l] = Vre[l] = Vim[l] = 0.0;
+#pragma unroll
+      for (int i = 0; i < QQ; i++) {
+        const double dx = ptx[i] - qx, dy = pty[i] - qy, dz = ptz[i] - qz;
+        double g, fr, fi;
+        kcore<KER>(fma(dx, dx, fma(dy, dy, dz * dz)), a.kr, a.ki, ph0, g, fr,
+                   fi);
+        double g1 = g, g2 = g;
+        if constexpr (DLP) {
+          g1 = g * fma(dx, n1[0], fma(dy, n1[1], dz * n1[2]));
+          if constexpr (TWO)
+            g2 = g * fma(dx, n2[0], fma(dy, n2[1], dz * n2[2]));
+        }
+#pragma unroll
+        for (int l = 0; l < NR; l++) {
+          const double wr = BR ? W[QQ * (1 + l) + i] : W[i];
+          Ure[l] = fma(wr, CPLX ? g1 * fr : g1, Ure[l]);
+          if constexpr (CPLX) Uim[l] = fma(wr, g1 * fi, Uim[l]);
+          if constexpr (TWO) {
+            Vre[l] = fma(wr, CPLX ? g2 * fr : g2, Vre[l]);
+            if constexpr (CPLX) Vim[l] = fma(wr, g2 * fi, Vim[l]);
+          }
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < NC; k++) {
+        const double wc = BC ? W[QQ * (1 + k) + b] : W[b];
+#pragma unroll
+        for (int l = 0; l < NR; l++) {
+          S1re[l][k] = fma(wc, Ure[l], S1re[l][k]);
+          if constexpr (CPLX) S1im[l][k] = fma(wc, Uim[l], S1im[l][k]);
+          if constexpr (TWO) {
+            S2re[l][k] = fma(wc, Vre[l], S2re[l][k]);
+            if constexpr (CPLX) S2im[l][k] = fma(wc, Vim[l], S2im[l][k]);
+          }
+        }
+      }
+    }
+    if constexpr (small_phase(KER)) {
+      double s0, c0;
+      h2hip::sincos_cw(ph0, s0, c0);
+#pragma unroll
+      for (int l = 0; l < NR; l++)
+#pragma unroll
+        for (int k = 0; k < NC; k++) {
+          const double x = S1re[l][k], y = S1im[l][k];
+          S1re[l][k] = fma(x, c0, -(y * s0));
+          S1im[l][k] = fma(x, s0, y * c0);
+          if constexpr (TWO) {
+            const double u = S2re[l][k], v = S2im[l][k];
+            S2re[l][k] = fma(u, c0, -(v * s0));
+            S2im[l][k] = fma(u, s0, v * c0);
+          }
+        }
+    }
+  }
+}
+
+// Whether a launch over mirrored tiles evaluates the regular pairs once for
+// both entries (nf_pair_kernel): equal bases; FP64, or the single layers in
+// mixed precision with FP64 outer sums.  Not the double layers in mixed
+// precision: their <d, n> of nearly coplanar triangles is the rounding of
+// d, which depends on the triangle whose point is the anchor.  Not the
+// linear-basis Helmholtz double layers, whose four accumulators (128 KB of
+// LDS) and 36 sums per lane leave one workgroup per CU.
+constexpr int pair_arrays(int ker, int basis) {
+  return basis == 0 ? 0 : (ker >= K_HELM_SLP ? 2 : 1) * (is_dlp(ker) ? 2 : 1);
+}
+constexpr bool paired(int ker, int rb, int cb, int mp) {
+  return rb == cb && (mp == 0 || (mp == 1 && !is_dlp(ker))) &&
+         pair_arrays(ker, rb) <= 2;
+}
+
+// The same sums for the entry (row triangle rt, column triangle ct).  The
+// constant basis evaluates a pair of triangles in one order, the smaller
+// number first, whichever of the two entries asks: both entries then have
+// the same bits in every schedule.
+template <int KER, int BR, int BC, int Q, int MP>
+__device__ __forceinline__ void entry_sums(
+    const KArgs &a, uint32_t rt, uint32_t ct,
+    double (&Sre)[BR ? 3 : 1][BC ? 3 : 1],
+    double (&Sim)[BR ? 3 : 1][BC ? 3 : 1]) {
+  constexpr bool CC = (BR == 0) && (BC == 0);
+  // The reference's lc far integrator maps the first rule coordinates onto
+  // the column triangle (Library/bem3d.c:2637-2649); kept as is.
+  const bool sw =
+      CC ? paired(KER, 0, 0, MP) && rt > ct : (BR && !BC) && a.far;
+  double nv[3] = {0.0, 0.0, 0.0};
+  if constexpr (is_dlp(KER)) {
+    layer_normal(a, rt, ct, nv);
+    if (CC && sw) {
+#pragma unroll
+      for (int d = 0; d < 3; d++) nv[d] = -nv[d];
+    }
+  }
+  double dre[BR ? 3 : 1][BC ? 3 : 1], dim[BR ? 3 : 1][BC ? 3 : 1];
+  pair_sums<KER, BR, BC, Q, MP, false>(a, sw ? ct : rt, sw ? rt : ct, nv, nv,
+                                       Sre, Sim, dre, dim);
+}
+
 template <int KER, int BR, int BC, int CLS, int Q2, bool MP>
 __device__ __forceinline__ void tile_singular(const KArgs &a, const Tile &T,
                                               const SPair *list, uint32_t n,
                                               double *acc_re, double *acc_im);
 
+// One tile of the regular kernel, run by all NTHREADS threads of a
+// workgroup (MP: pair_sums).
 // FUSED: the tile's workgroup also evaluates the tile's pairs with common
 // vertices (tlist + T.sbeg, T.ns[c] per class) before the tile is stored,
 // so they add into the LDS accumulator instead of the output (constant
@@ -178,11 +470,9 @@ template <int KER, int BR, int BC, int Q, int MP, bool FUSED = false>
 __device__ __forceinline__ void regular_tile(const KArgs &a, uint32_t tile,
                                              const SPair *tlist = nullptr) {
   constexpr bool CPLX = KER >= K_HELM_SLP;
-  constexpr bool DLP = (KER == K_LAP_DLP) || (KER == K_HELM_DLP);
   constexpr bool CC = (BR == 0) && (BC == 0);
   constexpr int NR = BR ? 3 : 1;
   constexpr int NC = BC ? 3 : 1;
-  constexpr int QQ = Q * Q;
 
   __shared__ double acc_re[CC ? 1 : TILE * TILE];
   __shared__ double acc_im[(CC || !CPLX) ? 1 : TILE * TILE];
@@ -192,7 +482,6 @@ __device__ __forceinline__ void regular_tile(const KArgs &a, uint32_t tile,
   const uint32_t nR = T.nrsup, nC = T.ncsup;
   const Supp *RS = a.supp + T.rsup;
   const Supp *CS = a.supp + T.csup;
-  const double *__restrict__ W = a.regw;  // w | phi0 w | phi1 w | phi2 w
   const bool conj = T.ntrans && (BR == BC);
 
   if constexpr (!CC) {
@@ -229,141 +518,9 @@ __device__ __forceinline__ void regular_tile(const KArgs &a, uint32_t tile,
 #pragma unroll
       for (int k = 0; k < NC; k++) Sre[l][k] = Sim[l][k] = 0.0;
     double f2 = 0.0;
-    if (MP && !shared) {
-      // Mixed precision: x_i - y_b = (P_t,i - P_s,0) - (P_s,b - P_s,0), the
-      // first difference in FP64 (then rounded), the offsets of the column
-      // points in FP32; kernel values and the sums over i in FP32, the sums
-      // over b in FP64.
-      const bool swapgeo = (BR && !BC) && a.far;
-      const uint32_t tt = swapgeo ? sc.tri : sr.tri;
-      const uint32_t ts = swapgeo ? sr.tri : sc.tri;
-      const double *__restrict__ Pt = a.regpts + (size_t)tt * (3 * QQ);
-      const double *__restrict__ Ps = a.regpts + (size_t)ts * (3 * QQ);
-      const float *__restrict__ Os = a.regoff + (size_t)ts * (3 * QQ);
-      const float *__restrict__ WF = a.regwf;
-      const double sx0 = Ps[0], sy0 = Ps[1], sz0 = Ps[2];
-      float ptx[QQ], pty[QQ], ptz[QQ];
-#pragma unroll
-      for (int i = 0; i < QQ; i++) {
-        ptx[i] = (float)(Pt[3 * i] - sx0);
-        pty[i] = (float)(Pt[3 * i + 1] - sy0);
-        ptz[i] = (float)(Pt[3 * i + 2] - sz0);
-      }
-      float nx = 0.0f, ny = 0.0f, nz = 0.0f;
-      if constexpr (DLP) {
-        double n64[3];
-        layer_normal(a, sr.tri, sc.tri, n64);
-        nx = (float)n64[0];
-        ny = (float)n64[1];
-        nz = (float)n64[2];
-      }
-      f2 = a.kc * a.g[sr.tri] * a.g[sc.tri];
-      // MP 2: the outer sums in FP32 with their compensations
-      float Fre[NR][NC], Fim[NR][NC], Cre[NR][NC], Cim[NR][NC];
-#pragma unroll
-      for (int l = 0; l < NR; l++)
-#pragma unroll
-        for (int k = 0; k < NC; k++)
-          Fre[l][k] = Fim[l][k] = Cre[l][k] = Cim[l][k] = 0.0f;
-#pragma unroll
-      for (int b = 0; b < QQ; b++) {
-        const float qx = Os[3 * b], qy = Os[3 * b + 1], qz = Os[3 * b + 2];
-        float Ure[NR], Uim[NR];
-#pragma unroll
-        for (int l = 0; l < NR; l++) Ure[l] = Uim[l] = 0.0f;
-#pragma unroll
-        for (int i = 0; i < QQ; i++) {
-          float vre, vim;
-          kval32<KER>(ptx[i] - qx, pty[i] - qy, ptz[i] - qz, nx, ny, nz,
-                      a.krf, a.krev, a.kil2, vre, vim);
-#pragma unroll
-          for (int l = 0; l < NR; l++) {
-            const float wr = BR ? WF[QQ * (1 + l) + i] : WF[i];
-            Ure[l] = fmaf(wr, vre, Ure[l]);
-            if constexpr (CPLX) Uim[l] = fmaf(wr, vim, Uim[l]);
-          }
-        }
-#pragma unroll
-        for (int k = 0; k < NC; k++) {
-          if constexpr (MP == 2) {
-            const float wc = BC ? WF[QQ * (1 + k) + b] : WF[b];
-#pragma unroll
-            for (int l = 0; l < NR; l++) {
-              kahan_add(Fre[l][k], Cre[l][k], wc * Ure[l]);
-              if constexpr (CPLX) kahan_add(Fim[l][k], Cim[l][k], wc * Uim[l]);
-            }
-          } else {
-            const double wc = BC ? W[QQ * (1 + k) + b] : W[b];
-#pragma unroll
-            for (int l = 0; l < NR; l++) {
-              Sre[l][k] = fma(wc, (double)Ure[l], Sre[l][k]);
-              if constexpr (CPLX)
-                Sim[l][k] = fma(wc, (double)Uim[l], Sim[l][k]);
-            }
-          }
-        }
-      }
-      if constexpr (MP == 2) {
-#pragma unroll
-        for (int l = 0; l < NR; l++)
-#pragma unroll
-          for (int k = 0; k < NC; k++) {
-            Sre[l][k] = (double)Fre[l][k] - (double)Cre[l][k];
-            Sim[l][k] = (double)Fim[l][k] - (double)Cim[l][k];
-          }
-      }
-    } else if (!MP && !shared) {
-      // The reference's lc far integrator maps the first rule coordinates
-      // onto the column triangle (Library/bem3d.c:2637-2649); kept as is.
-      const bool swapgeo = (BR && !BC) && a.far;
-      const double *__restrict__ Pt =
-          a.regpts + (size_t)(swapgeo ? sc.tri : sr.tri) * (3 * QQ);
-      const double *__restrict__ Ps =
-          a.regpts + (size_t)(swapgeo ? sr.tri : sc.tri) * (3 * QQ);
-      double ptx[QQ], pty[QQ], ptz[QQ];
-#pragma unroll
-      for (int i = 0; i < QQ; i++) {
-        ptx[i] = Pt[3 * i];
-        pty[i] = Pt[3 * i + 1];
-        ptz[i] = Pt[3 * i + 2];
-      }
-      double nx = 0.0, ny = 0.0, nz = 0.0;
-      if constexpr (DLP) {
-        double n64[3];
-        layer_normal(a, sr.tri, sc.tri, n64);
-        nx = n64[0];
-        ny = n64[1];
-        nz = n64[2];
-      }
-      f2 = a.kc * a.g[sr.tri] * a.g[sc.tri];
-#pragma unroll
-      for (int b = 0; b < QQ; b++) {
-        const double qx = Ps[3 * b], qy = Ps[3 * b + 1], qz = Ps[3 * b + 2];
-        double Ure[NR], Uim[NR];
-#pragma unroll
-        for (int l = 0; l < NR; l++) Ure[l] = Uim[l] = 0.0;
-#pragma unroll
-        for (int i = 0; i < QQ; i++) {
-          double vre, vim;
-          kval<KER>(ptx[i] - qx, pty[i] - qy, ptz[i] - qz, nx, ny, nz, a.kr,
-                    a.ki, vre, vim);
-#pragma unroll
-          for (int l = 0; l < NR; l++) {
-            const double wr = BR ? W[QQ * (1 + l) + i] : W[i];
-            Ure[l] = fma(wr, vre, Ure[l]);
-            if constexpr (CPLX) Uim[l] = fma(wr, vim, Uim[l]);
-          }
-        }
-#pragma unroll
-        for (int k = 0; k < NC; k++) {
-          const double wc = BC ? W[QQ * (1 + k) + b] : W[b];
-#pragma unroll
-          for (int l = 0; l < NR; l++) {
-            Sre[l][k] = fma(wc, Ure[l], Sre[l][k]);
-            if constexpr (CPLX) Sim[l][k] = fma(wc, Uim[l], Sim[l][k]);
-          }
-        }
-      }
+    if (!shared) {
+      f2 = pair_factor<CC>(a, sr.tri, sc.tri);
+      entry_sums<KER, BR, BC, Q, MP>(a, sr.tri, sc.tri, Sre, Sim);
     }
     if constexpr (CC) {
       // entry (r, c) of the tile; pairs with common vertices are stored as
@@ -432,6 +589,188 @@ __device__ __forceinline__ void regular_tile(const KArgs &a, uint32_t tile,
 template <int KER, int BR, int BC, int Q, int MP>
 __global__ __launch_bounds__(NTHREADS) void nf_regular_kernel(KArgs a) {
   regular_tile<KER, BR, BC, Q, MP>(a, blockIdx.x);
+}
+
+// Two mirrored tiles per workgroup: tile T = (rows R, columns C) and its
+// mirror (C, R) of a plan whose blocks come in mirrored pairs over one index
+// array, as the near field of a mesh does.  Every pair of triangles is
+// evaluated once for both entries (pair_sums TWO): the single layers' entry
+// is symmetric, the double layers share the distance, its root and the
+// phase.  A diagonal tile is its own mirror: its n (n - 1) / 2 unordered
+// pairs are taken by distance j = 1 .. n/2 around the list (r, r + j mod n),
+// so no lane idles.  Constant basis: both entries are stored at once.
+// Linear basis: the pairs' contributions are summed in LDS as in
+// regular_tile, the double layers with a second accumulator for the mirror
+// tile, and both tiles stored at the end.
+//
+// Bound by FP64 VALU issue (MP: VALU and the transcendental unit).  Threads
+// per workgroup follow the LDS accumulators so that 4 to 5 waves per SIMD
+// are resident: 256 for 32 KB, 512 for 64 KB.  Against one workgroup per
+// tile (nf_regular_kernel): Laplace double layer, linear basis, 32768
+// triangles 1431 -> 1011 us; Helmholtz single layer, constant basis, 131072
+// triangles 2735 -> 1208 us (with the small phase; vertex pairs
+// 1291 -> 465 us, edge pairs, small phase alone, 1153 -> 799 us).
+constexpr int pair_threads(int ker, int basis) {
+  return pair_arrays(ker, basis) > 1 ? 512 : NTHREADS;
+}
+constexpr int pair_waves(int ker, int basis) {
+  return (basis ? pair_arrays(ker, basis) > 1 : ker >= K_HELM_SLP) ? 4 : 5;
+}
+
+template <int KER, int B, int Q, int MP>
+__global__ __launch_bounds__(pair_threads(KER, B),
+                             pair_waves(KER, B)) void nf_pair_kernel(
+    KArgs a, const uint32_t *__restrict__ list) {
+  constexpr bool CPLX = KER >= K_HELM_SLP;
+  constexpr bool DLP = is_dlp(KER);
+  constexpr int NL = B ? 3 : 1;
+  constexpr int NTH = pair_threads(KER, B);
+  constexpr int NA = pair_arrays(KER, B);
+  // re, (im), (re of the mirror), (im of the mirror)
+  __shared__ double acc[NA ? NA * TILE * TILE : 1];
+  double *const acc_re = acc;
+  double *const acc_im = acc + (CPLX ? TILE * TILE : 0);
+  double *const mir_re = acc + (DLP ? (CPLX ? 2 : 1) * TILE * TILE : 0);
+  double *const mir_im = mir_re + (CPLX ? TILE * TILE : 0);
+
+  const int tid = threadIdx.x;
+  const uint32_t tile = list[blockIdx.x];
+  const Tile T = a.tiles[tile];
+  const bool diag = T.mirror == tile;
+  const Tile M = a.tiles[T.mirror];
+  const uint32_t nR = T.nrsup, nC = T.ncsup;
+  const Supp *RS = a.supp + T.rsup;
+  const Supp *CS = a.supp + T.csup;
+
+  if constexpr (B) {
+    for (int i = tid; i < NA * TILE * TILE; i += NTH) acc[i] = 0.0;
+    __syncthreads();
+  } else if (diag) {
+    // identical triangles: completed by the singular kernel
+    for (uint32_t r = tid; r < nR; r += NTH) {
+      const size_t pos = T.out_off + r + (size_t)r * T.ld;
+      if constexpr (CPLX)
+        a.out[2 * pos] = a.out[2 * pos + 1] = 0.0;
+      else
+        a.out[pos] = 0.0;
+    }
+  }
+
+  const uint32_t npairs = diag ? nR * (nR - 1) / 2 : nR * nC;
+  const uint32_t dc = nR ? NTH / nR : 0, dr = NTH - dc * nR;
+  uint32_t rr = nR ? tid % nR : 0, cc = nR ? tid / nR : 0;
+  for (uint32_t p = tid; p < npairs; p += NTH) {
+    const uint32_t r = rr;
+    uint32_t c = cc;
+    rr += dr;
+    cc += dc;
+    if (rr >= nR) {
+      rr -= nR;
+      cc++;
+    }
+    if (diag) {
+      c += r + 1;
+      c -= c >= nR ? nR : 0;
+    }
+    const Supp sr = RS[r], sc = CS[c];
+    int shared = 0;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+      for (int j = 0; j < 3; j++) shared += (sr.v[i] == sc.v[j]);
+    double S1re[NL][NL], S1im[NL][NL], S2re[NL][NL], S2im[NL][NL];
+    double f2 = 0.0;
+    // constant basis: in the order of the triangle numbers, as entry_sums
+    const bool sw = !B && sr.tri > sc.tri;
+    if (!shared) {
+      f2 = pair_factor<!B>(a, sr.tri, sc.tri);
+      double n1[3] = {0.0, 0.0, 0.0}, n2[3] = {0.0, 0.0, 0.0};
+      if constexpr (DLP) {
+        layer_normal(a, sr.tri, sc.tri, n1);
+        layer_normal(a, sc.tri, sr.tri, n2);
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+          n1[d] = sw ? -n1[d] : n1[d];
+          n2[d] = sw ? n2[d] : -n2[d];
+        }
+      }
+      pair_sums<KER, B, B, Q, MP, DLP>(a, sw ? sc.tri : sr.tri,
+                                       sw ? sr.tri : sc.tri, n1, n2, S1re,
+                                       S1im, S2re, S2im);
+    } else {
+#pragma unroll
+      for (int l = 0; l < NL; l++)
+#pragma unroll
+        for (int k = 0; k < NL; k++)
+          S1re[l][k] = S1im[l][k] = S2re[l][k] = S2im[l][k] = 0.0;
+    }
+    if constexpr (!B) {
+      // pairs with common vertices are stored as zero and completed by the
+      // singular kernel
+      const size_t pos = T.out_off + r + (size_t)c * T.ld;
+      const size_t mpos = M.out_off + c + (size_t)r * M.ld;
+      const double vre = f2 * S1re[0][0];
+      const double wre = DLP ? f2 * S2re[0][0] : vre;
+      if constexpr (CPLX) {
+        const double vim = f2 * S1im[0][0];
+        const double wim = DLP ? f2 * S2im[0][0] : vim;
+        a.out[2 * pos] = vre;
+        a.out[2 * pos + 1] = vim;
+        a.out[2 * mpos] = wre;
+        a.out[2 * mpos + 1] = wim;
+      } else {
+        a.out[pos] = vre;
+        a.out[mpos] = wre;
+      }
+    } else if (!shared) {
+#pragma unroll
+      for (int l = 0; l < NL; l++) {
+        const uint32_t lr = loc_of(sr.loc, l);
+        if (lr == 0xffu) continue;
+#pragma unroll
+        for (int k = 0; k < NL; k++) {
+          const uint32_t lc = loc_of(sc.loc, k);
+          if (lc == 0xffu) continue;
+          const int e = lr + TILE * lc;
+          atomicAdd(&acc_re[e], f2 * S1re[l][k]);
+          if constexpr (CPLX) atomicAdd(&acc_im[e], f2 * S1im[l][k]);
+          if constexpr (DLP) {
+            atomicAdd(&mir_re[e], f2 * S2re[l][k]);
+            if constexpr (CPLX) atomicAdd(&mir_im[e], f2 * S2im[l][k]);
+          }
+        }
+      }
+    }
+  }
+
+  if constexpr (B) {
+    // without a second accumulator mir_re is acc_re
+    __syncthreads();
+    const int nr = T.nr, nc = T.nc;
+    for (int e = tid; e < nr * nc; e += NTH) {
+      const int i = e % nr, j = e / nr;
+      const int s = i + TILE * j, t = j + TILE * i;
+      const size_t pos = T.out_off + (size_t)i + (size_t)j * T.ld;
+      if constexpr (CPLX) {
+        a.out[2 * pos] = acc_re[s] + (diag ? mir_re[t] : 0.0);
+        a.out[2 * pos + 1] = acc_im[s] + (diag ? mir_im[t] : 0.0);
+      } else {
+        a.out[pos] = acc_re[s] + (diag ? mir_re[t] : 0.0);
+      }
+    }
+    if (!diag)
+      for (int e = tid; e < nr * nc; e += NTH) {
+        const int j = e % nc, i = e / nc;
+        const int s = i + TILE * j;
+        const size_t pos = M.out_off + (size_t)j + (size_t)i * M.ld;
+        if constexpr (CPLX) {
+          a.out[2 * pos] = mir_re[s];
+          a.out[2 * pos + 1] = mir_im[s];
+        } else {
+          a.out[pos] = mir_re[s];
+        }
+      }
+  }
 }
 
 // Persistent form: a grid sized to the resident workgroups takes tiles from
@@ -566,15 +905,27 @@ __device__ __forceinline__ V sel3(const V (&v)[3], int i) {
 // global atomics for the launches per rule class, the tile's LDS
 // accumulator (or a plain store, constant basis) when the tile's own
 // workgroup evaluates its singular pairs.  The value is not conjugated.
-template <int KER, int BR, int BC, int CLS, int Q2, bool MP, class Sink>
+//
+// MIR: the entry of the exchanged pair (the column triangle as the row, in
+// the mirror tile) as well; sink(lr, lc, re, im, re2, im2).  The vertex
+// rule's two points of a tuple and the identical rule's six map onto each
+// other when the triangles are exchanged, so the exchanged pair has the
+// same points and the same moments, of the kernel with the other normal
+// (single layer: the same values).  The edge rule has no such symmetry.
+template <int KER, int BR, int BC, int CLS, int Q2, bool MP, bool MIR,
+          class Sink>
 __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
                                               const SPair &P, int sub,
                                               Sink &&sink) {
   constexpr bool CPLX = KER >= K_HELM_SLP;
-  constexpr bool DLP = (KER == K_LAP_DLP) || (KER == K_HELM_DLP);
+  constexpr bool DLP = is_dlp(KER);
   constexpr bool CC = (BR == 0) && (BC == 0);
   constexpr int NR = BR ? 3 : 1;
   constexpr int NC = BC ? 3 : 1;
+  static_assert(!MIR || CLS != CLS_EDGE, "the edge rule is not symmetric");
+  // directions summed: both only where the values differ beyond the sign
+  constexpr bool TWO = MIR && DLP && CLS == CLS_VERTEX;
+  constexpr int ND = TWO ? 2 : 1;
 
   const Supp sr = a.supp[T.rsup + P.r], sc = a.supp[T.csup + P.c];
   int tp[3], sp[3];
@@ -583,11 +934,14 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
     tp[i] = (P.perm >> (2 * i)) & 3;
     sp[i] = (P.perm >> (6 + 2 * i)) & 3;
   }
+  // constant basis: in the order of the triangle numbers, as entry_sums
+  const bool sw = CC && CLS == CLS_VERTEX && sr.tri > sc.tri;
   uint32_t tv[3], sv[3];
 #pragma unroll
   for (int i = 0; i < 3; i++) {
-    tv[i] = sel3(sr.v, tp[i]);
-    sv[i] = sel3(sc.v, sp[i]);
+    const uint32_t tvi = sel3(sr.v, tp[i]), svi = sel3(sc.v, sp[i]);
+    tv[i] = sw ? svi : tvi;
+    sv[i] = sw ? tvi : svi;
   }
   double D0[3], E1[3], E2[3], F1[3], F2[3];
 #pragma unroll
@@ -602,34 +956,58 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
     F1[d] = Bs - As;
     F2[d] = Cs - Bs;
   }
-  double nx = 0.0, ny = 0.0, nz = 0.0;
+  // normals of the entry and of the exchanged pair, for d = x - y
+  double n1[3] = {0.0, 0.0, 0.0}, n2[3] = {0.0, 0.0, 0.0};
   if constexpr (DLP) {
-    double n64[3];
-    layer_normal(a, sr.tri, sc.tri, n64);
-    nx = n64[0];
-    ny = n64[1];
-    nz = n64[2];
+    layer_normal(a, sr.tri, sc.tri, n1);
+    if constexpr (TWO) layer_normal(a, sc.tri, sr.tri, n2);
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      n1[d] = sw ? -n1[d] : n1[d];
+      n2[d] = sw ? n2[d] : -n2[d];
+    }
   }
-  double Sre[NR][NC], Sim[NR][NC];
+  double Sre[ND][NR][NC], Sim[ND][NR][NC];
 #pragma unroll
-  for (int l = 0; l < NR; l++)
+  for (int z = 0; z < ND; z++)
 #pragma unroll
-    for (int k = 0; k < NC; k++) Sre[l][k] = Sim[l][k] = 0.0;
+    for (int l = 0; l < NR; l++)
+#pragma unroll
+      for (int k = 0; k < NC; k++) Sre[z][l][k] = Sim[z][l][k] = 0.0;
 
   // Moments M[a][b] = sum w v m_a(x) m_b(y) with m = (1, tx, sx) resp.
   // (1, ty, sy); the linear basis functions are phi = (1 - tx, tx - sx, sx)
   // = A m, so the element matrix A M A^T is formed once after the sum.
-  // kernel value at the difference d (FP64; mixed precision: d in FP64,
+  // kernel values at the difference d (FP64; mixed precision: d in FP64,
   // the value in FP32)
-  auto value = [&](const double *d, double &vre, double &vim) {
+  auto value = [&](const double *d, double (&vre)[ND], double (&vim)[ND]) {
     if constexpr (MP) {
-      float fre, fim;
-      kval32<KER>((float)d[0], (float)d[1], (float)d[2], (float)nx,
-                  (float)ny, (float)nz, a.krf, a.krev, a.kil2, fre, fim);
-      vre = fre;
-      vim = fim;
+      const float dx = (float)d[0], dy = (float)d[1], dz = (float)d[2];
+      float g, fr, fi;
+      kcore32<KER>(fmaf(dx, dx, fmaf(dy, dy, dz * dz)), a.krf, a.krev,
+                   a.kil2, g, fr, fi);
+#pragma unroll
+      for (int z = 0; z < ND; z++) {
+        const double *n = z ? n2 : n1;
+        float v = g;
+        if constexpr (DLP)
+          v *= fmaf(dx, (float)n[0], fmaf(dy, (float)n[1], dz * (float)n[2]));
+        vre[z] = CPLX ? fr * v : v;
+        vim[z] = CPLX ? fi * v : 0.0f;
+      }
     } else {
-      kval<KER>(d[0], d[1], d[2], nx, ny, nz, a.kr, a.ki, vre, vim);
+      double g, fr, fi;
+      kcore<KER>(fma(d[0], d[0], fma(d[1], d[1], d[2] * d[2])), a.kr, a.ki,
+                 0.0, g, fr, fi);
+#pragma unroll
+      for (int z = 0; z < ND; z++) {
+        const double *n = z ? n2 : n1;
+        double v = g;
+        if constexpr (DLP)
+          v *= fma(d[0], n[0], fma(d[1], n[1], d[2] * n[2]));
+        vre[z] = CPLX ? fr * v : v;
+        vim[z] = CPLX ? fi * v : 0.0;
+      }
     }
   };
   auto point = [&](double wq, double tx, double sx, double ty, double sy) {
@@ -638,11 +1016,11 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
     for (int k = 0; k < 3; k++)
       d[k] = fma(-F2[k], sy,
                  fma(-F1[k], ty, fma(E2[k], sx, fma(E1[k], tx, D0[k]))));
-    double vre, vim;
+    double vre[ND], vim[ND];
     value(d, vre, vim);
     double ure[NR], uim[NR];
-    ure[0] = wq * vre;
-    uim[0] = wq * vim;
+    ure[0] = wq * vre[0];
+    uim[0] = wq * vim[0];
     if constexpr (BR) {
       ure[1] = ure[0] * tx;
       ure[2] = ure[0] * sx;
@@ -651,14 +1029,14 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
     }
 #pragma unroll
     for (int l = 0; l < NR; l++) {
-      Sre[l][0] += ure[l];
-      if constexpr (CPLX) Sim[l][0] += uim[l];
+      Sre[0][l][0] += ure[l];
+      if constexpr (CPLX) Sim[0][l][0] += uim[l];
       if constexpr (BC) {
-        Sre[l][1] = fma(ure[l], ty, Sre[l][1]);
-        Sre[l][2] = fma(ure[l], sy, Sre[l][2]);
+        Sre[0][l][1] = fma(ure[l], ty, Sre[0][l][1]);
+        Sre[0][l][2] = fma(ure[l], sy, Sre[0][l][2]);
         if constexpr (CPLX) {
-          Sim[l][1] = fma(uim[l], ty, Sim[l][1]);
-          Sim[l][2] = fma(uim[l], sy, Sim[l][2]);
+          Sim[0][l][1] = fma(uim[l], ty, Sim[0][l][1]);
+          Sim[0][l][2] = fma(uim[l], sy, Sim[0][l][2]);
         }
       }
     }
@@ -711,8 +1089,12 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
             t1[d] = fma(-c1[d], e1, a1[d]);
             t2[d] = fma(b2[d], e1, a2[d]);
           }
-          double U0r = 0.0, U0i = 0.0, U2r = 0.0, U2i = 0.0;
-          double V0r = 0.0, V0i = 0.0, V2r = 0.0, V2i = 0.0;
+          double U0r[ND], U0i[ND], U2r[ND], U2i[ND];
+          double V0r[ND], V0i[ND], V2r[ND], V2i[ND];
+#pragma unroll
+          for (int z = 0; z < ND; z++)
+            U0r[z] = U0i[z] = U2r[z] = U2i[z] = V0r[z] = V0i[z] = V2r[z] =
+                V2i[z] = 0.0;
 #pragma unroll
           for (int j = 0; j < Q2; j++) {
             const double e2 = gn[j], w = wi1 * gw[j];
@@ -722,20 +1104,23 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
               d1[d] = fma(b1[d], e2, t1[d]);
               d2[d] = fma(c2[d], e2, t2[d]);
             }
-            double v1r, v1i, v2r, v2i;
+            double v1r[ND], v1i[ND], v2r[ND], v2i[ND];
             value(d1, v1r, v1i);
             value(d2, v2r, v2i);
-            const double u1r = w * v1r, u2r = w * v2r;
-            U0r += u1r;
-            U2r = fma(u1r, e2, U2r);
-            V0r += u2r;
-            V2r = fma(u2r, e2, V2r);
-            if constexpr (CPLX) {
-              const double u1i = w * v1i, u2i = w * v2i;
-              U0i += u1i;
-              U2i = fma(u1i, e2, U2i);
-              V0i += u2i;
-              V2i = fma(u2i, e2, V2i);
+#pragma unroll
+            for (int z = 0; z < ND; z++) {
+              const double u1r = w * v1r[z], u2r = w * v2r[z];
+              U0r[z] += u1r;
+              U2r[z] = fma(u1r, e2, U2r[z]);
+              V0r[z] += u2r;
+              V2r[z] = fma(u2r, e2, V2r[z]);
+              if constexpr (CPLX) {
+                const double u1i = w * v1i[z], u2i = w * v2i[z];
+                U0i[z] += u1i;
+                U2i[z] = fma(u1i, e2, U2i[z]);
+                V0i[z] += u2i;
+                V2i[z] = fma(u2i, e2, V2i[z]);
+              }
             }
           }
           // P1: row moments (U0, xi U0, xi U2), column moments
@@ -743,21 +1128,24 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
           // column moments (V0, xi V0, xi V2)
           const double f1 = e1 * xi, f2 = e1 * e3 * xi;
           const double ms[3] = {1.0, f1, f2};
-          const double p1r[3] = {U0r, xi * U0r, xi * U2r};
-          const double p1i[3] = {U0i, xi * U0i, xi * U2i};
-          const double p2r[3] = {V0r, xi * V0r, xi * V2r};
-          const double p2i[3] = {V0i, xi * V0i, xi * V2i};
 #pragma unroll
-          for (int l = 0; l < NR; l++)
+          for (int z = 0; z < ND; z++) {
+            const double p1r[3] = {U0r[z], xi * U0r[z], xi * U2r[z]};
+            const double p1i[3] = {U0i[z], xi * U0i[z], xi * U2i[z]};
+            const double p2r[3] = {V0r[z], xi * V0r[z], xi * V2r[z]};
+            const double p2i[3] = {V0i[z], xi * V0i[z], xi * V2i[z]};
 #pragma unroll
-            for (int kk = 0; kk < NC; kk++) {
-              Sre[l][kk] = fma(p1r[l], ms[kk], Sre[l][kk]);
-              Sre[l][kk] = fma(ms[l], p2r[kk], Sre[l][kk]);
-              if constexpr (CPLX) {
-                Sim[l][kk] = fma(p1i[l], ms[kk], Sim[l][kk]);
-                Sim[l][kk] = fma(ms[l], p2i[kk], Sim[l][kk]);
+            for (int l = 0; l < NR; l++)
+#pragma unroll
+              for (int kk = 0; kk < NC; kk++) {
+                Sre[z][l][kk] = fma(p1r[l], ms[kk], Sre[z][l][kk]);
+                Sre[z][l][kk] = fma(ms[l], p2r[kk], Sre[z][l][kk]);
+                if constexpr (CPLX) {
+                  Sim[z][l][kk] = fma(p1i[l], ms[kk], Sim[z][l][kk]);
+                  Sim[z][l][kk] = fma(ms[l], p2i[kk], Sim[z][l][kk]);
+                }
               }
-            }
+          }
         }
       } else if constexpr (CLS == CLS_EDGE) {
         // The six points of SSTuple<CLS_EDGE> with e1 = g_i, e2 = g_j,
@@ -816,13 +1204,13 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
                                          : Hv[d];
                 dd[d] = fma(cq, pq, bs[m][d]);
               }
-              double vr, vi;
+              double vr[ND], vi[ND];
               value(dd, vr, vi);
-              const double ur = w * vr;
+              const double ur = w * vr[0];
               W0r[m] += ur;
               W1r[m] = fma(ur, pq, W1r[m]);
               if constexpr (CPLX) {
-                const double ui = w * vi;
+                const double ui = w * vi[0];
                 W0i[m] += ui;
                 W1i[m] = fma(ui, pq, W1i[m]);
               }
@@ -858,8 +1246,8 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
                 Sx[l][kk] = t;
               }
           };
-          accum(W0r, W1r, Sre);
-          if constexpr (CPLX) accum(W0i, W1i, Sim);
+          accum(W0r, W1r, Sre[0]);
+          if constexpr (CPLX) accum(W0i, W1i, Sim[0]);
         }
       } else {
         // The six points of SSTuple<CLS_IDENTICAL> with eta = g_i,
@@ -890,7 +1278,7 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
           for (int i = 0; i < Q2; i++) {
             const double eta = gn[i], w = gw[i] * wj1;
             const double bb = x1 * (1.0 - eta);
-            double dv[3][3];
+            double dv[3][3], pr[3], pi[3];
 #pragma unroll
             for (int d = 0; d < 3; d++) {
               dv[0][d] = x1 * fma(eta, E1[d], E2[d]);
@@ -899,19 +1287,23 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
             }
 #pragma unroll
             for (int m = 0; m < 6; m++) {
-              double dd[3];
-#pragma unroll
-              for (int d = 0; d < 3; d++)
-                dd[d] = m < 3 ? dv[m][d] : -dv[m - 3][d];
-              double vr, vi;
-              value(dd, vr, vi);
               // point order: P1 = +u1, P2 = +u2, P3 = +u3, P4 = -u1,
-              // P5 = -u2, P6 = -u3
-              const double ur = w * vr;
+              // P5 = -u2, P6 = -u3; the kernels take -u to the same value
+              // (single layer) or to its negative (double layer)
+              double vr[ND], vi[ND];
+              if (m < 3) {
+                value(dv[m], vr, vi);
+                pr[m] = vr[0];
+                pi[m] = vi[0];
+              } else {
+                vr[0] = DLP ? -pr[m - 3] : pr[m - 3];
+                vi[0] = DLP ? -pi[m - 3] : pi[m - 3];
+              }
+              const double ur = w * vr[0];
               W0r[m] += ur;
               W1r[m] = fma(ur, bb, W1r[m]);
               if constexpr (CPLX) {
-                const double ui = w * vi;
+                const double ui = w * vi[0];
                 W0i[m] += ui;
                 W1i[m] = fma(ui, bb, W1i[m]);
               }
@@ -949,8 +1341,8 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
                 Sx[l][kk] = t;
               }
           };
-          accum(W0r, W1r, Sre);
-          if constexpr (CPLX) accum(W0i, W1i, Sim);
+          accum(W0r, W1r, Sre[0]);
+          if constexpr (CPLX) accum(W0i, W1i, Sim[0]);
         }
       }
     }
@@ -969,32 +1361,35 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
     }
   }
 #pragma unroll
-  for (int l = 0; l < NR; l++)
+  for (int z = 0; z < ND; z++) {
 #pragma unroll
-    for (int k = 0; k < NC; k++) {
-      Sre[l][k] = row_sum(Sre[l][k]);
-      if constexpr (CPLX) Sim[l][k] = row_sum(Sim[l][k]);
-    }
-  // moments -> element matrix: (1, t, s) -> (1 - t, t - s, s) on each side
-  if constexpr (BR) {
+    for (int l = 0; l < NR; l++)
 #pragma unroll
-    for (int k = 0; k < NC; k++) {
-      Sre[0][k] -= Sre[1][k];
-      Sre[1][k] -= Sre[2][k];
-      if constexpr (CPLX) {
-        Sim[0][k] -= Sim[1][k];
-        Sim[1][k] -= Sim[2][k];
+      for (int k = 0; k < NC; k++) {
+        Sre[z][l][k] = row_sum(Sre[z][l][k]);
+        if constexpr (CPLX) Sim[z][l][k] = row_sum(Sim[z][l][k]);
+      }
+    // moments -> element matrix: (1, t, s) -> (1 - t, t - s, s) on each side
+    if constexpr (BR) {
+#pragma unroll
+      for (int k = 0; k < NC; k++) {
+        Sre[z][0][k] -= Sre[z][1][k];
+        Sre[z][1][k] -= Sre[z][2][k];
+        if constexpr (CPLX) {
+          Sim[z][0][k] -= Sim[z][1][k];
+          Sim[z][1][k] -= Sim[z][2][k];
+        }
       }
     }
-  }
-  if constexpr (BC) {
+    if constexpr (BC) {
 #pragma unroll
-    for (int l = 0; l < NR; l++) {
-      Sre[l][0] -= Sre[l][1];
-      Sre[l][1] -= Sre[l][2];
-      if constexpr (CPLX) {
-        Sim[l][0] -= Sim[l][1];
-        Sim[l][1] -= Sim[l][2];
+      for (int l = 0; l < NR; l++) {
+        Sre[z][l][0] -= Sre[z][l][1];
+        Sre[z][l][1] -= Sre[z][l][2];
+        if constexpr (CPLX) {
+          Sim[z][l][0] -= Sim[z][l][1];
+          Sim[z][l][1] -= Sim[z][l][2];
+        }
       }
     }
   }
@@ -1002,22 +1397,33 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
   // lane e hands over the entry of permuted local functions (l, k) =
   // (e % NR, e / NR)
   const int l = sub % NR, k = sub / NR;
-  double vre = 0.0, vim = 0.0;
+  double vre[2] = {0.0, 0.0}, vim[2] = {0.0, 0.0};
 #pragma unroll
-  for (int ll = 0; ll < NR; ll++)
+  for (int z = 0; z < ND; z++)
 #pragma unroll
-    for (int kk = 0; kk < NC; kk++)
-      if (ll == l && kk == k) {
-        vre = Sre[ll][kk];
-        vim = Sim[ll][kk];
-      }
+    for (int ll = 0; ll < NR; ll++)
+#pragma unroll
+      for (int kk = 0; kk < NC; kk++)
+        if (ll == l && kk == k) {
+          vre[z] = Sre[z][ll][kk];
+          vim[z] = Sim[z][ll][kk];
+        }
+  if constexpr (MIR && !TWO) {
+    // single layer: the same sums; identical triangles, double layer: the
+    // differences change sign and the normal does not
+    vre[1] = DLP ? -vre[0] : vre[0];
+    vim[1] = DLP ? -vim[0] : vim[0];
+  }
   const uint32_t lr = loc_of(sr.loc, BR ? sel3(tp, l) : 0);
   const uint32_t lc = loc_of(sc.loc, BC ? sel3(sp, k) : 0);
   if (lr == 0xffu || lc == 0xffu) return;
   const double gt = a.g[sr.tri];
-  const double f2 = a.kc * gt * a.g[sc.tri];
-  vre *= f2;
-  vim *= f2;
+  const double f2 = pair_factor<CC>(a, sr.tri, sc.tri);
+#pragma unroll
+  for (int z = 0; z < 2; z++) {
+    vre[z] *= f2;
+    vim[z] *= f2;
+  }
   if constexpr (CLS == CLS_IDENTICAL) {
     // identity term of the double layer on identical triangles (tp, sp are
     // the identity here): cc at (t, t) of the block
@@ -1025,8 +1431,8 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
     // (Library/bem3d.c:3205-3242, 1934-1966, 2530-2562)
     if constexpr (CC) {
       if (T.row0 + lr == T.col0 + lc) {
-        vre += 0.5 * a.are * gt;
-        vim += 0.5 * a.aim * gt;
+        vre[0] += 0.5 * a.are * gt;
+        vim[0] += 0.5 * a.aim * gt;
       }
     } else {
       // the linear-basis integrators hold alpha g in a real variable
@@ -1035,17 +1441,20 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
       const bool allowed = (BR && !BC) ? (T.flags & 1) : true;
       if (allowed) {
         const double m = (BR && BC) ? a.mass[l + 3 * k] : a.mass[BR ? l : k];
-        vre += m * a.are * gt;
+        vre[0] += m * a.are * gt;
+        vre[1] += m * a.are * gt;  // the mass matrix is symmetric
       }
     }
   }
-  sink(lr, lc, vre, vim);
+  sink(lr, lc, vre[0], vim[0], vre[1], vim[1]);
 }
 
 // The pairs with common vertices of one rule class, one pair per row of 16
 // lanes (16 pairs per workgroup), added into the output with FP64 atomics
 // (the regular kernel has stored the tiles before).
-template <int KER, int BR, int BC, int CLS, int Q2, bool MP>
+// MIR: the list holds one of each two exchanged pairs; the other's entry is
+// added into the mirror tile.
+template <int KER, int BR, int BC, int CLS, int Q2, bool MP, bool MIR>
 __global__ __launch_bounds__(NTHREADS) void nf_singular_kernel(
     KArgs a, const SPair *__restrict__ list, uint32_t npairs) {
   constexpr bool CPLX = KER >= K_HELM_SLP;
@@ -1055,8 +1464,13 @@ __global__ __launch_bounds__(NTHREADS) void nf_singular_kernel(
   const SPair P = list[w];
   const Tile T = a.tiles[P.tile];
   const bool conj = T.ntrans && (BR == BC);
-  singular_pair<KER, BR, BC, CLS, Q2, MP>(
-      a, T, P, sub, [&](uint32_t lr, uint32_t lc, double vre, double vim) {
+  // identical triangles of a diagonal tile have no exchanged pair
+  const bool mir =
+      MIR && !(CLS == CLS_IDENTICAL && T.mirror == P.tile);
+  singular_pair<KER, BR, BC, CLS, Q2, MP, MIR>(
+      a, T, P, sub,
+      [&](uint32_t lr, uint32_t lc, double vre, double vim, double vre2,
+          double vim2) {
         const size_t pos =
             T.out_off + (T.ntrans ? (size_t)lc + (size_t)lr * T.ld
                                   : (size_t)lr + (size_t)lc * T.ld);
@@ -1065,6 +1479,16 @@ __global__ __launch_bounds__(NTHREADS) void nf_singular_kernel(
           atomicAdd(&a.out[2 * pos + 1], conj ? -vim : vim);
         } else {
           atomicAdd(&a.out[pos], vre);
+        }
+        if (mir) {
+          const Tile &M = a.tiles[T.mirror];
+          const size_t mpos = M.out_off + (size_t)lc + (size_t)lr * M.ld;
+          if constexpr (CPLX) {
+            atomicAdd(&a.out[2 * mpos], vre2);
+            atomicAdd(&a.out[2 * mpos + 1], vim2);
+          } else {
+            atomicAdd(&a.out[mpos], vre2);
+          }
         }
       });
 }
@@ -1085,9 +1509,10 @@ __device__ __forceinline__ void tile_singular(const KArgs &a, const Tile &T,
   for (uint32_t p0 = 0; p0 < n; p0 += NTHREADS / 16) {
     const uint32_t w = p0 + row;
     if (w >= n) continue;  // uniform per row of 16 lanes
-    singular_pair<KER, BR, BC, CLS, Q2, MP>(
+    singular_pair<KER, BR, BC, CLS, Q2, MP, false>(
         a, T, list[w], sub,
-        [&](uint32_t lr, uint32_t lc, double vre, double vim) {
+        [&](uint32_t lr, uint32_t lc, double vre, double vim, double,
+            double) {
           if constexpr (CC) {
             const size_t pos =
                 T.out_off + (T.ntrans ? (size_t)lc + (size_t)lr * T.ld
@@ -1136,6 +1561,36 @@ int launch_bases_p(uint32_t q, const KArgs &a, uint32_t ntiles,
     }
     return H2HIP_OK;
   }
+  constexpr bool SMP = MP != 0;
+  constexpr uint32_t PPB = NTHREADS / 16;  // pairs per workgroup
+  auto singular = [&](void (*k)(KArgs, const SPair *, uint32_t),
+                      const SPair *list, uint32_t n) {
+    if (n)
+      hipLaunchKernelGGL(k, dim3((n + PPB - 1) / PPB), dim3(NTHREADS), 0,
+                         stream, a, list, n);
+  };
+  const uint32_t n3 = ncls[CLS_IDENTICAL], n2 = ncls[CLS_EDGE],
+                 n1 = ncls[CLS_VERTEX];
+  if constexpr (BR == BC) {
+    // mirrored tiles: half the regular, vertex and (linear basis) identical
+    // pairs; the lists hold the pairs to evaluate first
+    if (a.nmir && !a.far && q == 2 && a.q2 == 4) {
+      if constexpr (paired(KER, BR, BC, MP))
+        hipLaunchKernelGGL((nf_pair_kernel<KER, BR, 2, MP>), dim3(a.nmir),
+                           dim3(pair_threads(KER, BR)), 0, stream, a,
+                           a.mirlist);
+      else
+        hipLaunchKernelGGL((nf_regular_kernel<KER, BR, BC, 2, MP>),
+                           dim3(ntiles), dim3(NTHREADS), 0, stream, a);
+      singular(nf_singular_kernel<KER, BR, BC, CLS_IDENTICAL, 4, SMP, BR != 0>,
+               sp, BR ? a.nmain3 : n3);
+      singular(nf_singular_kernel<KER, BR, BC, CLS_EDGE, 4, SMP, false>,
+               sp + n3, n2);
+      singular(nf_singular_kernel<KER, BR, BC, CLS_VERTEX, 4, SMP, true>,
+               sp + n3 + n2, a.nmain1);
+      return H2HIP_OK;
+    }
+  }
   if (ntiles && a.counter) {
     void (*reg)(KArgs, uint32_t, uint32_t *) = nullptr;
     switch (q) {
@@ -1169,27 +1624,16 @@ int launch_bases_p(uint32_t q, const KArgs &a, uint32_t ntiles,
     hipLaunchKernelGGL(reg, dim3(ntiles), dim3(NTHREADS), 0, stream, a);
   }
   if (a.far) return H2HIP_OK;
-  constexpr uint32_t PPB = NTHREADS / 16;  // pairs per workgroup
-  const uint32_t n3 = ncls[CLS_IDENTICAL], n2 = ncls[CLS_EDGE],
-                 n1 = ncls[CLS_VERTEX];
-  using SK = void (*)(KArgs, const SPair *, uint32_t);
   const bool q4 = a.q2 == 4;
-  constexpr bool SMP = MP != 0;
-  const SK k3 = q4 ? nf_singular_kernel<KER, BR, BC, CLS_IDENTICAL, 4, SMP>
-                   : nf_singular_kernel<KER, BR, BC, CLS_IDENTICAL, 0, SMP>;
-  const SK k2 = q4 ? nf_singular_kernel<KER, BR, BC, CLS_EDGE, 4, SMP>
-                   : nf_singular_kernel<KER, BR, BC, CLS_EDGE, 0, SMP>;
-  const SK k1 = q4 ? nf_singular_kernel<KER, BR, BC, CLS_VERTEX, 4, SMP>
-                   : nf_singular_kernel<KER, BR, BC, CLS_VERTEX, 0, SMP>;
-  if (n3)
-    hipLaunchKernelGGL(k3, dim3((n3 + PPB - 1) / PPB), dim3(NTHREADS), 0,
-                       stream, a, sp, n3);
-  if (n2)
-    hipLaunchKernelGGL(k2, dim3((n2 + PPB - 1) / PPB), dim3(NTHREADS), 0,
-                       stream, a, sp + n3, n2);
-  if (n1)
-    hipLaunchKernelGGL(k1, dim3((n1 + PPB - 1) / PPB), dim3(NTHREADS), 0,
-                       stream, a, sp + n3 + n2, n1);
+  singular(q4 ? nf_singular_kernel<KER, BR, BC, CLS_IDENTICAL, 4, SMP, false>
+              : nf_singular_kernel<KER, BR, BC, CLS_IDENTICAL, 0, SMP, false>,
+           sp, n3);
+  singular(q4 ? nf_singular_kernel<KER, BR, BC, CLS_EDGE, 4, SMP, false>
+              : nf_singular_kernel<KER, BR, BC, CLS_EDGE, 0, SMP, false>,
+           sp + n3, n2);
+  singular(q4 ? nf_singular_kernel<KER, BR, BC, CLS_VERTEX, 4, SMP, false>
+              : nf_singular_kernel<KER, BR, BC, CLS_VERTEX, 0, SMP, false>,
+           sp + n3 + n2, n1);
   return H2HIP_OK;
 }
 
@@ -1200,10 +1644,14 @@ int launch_bases_p(uint32_t q, const KArgs &a, uint32_t ntiles,
 template <int KER, int BR, int BC>
 int launch_bases(uint32_t q, const KArgs &a, uint32_t ntiles,
                  const SPair *sp, const uint32_t *ncls, hipStream_t stream) {
-  if (a.mp == 2)
-    return launch_bases_p<KER, BR, BC, 2>(q, a, ntiles, sp, ncls, stream);
-  if (a.mp == 1)
-    return launch_bases_p<KER, BR, BC, 1>(q, a, ntiles, sp, ncls, stream);
+  if constexpr (!small_phase(KER)) {
+    // (the FP32 kernels reduce every phase: their sine and cosine take
+    // revolutions)
+    if (a.mp == 2)
+      return launch_bases_p<KER, BR, BC, 2>(q, a, ntiles, sp, ncls, stream);
+    if (a.mp == 1)
+      return launch_bases_p<KER, BR, BC, 1>(q, a, ntiles, sp, ncls, stream);
+  }
   return launch_bases_p<KER, BR, BC, 0>(q, a, ntiles, sp, ncls, stream);
 }
 

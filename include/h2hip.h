@@ -156,7 +156,10 @@ int h2hip_nearfield_flush(const h2hip_op *op);
  * packed output stores block b column-major with leading dimension rows at
  * element offset off[b] (h2hip_nfplan_offsets).  This is the near-field
  * part of assemble_bem3d_h2matrix (Library/bem3d.c:10313-10346), which calls
- * bem->nearfield for every inadmissible leaf block. */
+ * bem->nearfield for every inadmissible leaf block.  Where both sides have
+ * one basis and equal index arrays and every block comes with its mirror
+ * (cols x rows), the default schedule evaluates each pair of triangles once
+ * for both entries. */
 int h2hip_nfplan_create(h2hip_nfplan **out, const h2hip_surface *s,
                         int row_basis, int col_basis,
                         const uint32_t *ridx_all, uint32_t nridx,

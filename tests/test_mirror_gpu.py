@@ -1,0 +1,98 @@
+"""Mirrored tiles of the near-field plan (needs a GPU).
+
+A plan over one index array whose blocks come in mirrored pairs evaluates
+each pair of triangles once for both entries; the persistent schedule does
+not, and evaluates every tile for itself.  Constant basis: the same bits;
+linear basis: the same up to the order of the sums (1e-14 of the largest
+entry, a few thousand terms).  Both against the oracle to 1e-12.  The blocks
+have sides of 1, 2, 63, 64 and 65 DOFs (diagonal tiles of odd and even
+size, tile edges and remainders).
+"""
+import numpy as np
+import pytest
+
+from conftest import rel_block_err
+from oracle_ffi import OracleBem
+
+pytestmark = pytest.mark.gpu
+
+SIDES = (1, 2, 63, 64, 65)
+
+
+def mirrored_blocks(sides=SIDES):
+    off = np.concatenate([[0], np.cumsum(sides)])
+    return [(int(off[i]), sides[i], int(off[j]), sides[j])
+            for i in range(len(sides)) for j in range(len(sides))]
+
+
+def run(h, plan, op, schedule):
+    plan.set_schedule(*schedule)
+    out = h.DeviceArray(plan.entries, op.dtype)
+    out.fill_nan()
+    stream = h.Stream()
+    plan.execute(op, out.ptr, stream.handle)
+    stream.sync()
+    return out.download()
+
+
+# wave numbers on both sides of the small-phase bound 2 |k| h <= pi/4 (k = 1.3
+# and 1.31 on this mesh, h = 0.3015), and a damped one
+@pytest.mark.parametrize("kern,k", [(0, 0.0), (1, 1.3), (1, 1.31),
+                                    (1, 1.3 + 0.5j)])
+@pytest.mark.parametrize("layer", [0, 1, 2])
+@pytest.mark.parametrize("basis", [0, 1])
+def test_mirrored_tiles_match_single_tiles(kern, k, layer, basis, sphere8):
+    import h2lib_amd as h
+    gr = h.Surface3d(sphere8["x"], sphere8["t"])
+    n = gr.vertices if basis else gr.triangles
+    idx = np.random.default_rng(3).permutation(n).astype(np.uint32)
+    blocks = mirrored_blocks()
+    plan = h.NearfieldPlan(gr, basis, basis, idx, idx.copy(), blocks)
+    alpha = 0.5 if layer else 0.0
+    op = h.Bem3d(gr, kern, layer, 2, 4, basis, basis, alpha=alpha, k=k)
+    orc = OracleBem(kern, layer, basis, basis, sphere8["x"], sphere8["t"],
+                    q=2, q2=4, alpha=alpha, k=k)
+    for mode in (0, 1, 2):
+        op.set_precision(mode)
+        got = run(h, plan, op, (0, 0, 0))
+        want = run(h, plan, op, (0, 1, 0))
+        if basis == 0:
+            assert np.array_equal(got, want), mode
+        else:
+            err = np.abs(got - want).max() / np.abs(want).max()
+            # mixed precision sums FP32 values formed from the other
+            # triangle's anchor point: FP32 rounding of the entries
+            assert err < (1e-14 if mode == 0 else 2e-6), (mode, err)
+        if mode == 0:
+            for b in (0, 1, 6, 12, 14, 18, 22, 24):
+                ro, r, co, c = blocks[b]
+                ref = orc.nearfield(idx[ro:ro + r], idx[co:co + c])
+                assert rel_block_err(plan.block(got, b), ref) < 1e-12, b
+
+
+@pytest.mark.parametrize("basis", [0, 1])
+def test_unpaired_and_repeated_blocks_keep_single_tiles(basis, sphere8):
+    """A block without its mirror, a block listed twice and index arrays that
+    repeat DOFs take the general path or give its entries."""
+    import h2lib_amd as h
+    gr = h.Surface3d(sphere8["x"], sphere8["t"])
+    n = gr.vertices if basis else gr.triangles
+    rng = np.random.default_rng(4)
+    idx = rng.permutation(n).astype(np.uint32)
+    rep = idx.copy()
+    rep[10] = rep[70]
+    rep[71] = rep[72]
+    op = h.Bem3d(gr, 0, 1, 2, 4, basis, basis, alpha=0.5)
+    orc = OracleBem(0, 1, basis, basis, sphere8["x"], sphere8["t"], q=2,
+                    q2=4, alpha=0.5)
+    full = mirrored_blocks()
+    for ix, blocks in ((idx, full[:-1]), (idx, full + full[1:2]),
+                       (rep, full)):
+        plan = h.NearfieldPlan(gr, basis, basis, ix, ix, blocks)
+        got = run(h, plan, op, (0, 0, 0))
+        want = run(h, plan, op, (0, 1, 0))
+        scale = np.abs(want).max()
+        assert np.abs(got - want).max() <= (1e-14 * scale if basis else 0.0)
+        for b, (ro, r, co, c) in enumerate(blocks):
+            ref = orc.nearfield(ix[ro:ro + r], ix[co:co + c])
+            assert rel_block_err(plan.block(got, b), ref) < 1e-12, b
