@@ -56,17 +56,6 @@ template <class T> struct DevBuf {
     if (e != hipSuccess || count == 0) return e;
     return hipMemcpy(p, src, sizeof(T) * count, hipMemcpyHostToDevice);
   }
-  // as upload, but keeps an allocation that is large enough (n is then the
-  // capacity), ordered on a stream
-  hipError_t upload_grow(const T *src, size_t count, hipStream_t st) {
-    if (count == 0) return hipSuccess;
-    if (!p || n < count) {
-      hipError_t e = alloc(count);
-      if (e != hipSuccess) return e;
-    }
-    return hipMemcpyAsync(p, src, sizeof(T) * count, hipMemcpyHostToDevice,
-                          st);
-  }
 };
 
 // ---- quadrature rules (host) -------------------------------------------------
@@ -118,7 +107,8 @@ struct Tile {
   uint8_t nr, nc;       // tile size
   uint8_t ntrans;
   uint8_t flags;        // bit 0: identity term allowed (lc quirk)
-  // the tile's pairs with common vertices in the list grouped by tile:
+  // the tile's pairs with common vertices in the list grouped by tile (set
+  // for the fused schedule):
   // from sbeg, ns[0] identical, then ns[1] edge, then ns[2] vertex pairs
   uint32_t sbeg;
   uint16_t ns[3];
@@ -174,6 +164,10 @@ struct KArgs {
   // first in their class's list)
   const uint32_t *mirlist;
   uint32_t nmir, nmain3, nmain1;
+  // workgroups per tile of the regular launch; more than one with the
+  // linear basis add into the output (entries elements), zeroed before
+  uint32_t split;
+  uint64_t entries;
 };
 
 // Launches the regular tile kernel over `ntiles` tiles and then (unless
@@ -280,17 +274,20 @@ struct h2hip_nfplan {
   std::vector<h2hip::Supp> supp;
   std::vector<h2hip::Fixup> fix;
   std::vector<h2hip::SPair> spairs;  // sorted by class, identical first
-  std::vector<h2hip::SPair> tpairs;  // grouped by tile (Tile::sbeg, ns)
   uint64_t pairs[4] = {0, 0, 0, 0};  // support pairs per class
   // mirrored tiles (nf::KArgs::mirlist), empty unless every tile has its
   // mirror
   std::vector<uint32_t> mirlist;
   uint32_t nmain[4] = {0, 0, 0, 0};
-  h2hip::DevBuf<uint32_t> d_mirlist;
-  h2hip::DevBuf<h2hip::Tile> d_tiles;
-  h2hip::DevBuf<h2hip::Supp> d_supp;
-  h2hip::DevBuf<h2hip::Fixup> d_fix;
-  h2hip::DevBuf<h2hip::SPair> d_spairs;
+  // the lists on the device, in one allocation (small plans: one copy from
+  // h_lists)
+  h2hip::DevBuf<unsigned char> d_lists;
+  std::vector<unsigned char> h_lists;
+  h2hip::Tile *d_tiles = nullptr;
+  h2hip::Supp *d_supp = nullptr;
+  h2hip::Fixup *d_fix = nullptr;
+  h2hip::SPair *d_spairs = nullptr;
+  uint32_t *d_mirlist = nullptr;
   // schedule: tiles in decreasing order of their pair count, and the
   // persistent regular kernel with its tile counter
   int sorted = 0, persistent = 0;

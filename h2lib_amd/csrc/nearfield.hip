@@ -289,6 +289,45 @@ void set_mirrors(std::vector<Tile> &tiles, const std::vector<uint64_t> &key,
   }
 }
 
+// Copies the plan's lists to the device, into one allocation.  grow: keeps
+// one that is large enough, ordered on st (otherwise complete on return).
+// Each allocation and each small copy costs 10 us and more, as much as a
+// small block's kernels, so lists of up to 1 MB are put together first.
+int upload_lists(h2hip_nfplan *P, bool grow, hipStream_t st) {
+  const void *src[5] = {P->tiles.data(), P->supp.data(), P->fix.data(),
+                        P->spairs.data(), P->mirlist.data()};
+  const size_t bytes[5] = {
+      sizeof(Tile) * P->tiles.size(), sizeof(Supp) * P->supp.size(),
+      sizeof(Fixup) * P->fix.size(), sizeof(SPair) * P->spairs.size(),
+      sizeof(uint32_t) * P->mirlist.size()};
+  size_t off[6] = {0};
+  for (int i = 0; i < 5; i++)
+    off[i + 1] = off[i] + (bytes[i] + 255) / 256 * 256;
+  const size_t total = off[5];
+  if (!grow || !P->d_lists.p || P->d_lists.n < total)
+    H2HIP_CHECK(P->d_lists.alloc(total));
+  unsigned char *d = P->d_lists.p;
+  P->d_tiles = (Tile *)(d + off[0]);
+  P->d_supp = (Supp *)(d + off[1]);
+  P->d_fix = (Fixup *)(d + off[2]);
+  P->d_spairs = (SPair *)(d + off[3]);
+  P->d_mirlist = (uint32_t *)(d + off[4]);
+  auto copy = [&](void *dst, const void *from, size_t n) {
+    if (n == 0) return hipSuccess;
+    return grow ? hipMemcpyAsync(dst, from, n, hipMemcpyHostToDevice, st)
+                : hipMemcpy(dst, from, n, hipMemcpyHostToDevice);
+  };
+  if (total <= ((size_t)1 << 20)) {
+    P->h_lists.resize(total);
+    for (int i = 0; i < 5; i++)
+      if (bytes[i]) std::memcpy(P->h_lists.data() + off[i], src[i], bytes[i]);
+    H2HIP_CHECK(copy(d, P->h_lists.data(), total));
+    return H2HIP_OK;
+  }
+  for (int i = 0; i < 5; i++) H2HIP_CHECK(copy(d + off[i], src[i], bytes[i]));
+  return H2HIP_OK;
+}
+
 // ntr: per-block ntrans flags (nullptr: ntrans for every block); st: the
 // uploads keep large enough device buffers of P and are ordered on st
 // (otherwise new buffers, complete on return).
@@ -308,7 +347,6 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
   P->supp.clear();
   P->fix.clear();
   P->spairs.clear();
-  P->tpairs.clear();
   // a fused schedule is set again for the new plan
   P->fused = 0;
   P->d_tiles_f.release();
@@ -342,8 +380,11 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
   P->entries = total;
 
   // Mirrored tiles need one index array (and basis) on both sides
+  const bool plain =
+      ntr ? std::all_of(ntr, ntr + nblocks, [](uint8_t t) { return !t; })
+          : !ntrans;
   const bool mirrors =
-      rb == cb && nridx == ncidx && !ntr && !ntrans &&
+      rb == cb && nridx == ncidx && plain &&
       (ridx_all == cidx_all ||
        std::memcmp(ridx_all, cidx_all, sizeof(uint32_t) * nridx) == 0);
 
@@ -544,9 +585,7 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
   struct SPart {
     std::vector<SPair> by_cls[4];
     size_t nmain[4] = {0, 0, 0, 0};  // pairs to evaluate (mirrored tiles)
-    std::vector<SPair> tp;  // grouped by tile
     uint64_t pairs0 = 0;
-    std::string err;
   };
   const uint32_t ntiles = (uint32_t)P->tiles.size();
   const bool mir = !P->mirlist.empty();
@@ -565,15 +604,15 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
                   [&](unsigned t, uint32_t lo, uint32_t hi) {
     SPart &W = sparts[t];
     std::vector<int32_t> cpos(s->nt, -1), cnext;
+    std::vector<uint32_t> met;  // row that last met the triangle at c
     for (uint32_t ti = lo; ti < hi; ti++) {
-      Tile &T = P->tiles[ti];
+      const Tile &T = P->tiles[ti];
       W.pairs0 += (uint64_t)T.nrsup * T.ncsup;
-      size_t b0[4];
-      for (int c = 1; c < 4; c++) b0[c] = W.by_cls[c].size();
       // the first column position of each triangle; the further positions
       // of a triangle that the column indices repeat (constant basis)
       // chained behind it in increasing order
       cnext.assign(T.ncsup, -1);
+      met.assign(T.ncsup, 0);
       for (uint32_t c = T.ncsup; c-- > 0;) {
         const uint32_t tri = P->supp[T.csup + c].tri;
         cnext[c] = cpos[tri];
@@ -581,17 +620,12 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
       }
       for (uint32_t r = 0; r < T.nrsup; r++) {
         const Supp &sr = P->supp[T.rsup + r];
-        uint32_t seen[64];
-        int nseen = 0;
         for (int l = 0; l < 3; l++) {
           const uint32_t v = sr.v[l];
           for (uint32_t p = s->v2t_ptr[v]; p < s->v2t_ptr[v + 1]; p++) {
             const uint32_t tri = s->v2t[p];
-            if (cpos[tri] < 0) continue;
-            bool dup = false;
-            for (int k = 0; k < nseen; k++) dup |= (seen[k] == tri);
-            if (dup) continue;
-            if (nseen < 64) seen[nseen++] = tri;
+            if (cpos[tri] < 0 || met[cpos[tri]] == r + 1) continue;
+            met[cpos[tri]] = r + 1;
             for (int32_t c = cpos[tri]; c >= 0; c = cnext[c]) {
               SPair q;
               q.tile = ti;
@@ -607,37 +641,15 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
       }
       for (uint32_t c = 0; c < T.ncsup; c++)
         cpos[P->supp[T.csup + c].tri] = -1;
-      // the tile's pairs again, grouped by tile: identical, edge, vertex
-      T.sbeg = (uint32_t)W.tp.size();  // relative to the part's list
-      for (int c = 3; c >= 1; c--) {
-        const size_t cnt = W.by_cls[c].size() - b0[c];
-        if (cnt > 0xffff) {
-          W.err = "too many pairs with common vertices in one tile";
-          return;
-        }
-        T.ns[3 - c] = (uint16_t)cnt;
-        W.tp.insert(W.tp.end(), W.by_cls[c].begin() + b0[c],
-                    W.by_cls[c].end());
-      }
     }
   });
-  for (auto &W : sparts) {
-    if (!W.err.empty()) {
-      set_error(W.err);
-      return H2HIP_EINVAL;
-    }
-  }
-  // where each part's pairs go: the tile-grouped list in part order; the
-  // class lists (identical, edge, vertex) one after the other, each in part
-  // order; then the parts copy their pieces at the same time
+  // where each part's pairs go: the class lists (identical, edge, vertex)
+  // one after the other, each in part order; then the parts copy their
+  // pieces at the same time
   const unsigned np = (unsigned)sparts.size();
-  std::vector<size_t> tdst(np), cdst(4 * (size_t)np), odst(4 * (size_t)np);
-  size_t ntp = 0, nsp = 0;
-  for (unsigned part = 0; part < np; part++) {
-    tdst[part] = ntp;
-    ntp += sparts[part].tp.size();
-    P->pairs[0] += sparts[part].pairs0;
-  }
+  std::vector<size_t> cdst(4 * (size_t)np), odst(4 * (size_t)np);
+  size_t nsp = 0;
+  for (auto &W : sparts) P->pairs[0] += W.pairs0;
   for (int c = 3; c >= 1; c--) {
     // mirrored tiles: the pairs to evaluate first, then the others
     size_t nmain = 0;
@@ -658,20 +670,15 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
     P->nmain[c] = (uint32_t)nmain;
     P->pairs[0] -= P->pairs[c];
   }
-  if (ntp > 0xffffffffull) {
+  if (nsp > 0xffffffffull) {
     set_error("too many pairs with common vertices");
     return H2HIP_EINVAL;
   }
-  P->tpairs.resize(ntp);
   P->spairs.resize(nsp);
-  parallel_ranges(np, np, [&](unsigned, uint32_t lo, uint32_t hi) {
+  // (threads only where the copies take longer than starting them)
+  parallel_ranges(np, nsp > 200000 ? np : 1, [&](unsigned, uint32_t lo, uint32_t hi) {
     for (uint32_t part = lo; part < hi; part++) {
       SPart &W = sparts[part];
-      const uint32_t t0 = (uint32_t)((uint64_t)ntiles * part / np);
-      const uint32_t t1 = (uint32_t)((uint64_t)ntiles * (part + 1) / np);
-      for (uint32_t ti = t0; ti < t1; ti++)
-        P->tiles[ti].sbeg += (uint32_t)tdst[part];
-      std::copy(W.tp.begin(), W.tp.end(), P->tpairs.begin() + tdst[part]);
       for (int c = 1; c < 4; c++) {
         auto first = P->spairs.begin() + cdst[4 * part + c],
              rest = P->spairs.begin() + odst[4 * part + c];
@@ -685,22 +692,7 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
     }
   });
   sparts.clear();
-  if (grow) {
-    H2HIP_CHECK(P->d_tiles.upload_grow(P->tiles.data(), P->tiles.size(), st));
-    H2HIP_CHECK(P->d_supp.upload_grow(P->supp.data(), P->supp.size(), st));
-    H2HIP_CHECK(P->d_fix.upload_grow(P->fix.data(), P->fix.size(), st));
-    H2HIP_CHECK(
-        P->d_spairs.upload_grow(P->spairs.data(), P->spairs.size(), st));
-    H2HIP_CHECK(
-        P->d_mirlist.upload_grow(P->mirlist.data(), P->mirlist.size(), st));
-    return H2HIP_OK;
-  }
-  H2HIP_CHECK(P->d_tiles.upload(P->tiles.data(), P->tiles.size()));
-  H2HIP_CHECK(P->d_supp.upload(P->supp.data(), P->supp.size()));
-  H2HIP_CHECK(P->d_fix.upload(P->fix.data(), P->fix.size()));
-  H2HIP_CHECK(P->d_spairs.upload(P->spairs.data(), P->spairs.size()));
-  H2HIP_CHECK(P->d_mirlist.upload(P->mirlist.data(), P->mirlist.size()));
-  return H2HIP_OK;
+  return upload_lists(P, grow, st);
 }
 
 int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
@@ -712,8 +704,8 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
   if (P->tiles.empty()) return H2HIP_OK;
   const h2hip_surface *s = op->s;
   nf::KArgs a;
-  a.tiles = P->d_tiles.p;
-  a.supp = P->d_supp.p;
+  a.tiles = P->d_tiles;
+  a.supp = P->d_supp;
   a.x = s->d_x.p;
   a.n = s->d_n.p;
   a.g = s->d_g.p;
@@ -741,10 +733,29 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
   // mirrored tiles in the launches per rule class of the plan's own order
   const bool mir = !P->mirlist.empty() && !P->sorted && !P->persistent &&
                    !P->fused && !far;
-  a.mirlist = P->d_mirlist.p;
+  a.mirlist = P->d_mirlist;
   a.nmir = mir ? (uint32_t)P->mirlist.size() : 0;
   a.nmain3 = P->nmain[CLS_IDENTICAL];
   a.nmain1 = P->nmain[CLS_VERTEX];
+  // Plans of few tiles: a 64-DOF linear-basis tile keeps one workgroup busy
+  // for 150 us whatever else is idle, so its pairs are split over several
+  // workgroups until about four per CU are there, each with at least two
+  // rounds of pairs.  A 49 x 61 block (Laplace double layer, linear basis):
+  // regular launch 163 -> 11 us; 2028 triangles (single layer, linear): 172
+  // -> 72 us.  Finer tiles instead evaluate triangles at their edges several
+  // times (46 us for the block's launches at edge 16, 33 with the split;
+  // 2592 triangles 156 us at edge 32, 128 with the split) and cost the
+  // planner more than they gain.
+  a.split = 1;
+  a.entries = P->entries;
+  if (!P->persistent && !P->fused) {
+    const uint64_t run = a.nmir ? a.nmir : P->tiles.size();
+    const uint64_t pairs =
+        std::max<uint64_t>(1, (P->pairs[0] + P->pairs[1] + P->pairs[2] +
+                               P->pairs[3]) / P->tiles.size());
+    a.split = (uint32_t)std::max<uint64_t>(
+        1, std::min<uint64_t>({(1024 + run - 1) / run, pairs / 512, 64}));
+  }
   if (P->fused && !far && op->q == 2 && op->q2 == 4) {
     a.tiles = P->d_tiles_f.p;
     a.tlist = P->d_tpairs.p;
@@ -764,10 +775,10 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
                     : (small ? nf::launch_helmholtz_dlp_sp
                              : nf::launch_helmholtz_dlp);
   const int rc =
-      launch ? launch(op->rb, op->cb, op->q, a, ntiles, P->d_spairs.p, ncls,
+      launch ? launch(op->rb, op->cb, op->q, a, ntiles, P->d_spairs, ncls,
                       stream)
              : nf::launch_laplace(op->layer, op->rb, op->cb, op->q, a, ntiles,
-                                  P->d_spairs.p, ncls, stream);
+                                  P->d_spairs, ncls, stream);
   if (rc != H2HIP_OK) {
     set_error("unsupported regular quadrature order (1..4 supported)");
     return rc;
@@ -777,7 +788,7 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
     const uint32_t nfix = (uint32_t)P->fix.size();
     const int ntr = 0;  // each fix carries its block's ntrans
     hipLaunchKernelGGL(nf_fixup_kernel, dim3((nfix + 255) / 256), dim3(256),
-                       0, stream, P->d_fix.p, nfix, s->d_g.p, a.are, a.aim,
+                       0, stream, P->d_fix, nfix, s->d_g.p, a.are, a.aim,
                        op->kernel == H2HIP_HELMHOLTZ ? 1 : 0, ntr,
                        (double *)d_out);
     H2HIP_CHECK(hipGetLastError());
@@ -1373,8 +1384,14 @@ int h2hip_nfplan_set_schedule(h2hip_nfplan *p, int sorted, int persistent) {
     p->tiles = p->tiles0;
     p->spairs = p->spairs0;
   }
-  H2HIP_CHECK(p->d_tiles.upload(p->tiles.data(), p->tiles.size()));
-  H2HIP_CHECK(p->d_spairs.upload(p->spairs.data(), p->spairs.size()));
+  if (!p->tiles.empty())
+    H2HIP_CHECK(hipMemcpy(p->d_tiles, p->tiles.data(),
+                          sizeof(Tile) * p->tiles.size(),
+                          hipMemcpyHostToDevice));
+  if (!p->spairs.empty())
+    H2HIP_CHECK(hipMemcpy(p->d_spairs, p->spairs.data(),
+                          sizeof(SPair) * p->spairs.size(),
+                          hipMemcpyHostToDevice));
   p->sorted = sorted;
   return H2HIP_OK;
 }
@@ -1389,6 +1406,24 @@ int h2hip_nfplan_set_fused(h2hip_nfplan *p, int fused) {
     // (16 evaluations per regular pair, 1536 per identical or edge pair,
     // 512 per vertex pair)
     std::vector<Tile> tf = p->tiles;
+    // the pairs grouped by tile: identical, edge, vertex (spairs is ordered
+    // so by class)
+    for (const SPair &q : p->spairs) {
+      uint16_t &n = tf[q.tile].ns[3 - q.cls];
+      if (n == 0xffff) {
+        set_error("too many pairs with common vertices in one tile");
+        return H2HIP_EINVAL;
+      }
+      n++;
+    }
+    std::vector<uint32_t> at(tf.size());
+    uint32_t sum = 0;
+    for (size_t i = 0; i < tf.size(); i++) {
+      at[i] = tf[i].sbeg = sum;
+      sum += (uint32_t)tf[i].ns[0] + tf[i].ns[1] + tf[i].ns[2];
+    }
+    std::vector<SPair> tpairs(p->spairs.size());
+    for (const SPair &q : p->spairs) tpairs[at[q.tile]++] = q;
     auto work = [](const Tile &T) {
       return (uint64_t)T.nrsup * T.ncsup * 16 +
              ((uint64_t)T.ns[0] + T.ns[1]) * 1536 + (uint64_t)T.ns[2] * 512;
@@ -1397,7 +1432,7 @@ int h2hip_nfplan_set_fused(h2hip_nfplan *p, int fused) {
       return work(x) > work(y);
     });
     H2HIP_CHECK(p->d_tiles_f.upload(tf.data(), tf.size()));
-    H2HIP_CHECK(p->d_tpairs.upload(p->tpairs.data(), p->tpairs.size()));
+    H2HIP_CHECK(p->d_tpairs.upload(tpairs.data(), tpairs.size()));
   }
   p->fused = fused;
   return H2HIP_OK;

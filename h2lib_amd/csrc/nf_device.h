@@ -197,6 +197,23 @@ __device__ __forceinline__ double pair_factor(const KArgs &a, uint32_t rt,
   return a.kc * a.g[lo] * a.g[hi];
 }
 
+// a summed entry: stored, or added where a tile's pairs are split over
+// several workgroups
+__device__ __forceinline__ void put(const KArgs &a, size_t pos, double v,
+                                    uint32_t nslice) {
+  if (nslice > 1)
+    atomicAdd(&a.out[pos], v);
+  else
+    a.out[pos] = v;
+}
+
+static __global__ __launch_bounds__(NTHREADS) void zero_out(double *out,
+                                                            uint64_t n) {
+  for (uint64_t i = blockIdx.x * (uint64_t)NTHREADS + threadIdx.x; i < n;
+       i += gridDim.x * (uint64_t)NTHREADS)
+    out[i] = 0.0;
+}
+
 static __global__ void zero_counter(uint32_t *c) { *c = 0u; }
 
 __device__ __forceinline__ uint32_t loc_of(uint32_t packed, int l) {
@@ -461,14 +478,16 @@ __device__ __forceinline__ void tile_singular(const KArgs &a, const Tile &T,
                                               double *acc_re, double *acc_im);
 
 // One tile of the regular kernel, run by all NTHREADS threads of a
-// workgroup (MP: pair_sums).
+// workgroup (MP: pair_sums), or the slice-th of nslice parts of its pairs.
 // FUSED: the tile's workgroup also evaluates the tile's pairs with common
 // vertices (tlist + T.sbeg, T.ns[c] per class) before the tile is stored,
 // so they add into the LDS accumulator instead of the output (constant
 // basis: the regular pass leaves their entries to the singular pass).
 template <int KER, int BR, int BC, int Q, int MP, bool FUSED = false>
 __device__ __forceinline__ void regular_tile(const KArgs &a, uint32_t tile,
-                                             const SPair *tlist = nullptr) {
+                                             const SPair *tlist = nullptr,
+                                             uint32_t slice = 0,
+                                             uint32_t nslice = 1) {
   constexpr bool CPLX = KER >= K_HELM_SLP;
   constexpr bool CC = (BR == 0) && (BC == 0);
   constexpr int NR = BR ? 3 : 1;
@@ -493,10 +512,11 @@ __device__ __forceinline__ void regular_tile(const KArgs &a, uint32_t tile,
   }
 
   const uint32_t npairs = nR * nC;
-  // pair p = r + nR c, advanced by NTHREADS without a division per pair
-  const uint32_t dc = nR ? NTHREADS / nR : 0, dr = NTHREADS - dc * nR;
-  uint32_t rr = nR ? tid % nR : 0, cc = nR ? tid / nR : 0;
-  for (uint32_t p = tid; p < npairs; p += NTHREADS) {
+  // pair p = r + nR c, advanced without a division per pair
+  const uint32_t p0 = tid + NTHREADS * slice, step = NTHREADS * nslice;
+  const uint32_t dc = nR ? step / nR : 0, dr = step - dc * nR;
+  uint32_t rr = nR ? p0 % nR : 0, cc = nR ? p0 / nR : 0;
+  for (uint32_t p = p0; p < npairs; p += step) {
     const uint32_t r = rr, c = cc;
     rr += dr;
     cc += dc;
@@ -577,10 +597,10 @@ __device__ __forceinline__ void regular_tile(const KArgs &a, uint32_t tile,
                                 : (size_t)i + (size_t)j * T.ld);
       const int s = i + TILE * j;
       if constexpr (CPLX) {
-        a.out[2 * pos] = acc_re[s];
-        a.out[2 * pos + 1] = conj ? -acc_im[s] : acc_im[s];
+        put(a, 2 * pos, acc_re[s], nslice);
+        put(a, 2 * pos + 1, conj ? -acc_im[s] : acc_im[s], nslice);
       } else {
-        a.out[pos] = acc_re[s];
+        put(a, pos, acc_re[s], nslice);
       }
     }
   }
@@ -588,7 +608,8 @@ __device__ __forceinline__ void regular_tile(const KArgs &a, uint32_t tile,
 
 template <int KER, int BR, int BC, int Q, int MP>
 __global__ __launch_bounds__(NTHREADS) void nf_regular_kernel(KArgs a) {
-  regular_tile<KER, BR, BC, Q, MP>(a, blockIdx.x);
+  regular_tile<KER, BR, BC, Q, MP>(a, blockIdx.x / a.split, nullptr,
+                                   blockIdx.x % a.split, a.split);
 }
 
 // Two mirrored tiles per workgroup: tile T = (rows R, columns C) and its
@@ -634,7 +655,8 @@ __global__ __launch_bounds__(pair_threads(KER, B),
   double *const mir_im = mir_re + (CPLX ? TILE * TILE : 0);
 
   const int tid = threadIdx.x;
-  const uint32_t tile = list[blockIdx.x];
+  const uint32_t slice = blockIdx.x % a.split, nslice = a.split;
+  const uint32_t tile = list[blockIdx.x / nslice];
   const Tile T = a.tiles[tile];
   const bool diag = T.mirror == tile;
   const Tile M = a.tiles[T.mirror];
@@ -645,7 +667,7 @@ __global__ __launch_bounds__(pair_threads(KER, B),
   if constexpr (B) {
     for (int i = tid; i < NA * TILE * TILE; i += NTH) acc[i] = 0.0;
     __syncthreads();
-  } else if (diag) {
+  } else if (diag && slice == 0) {
     // identical triangles: completed by the singular kernel
     for (uint32_t r = tid; r < nR; r += NTH) {
       const size_t pos = T.out_off + r + (size_t)r * T.ld;
@@ -657,9 +679,10 @@ __global__ __launch_bounds__(pair_threads(KER, B),
   }
 
   const uint32_t npairs = diag ? nR * (nR - 1) / 2 : nR * nC;
-  const uint32_t dc = nR ? NTH / nR : 0, dr = NTH - dc * nR;
-  uint32_t rr = nR ? tid % nR : 0, cc = nR ? tid / nR : 0;
-  for (uint32_t p = tid; p < npairs; p += NTH) {
+  const uint32_t p0 = tid + NTH * slice, step = NTH * nslice;
+  const uint32_t dc = nR ? step / nR : 0, dr = step - dc * nR;
+  uint32_t rr = nR ? p0 % nR : 0, cc = nR ? p0 / nR : 0;
+  for (uint32_t p = p0; p < npairs; p += step) {
     const uint32_t r = rr;
     uint32_t c = cc;
     rr += dr;
@@ -752,10 +775,10 @@ __global__ __launch_bounds__(pair_threads(KER, B),
       const int s = i + TILE * j, t = j + TILE * i;
       const size_t pos = T.out_off + (size_t)i + (size_t)j * T.ld;
       if constexpr (CPLX) {
-        a.out[2 * pos] = acc_re[s] + (diag ? mir_re[t] : 0.0);
-        a.out[2 * pos + 1] = acc_im[s] + (diag ? mir_im[t] : 0.0);
+        put(a, 2 * pos, acc_re[s] + (diag ? mir_re[t] : 0.0), nslice);
+        put(a, 2 * pos + 1, acc_im[s] + (diag ? mir_im[t] : 0.0), nslice);
       } else {
-        a.out[pos] = acc_re[s] + (diag ? mir_re[t] : 0.0);
+        put(a, pos, acc_re[s] + (diag ? mir_re[t] : 0.0), nslice);
       }
     }
     if (!diag)
@@ -764,10 +787,10 @@ __global__ __launch_bounds__(pair_threads(KER, B),
         const int s = i + TILE * j;
         const size_t pos = M.out_off + (size_t)j + (size_t)i * M.ld;
         if constexpr (CPLX) {
-          a.out[2 * pos] = mir_re[s];
-          a.out[2 * pos + 1] = mir_im[s];
+          put(a, 2 * pos, mir_re[s], nslice);
+          put(a, 2 * pos + 1, mir_im[s], nslice);
         } else {
-          a.out[pos] = mir_re[s];
+          put(a, pos, mir_re[s], nslice);
         }
       }
   }
@@ -1571,17 +1594,26 @@ int launch_bases_p(uint32_t q, const KArgs &a, uint32_t ntiles,
   };
   const uint32_t n3 = ncls[CLS_IDENTICAL], n2 = ncls[CLS_EDGE],
                  n1 = ncls[CLS_VERTEX];
+  if ((BR || BC) && a.split > 1) {
+    const uint64_t n = a.entries * (KER >= K_HELM_SLP ? 2 : 1);
+    const uint64_t blocks = (n + NTHREADS - 1) / NTHREADS;
+    hipLaunchKernelGGL(zero_out, dim3((uint32_t)std::min<uint64_t>(blocks,
+                                                                   2048)),
+                       dim3(NTHREADS), 0, stream, a.out, n);
+  }
   if constexpr (BR == BC) {
     // mirrored tiles: half the regular, vertex and (linear basis) identical
     // pairs; the lists hold the pairs to evaluate first
     if (a.nmir && !a.far && q == 2 && a.q2 == 4) {
       if constexpr (paired(KER, BR, BC, MP))
-        hipLaunchKernelGGL((nf_pair_kernel<KER, BR, 2, MP>), dim3(a.nmir),
+        hipLaunchKernelGGL((nf_pair_kernel<KER, BR, 2, MP>),
+                           dim3(a.nmir * a.split),
                            dim3(pair_threads(KER, BR)), 0, stream, a,
                            a.mirlist);
       else
         hipLaunchKernelGGL((nf_regular_kernel<KER, BR, BC, 2, MP>),
-                           dim3(ntiles), dim3(NTHREADS), 0, stream, a);
+                           dim3(ntiles * a.split), dim3(NTHREADS), 0, stream,
+                           a);
       singular(nf_singular_kernel<KER, BR, BC, CLS_IDENTICAL, 4, SMP, BR != 0>,
                sp, BR ? a.nmain3 : n3);
       singular(nf_singular_kernel<KER, BR, BC, CLS_EDGE, 4, SMP, false>,
@@ -1621,7 +1653,8 @@ int launch_bases_p(uint32_t q, const KArgs &a, uint32_t ntiles,
       case 4: reg = nf_regular_kernel<KER, BR, BC, 4, MP>; break;
       default: return H2HIP_EINVAL;
     }
-    hipLaunchKernelGGL(reg, dim3(ntiles), dim3(NTHREADS), 0, stream, a);
+    hipLaunchKernelGGL(reg, dim3(ntiles * a.split), dim3(NTHREADS), 0, stream,
+                       a);
   }
   if (a.far) return H2HIP_OK;
   const bool q4 = a.q2 == 4;
