@@ -23,6 +23,7 @@
 #pragma once
 
 #include <algorithm>
+#include <type_traits>
 
 #include "dmath.h"
 #include "h2hip_internal.h"
@@ -32,6 +33,8 @@ namespace nf {
 
 constexpr int NTHREADS = 256;
 constexpr int NWAVES = NTHREADS / 64;
+// pairs with common vertices up to which their three classes share a launch
+constexpr uint32_t SING_ALL = 32768;
 
 // K_HELM_*_SP: the Helmholtz kernels for surfaces on which the phase varies
 // by less than pi/4 within a pair of triangles with common vertices and
@@ -1478,10 +1481,12 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
 // MIR: the list holds one of each two exchanged pairs; the other's entry is
 // added into the mirror tile.
 template <int KER, int BR, int BC, int CLS, int Q2, bool MP, bool MIR>
-__global__ __launch_bounds__(NTHREADS) void nf_singular_kernel(
-    KArgs a, const SPair *__restrict__ list, uint32_t npairs) {
+__device__ __forceinline__ void singular_list(const KArgs &a,
+                                              const SPair *__restrict__ list,
+                                              uint32_t npairs,
+                                              uint32_t block) {
   constexpr bool CPLX = KER >= K_HELM_SLP;
-  const uint32_t w = blockIdx.x * (NTHREADS / 16) + (threadIdx.x >> 4);
+  const uint32_t w = block * (NTHREADS / 16) + (threadIdx.x >> 4);
   const int sub = threadIdx.x & 15;
   if (w >= npairs) return;  // uniform per row of 16 lanes
   const SPair P = list[w];
@@ -1514,6 +1519,34 @@ __global__ __launch_bounds__(NTHREADS) void nf_singular_kernel(
           }
         }
       });
+}
+
+template <int KER, int BR, int BC, int CLS, int Q2, bool MP, bool MIR>
+__global__ __launch_bounds__(NTHREADS) void nf_singular_kernel(
+    KArgs a, const SPair *__restrict__ list, uint32_t npairs) {
+  singular_list<KER, BR, BC, CLS, Q2, MP, MIR>(a, list, npairs, blockIdx.x);
+}
+
+// The three classes (order 4) in one launch: identical pairs in the first
+// b3 workgroups, edge pairs in the next b2, vertex pairs in the rest.  For
+// lists that fit on the chip at once, where the launches one after the other
+// cost each class its own latency (a 49 x 61 block, linear basis: 24 -> 9.5
+// us, its launches 33 -> 20; 2048 triangles, constant basis: 25 -> 16 us;
+// 2028 triangles, linear, 30000 pairs: 40 -> 35 us); the registers are
+// those of the largest class, so long lists keep a launch per class.
+template <int KER, int BR, int BC, bool MP, bool MIR>
+__global__ __launch_bounds__(NTHREADS) void nf_singular_all(
+    KArgs a, const SPair *__restrict__ l3, uint32_t n3,
+    const SPair *__restrict__ l2, uint32_t n2, const SPair *__restrict__ l1,
+    uint32_t n1, uint32_t b3, uint32_t b2) {
+  const uint32_t b = blockIdx.x;
+  if (b < b3)
+    singular_list<KER, BR, BC, CLS_IDENTICAL, 4, MP, MIR && BR != 0>(a, l3, n3,
+                                                                    b);
+  else if (b < b3 + b2)
+    singular_list<KER, BR, BC, CLS_EDGE, 4, MP, false>(a, l2, n2, b - b3);
+  else
+    singular_list<KER, BR, BC, CLS_VERTEX, 4, MP, MIR>(a, l1, n1, b - b3 - b2);
 }
 
 // The pairs with common vertices of one tile and one rule class, by the
@@ -1594,6 +1627,27 @@ int launch_bases_p(uint32_t q, const KArgs &a, uint32_t ntiles,
   };
   const uint32_t n3 = ncls[CLS_IDENTICAL], n2 = ncls[CLS_EDGE],
                  n1 = ncls[CLS_VERTEX];
+  // order 4, all classes: one launch while every pair has its lanes at once
+  // (SING_ALL), else one per class
+  auto singular4 = [&](auto mir, uint32_t c3, uint32_t c1) {
+    constexpr bool MIR = decltype(mir)::value;
+    if (c3 + n2 + c1 <= SING_ALL) {
+      auto nb = [](uint32_t n) { return (n + PPB - 1) / PPB; };
+      if (c3 + n2 + c1)
+        hipLaunchKernelGGL((nf_singular_all<KER, BR, BC, SMP, MIR>),
+                           dim3(nb(c3) + nb(n2) + nb(c1)), dim3(NTHREADS), 0,
+                           stream, a, sp, c3, sp + n3, n2, sp + n3 + n2, c1,
+                           nb(c3), nb(n2));
+      return;
+    }
+    singular(nf_singular_kernel<KER, BR, BC, CLS_IDENTICAL, 4, SMP,
+                                MIR && BR != 0>,
+             sp, c3);
+    singular(nf_singular_kernel<KER, BR, BC, CLS_EDGE, 4, SMP, false>,
+             sp + n3, n2);
+    singular(nf_singular_kernel<KER, BR, BC, CLS_VERTEX, 4, SMP, MIR>,
+             sp + n3 + n2, c1);
+  };
   if ((BR || BC) && a.split > 1) {
     const uint64_t n = a.entries * (KER >= K_HELM_SLP ? 2 : 1);
     const uint64_t blocks = (n + NTHREADS - 1) / NTHREADS;
@@ -1614,12 +1668,7 @@ int launch_bases_p(uint32_t q, const KArgs &a, uint32_t ntiles,
         hipLaunchKernelGGL((nf_regular_kernel<KER, BR, BC, 2, MP>),
                            dim3(ntiles * a.split), dim3(NTHREADS), 0, stream,
                            a);
-      singular(nf_singular_kernel<KER, BR, BC, CLS_IDENTICAL, 4, SMP, BR != 0>,
-               sp, BR ? a.nmain3 : n3);
-      singular(nf_singular_kernel<KER, BR, BC, CLS_EDGE, 4, SMP, false>,
-               sp + n3, n2);
-      singular(nf_singular_kernel<KER, BR, BC, CLS_VERTEX, 4, SMP, true>,
-               sp + n3 + n2, a.nmain1);
+      singular4(std::true_type{}, BR ? a.nmain3 : n3, a.nmain1);
       return H2HIP_OK;
     }
   }
@@ -1657,15 +1706,15 @@ int launch_bases_p(uint32_t q, const KArgs &a, uint32_t ntiles,
                        a);
   }
   if (a.far) return H2HIP_OK;
-  const bool q4 = a.q2 == 4;
-  singular(q4 ? nf_singular_kernel<KER, BR, BC, CLS_IDENTICAL, 4, SMP, false>
-              : nf_singular_kernel<KER, BR, BC, CLS_IDENTICAL, 0, SMP, false>,
-           sp, n3);
-  singular(q4 ? nf_singular_kernel<KER, BR, BC, CLS_EDGE, 4, SMP, false>
-              : nf_singular_kernel<KER, BR, BC, CLS_EDGE, 0, SMP, false>,
-           sp + n3, n2);
-  singular(q4 ? nf_singular_kernel<KER, BR, BC, CLS_VERTEX, 4, SMP, false>
-              : nf_singular_kernel<KER, BR, BC, CLS_VERTEX, 0, SMP, false>,
+  if (a.q2 == 4) {
+    singular4(std::false_type{}, n3, n1);
+    return H2HIP_OK;
+  }
+  singular(nf_singular_kernel<KER, BR, BC, CLS_IDENTICAL, 0, SMP, false>, sp,
+           n3);
+  singular(nf_singular_kernel<KER, BR, BC, CLS_EDGE, 0, SMP, false>, sp + n3,
+           n2);
+  singular(nf_singular_kernel<KER, BR, BC, CLS_VERTEX, 0, SMP, false>,
            sp + n3 + n2, n1);
   return H2HIP_OK;
 }
