@@ -65,4 +65,37 @@ __device__ __forceinline__ void sincos_cw(double x, double &s, double &c) {
   c = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, c0) ^ cs);
 }
 
+// e^x: n the integer next to x / ln 2, r = x - n ln 2 with ln 2 in two parts
+// and fused products, |r| <= 0.3466, the Taylor polynomial of degree 13 (the
+// first term left out is 4.2e-18 at most) and a scaling by 2^n.  Relative
+// error below 0.63 * 2^-52 (4e6 arguments against long-double expl, the same
+// operations in C).  No branches, for the damping of the coupling values
+// (the library's exponential breaks up the evaluations of a lane).
+__device__ __forceinline__ double exp_cw(double x) {
+  constexpr double LOG2E = 1.4426950408889634;
+  constexpr double L1 = 0.6931471805599453, L2 = 2.3190468138462996e-17;
+  constexpr double MAGIC = 6755399441055744.0;
+  // beyond, the result is 0 or infinite
+  x = fmin(fmax(x, -1100.0), 1100.0);
+  const double m = fma(x, LOG2E, MAGIC);
+  const double n = m - MAGIC;
+  double r = fma(-n, L1, x);
+  r = fma(-n, L2, r);
+  double p = 1.0 / 6227020800.0;  // 1 / 13!
+  p = fma(p, r, 1.0 / 479001600.0);
+  p = fma(p, r, 1.0 / 39916800.0);
+  p = fma(p, r, 1.0 / 3628800.0);
+  p = fma(p, r, 1.0 / 362880.0);
+  p = fma(p, r, 1.0 / 40320.0);
+  p = fma(p, r, 1.0 / 5040.0);
+  p = fma(p, r, 1.0 / 720.0);
+  p = fma(p, r, 1.0 / 120.0);
+  p = fma(p, r, 1.0 / 24.0);
+  p = fma(p, r, 1.0 / 6.0);
+  p = fma(p, r, 0.5);
+  p = fma(p, r, 1.0);
+  p = fma(p, r, 1.0);
+  return __builtin_amdgcn_ldexp(p, (int)(uint32_t)__builtin_bit_cast(uint64_t, m));
+}
+
 }  // namespace h2hip

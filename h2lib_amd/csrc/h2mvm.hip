@@ -29,6 +29,7 @@
 #include <algorithm>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 
 #include "h2hip_internal.h"
 #include "dmath.h"
@@ -421,7 +422,7 @@ __device__ __forceinline__ void cpl_from_r2(double r2, int helmholtz,
     si = 0.0;
   } else {
     const double r = r2 * rs;
-    if (kdamp != 0.0) rs *= exp(kdamp * r);
+    if (kdamp != 0.0) rs *= h2hip::exp_cw(kdamp * r);
     double sn, cs;
     h2hip::sincos_cw(kr * r, sn, cs);
     sr = KCONST * (rs * cs);
@@ -448,13 +449,16 @@ struct CplSrc {
   double kr, kdamp;
 };
 
-// A mirrored pair of far blocks (r, c) / (c, r), r > c, for
-// couple_mf_pairs: the nodes and the four coefficient offsets, so that a
-// wave needs one load before its inputs
+// A mirrored pair of far blocks (r, c) / (c, r), r > c, for couple_mf_pairs
+// and couple_pairs64: the nodes and the four coefficient offsets, so that a
+// wave needs one load before its inputs, and the stored coupling of (r, c).
+// The adjoint product exchanges the sides, out_r with in_r and out_c with
+// in_c.
 struct PairD {
   uint32_t r, c;
   uint64_t out_r, in_c;  // block (r, c): yt of row node r, xt of column node c
   uint64_t out_c, in_r;  // mirror (c, r): yt of row node c, xt of column node r
+  uint64_t soff;
 };
 
 struct CNArgs {
@@ -675,6 +679,71 @@ __device__ __forceinline__ void mf_laplace4(const double *p3,
   }
 }
 
+// y|_c += alpha N^* x|_r for a near block of at most 64 x 64 by one wave:
+// lane l reads rows l % 16 + 16 k of columns l / 16 + 4 t (16 consecutive
+// entries of 4 columns per load) and sums its columns over its rows; the
+// sums over the 16 lanes of a column set are formed by a butterfly that
+// halves the columns a lane holds, 15 exchanges for the whole block.  Read
+// once, as the forward product reads it (couple_trans_wg, one workgroup per
+// block through LDS, did these and the far blocks before).
+template <int C>
+__device__ __forceinline__ void near_adjoint64(const CNArgs &a,
+                                               const NearD &b, int lane) {
+  const uint32_t la = lane & 15, lb = lane >> 4;
+  double xr[4], xi[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    xr[k] = xi[k] = 0.0;
+    const uint32_t i = la + 16 * k;
+    if (i < b.rows) ld<C>(a.v.x[0], a.ridx[b.roff + i], xr[k], xi[k]);
+  }
+  double cr[16], ci[C ? 16 : 1];
+#pragma unroll
+  for (int t0 = 0; t0 < 16; t0 += 4) {
+    double mr[4][4], mi[4][4];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const uint32_t i = la + 16 * k, j = lb + 4 * (t0 + t);
+        mr[t][k] = mi[t][k] = 0.0;
+        if (i < b.rows && j < b.cols)
+          ld<C>(a.N, b.noff + i + (uint64_t)j * b.rows, mr[t][k], mi[t][k]);
+      }
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      double sr = 0.0, si = 0.0;
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        // conj(N) x
+        sr = fma(mr[t][k], xr[k], sr);
+        if constexpr (C) {
+          sr = fma(mi[t][k], xi[k], sr);
+          si = fma(mr[t][k], xi[k], fma(-mi[t][k], xr[k], si));
+        }
+      }
+      cr[t0 + t] = sr;
+      if constexpr (C) ci[t0 + t] = si;
+    }
+  }
+  h2hip::bfly_step<8>(cr, lane);
+  h2hip::bfly_step<4>(cr, lane);
+  h2hip::bfly_step<2>(cr, lane);
+  h2hip::bfly_step<1>(cr, lane);
+  if constexpr (C) {
+    h2hip::bfly_step<8>(ci, lane);
+    h2hip::bfly_step<4>(ci, lane);
+    h2hip::bfly_step<2>(ci, lane);
+    h2hip::bfly_step<1>(ci, lane);
+  }
+  const uint32_t j = lb + 4 * la;
+  if (j >= b.cols) return;
+  const double sr = cr[0], si = C ? ci[0] : 0.0;
+  atomic_add<C>(a.v.y[0], a.cidx[b.coff + j],
+                a.v.are[0] * sr - a.v.aim[0] * si,
+                a.v.are[0] * si + a.v.aim[0] * sr);
+}
+
 // yt_r += S_rc xt_c and y|_r += alpha N_rc x|_c; TRANS: yt_c += S^* xt_r and
 // y|_c += alpha N^* x|_r.  One wave per block; the wave first gathers its
 // block's input entries into its own LDS slice.
@@ -805,6 +874,12 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
   const uint32_t nb = w - a.nfar;
   if (nb >= a.nnear) return;
   const NearD b = a.near[nb];
+  if constexpr (TRANS && NV == 1 && !ORD && !MF) {
+    if (b.rows <= 64 && b.cols <= 64) {
+      near_adjoint64<C>(a, b, lane);
+      return;
+    }
+  }
   const uint32_t nout = TRANS ? b.cols : b.rows, nin = TRANS ? b.rows : b.cols;
   const uint32_t *oidx = TRANS ? a.cidx + b.coff : a.ridx + b.roff;
   const uint32_t *iidx = TRANS ? a.ridx + b.roff : a.cidx + b.coff;
@@ -1029,15 +1104,15 @@ __global__ __launch_bounds__(NT) void couple_trans_wg(CNArgs a) {
   }
 }
 
-// Couplings computed in the product at interpolation order M = 4 or 5, one
-// vector, for a symmetric block structure (row and column trees with the
+// Couplings computed in the product at interpolation order M = 5 (order 4:
+// couple_pairs64), one vector, for a symmetric block structure (row and column trees with the
 // same points, every admissible block (r, c) with its mirror (c, r), whose
 // coupling matrix is S_rc^T: the squared distances, and so the values of
 // 1/r or e^{ikr}/r, are the same bit for bit).  One wave per pair r > c
 // evaluates each value once for both blocks: lane l keeps the sums of row
 // points l and l + 64 (rank M^3 <= 128) of block (r, c), yt_r[i] += sum_j
 // S_ij xt_c[j], with the arithmetic and order of the per-block kernel
-// (mf_laplace4, the general loop otherwise), and the products S_ij xt_r[i]
+// (the general loop), and the products S_ij xt_r[i]
 // of W columns at a time, whose sums over the rows, yt_c[j] += sum_i S_ij
 // xt_r[i] for the mirror block, a butterfly over the lanes forms.  Half the
 // evaluations of the two blocks' waves.  C: Helmholtz (complex).
@@ -1149,6 +1224,203 @@ __global__ __launch_bounds__(NT) void couple_mf_pairs(CNArgs a,
       }
     }
   }
+}
+
+// Sum of CW (8 or 4) values over the lanes that share lane & 7: lane l
+// returns value (l >> 3) & (CW - 1).  v is clobbered.
+template <int CW>
+__device__ __forceinline__ double column_sum(double (&v)[CW], int lane) {
+  auto step = [&](int s, int bit) {
+    const bool up = (lane & bit) != 0;
+#pragma unroll
+    for (int t = 0; t < CW / 2; t++)
+      if (t < s) {
+        const double send = up ? v[t] : v[t + s];
+        const double keep = up ? v[t + s] : v[t];
+        v[t] = keep + __shfl_xor(send, bit, 64);
+      }
+  };
+  if constexpr (CW == 8) step(4, 32);
+  step(2, 16);
+  step(1, 8);
+  if constexpr (CW == 4) v[0] += __shfl_xor(v[0], 32, 64);
+  return v[0];
+}
+
+// Mirrored pairs of couplings of rank 64 (order 4), one vector, forward
+// (ADJ: adjoint) product: one wave per pair r > c forms yt_r += S xt_c and
+// yt_c += S^T xt_r (the mirror block's coupling is S_rc^T bit for bit; ADJ:
+// the conjugates, which for the adjoint product of the pair are the same
+// two products with the sides' coefficients exchanged) from each value of
+// S once, read (MF = false) or computed.
+//
+// The wave is an 8 x 8 grid of lanes and the block an 8 x 8 grid of 8 x 8
+// sub-blocks, one per lane: a lane sums its 8 rows over its 8 columns and
+// its 8 columns over its 8 rows in registers, and the sums over the lanes
+// of a row or a column are formed once at the end by butterflies that halve
+// the values a lane holds, 7 exchanges each way, after which lane l has one
+// row and one column of the block.  With one row per lane instead
+// (couple_mf_pairs) every column needs its sum over all 64 lanes: 68
+// exchanges, and as many selects, in the real case, 224 in the complex one.
+// Computed: the 8 points of a lane share x, take two y and four z, so the
+// squared distances of its 64 values need one product each.  Read: the
+// lanes of a column read 128 consecutive bytes per load, streaming (no
+// reuse).  DAMP: complex wave number (without it no exponential, whose
+// branch breaks up the evaluations).  Bound: computed complex values by FP64
+// VALU issue (sine and cosine), read ones by HBM.  Computed couplings,
+// Helmholtz 131072 triangles 527 -> 318 us (couple_mf_pairs at order 4
+// before), Laplace 2048 triangles 7.6 -> 4.4 us; read ones, 32768
+// triangles, 48 -> 34 us (one wave per block before); adjoint with the near
+// blocks, 31212 triangles, 159 -> 34 + 18 us (couple_trans_wg before).
+typedef double dbl2 __attribute__((ext_vector_type(2)));
+
+template <int C, bool MF, bool ADJ, bool DAMP>
+__global__ __launch_bounds__(NT) void couple_pairs64(
+    CNArgs a, const PairD *__restrict__ pairs, uint32_t npair) {
+  constexpr double KCONST = 0.0795774715459476679;
+  // columns per pass: complex computed values leave registers for 4
+  constexpr int CW = C ? 4 : 8, NPASS = 8 / CW;
+  const uint32_t w = __builtin_amdgcn_readfirstlane(
+      blockIdx.x * WPB + (threadIdx.x >> 6));
+  if (w >= npair) return;  // uniform over the wave; no block barrier
+  const int lane = threadIdx.x & 63, la = lane >> 3, lb = lane & 7;
+  const PairD b = pairs[w];
+  const uint64_t out_r = ADJ ? b.in_r : b.out_r, in_r = ADJ ? b.out_r : b.in_r;
+  const uint64_t out_c = ADJ ? b.in_c : b.out_c, in_c = ADJ ? b.out_c : b.in_c;
+  // the lane's rows: eight in sequence when computed (they share points);
+  // read: pairs (real) or single entries (complex) 16 or 8 rows apart
+  auto row = [&](int u) {
+    return MF ? 8 * la + u
+              : C ? la + 8 * u : 2 * la + (u & 1) + 16 * (u >> 1);
+  };
+  double xrr[8], xri[8], ar[8], ai[8];
+#pragma unroll
+  for (int u = 0; u < 8; u++) {
+    xri[u] = 0.0;
+    ld<C>(a.xt, in_r + row(u), xrr[u], xri[u]);
+    if constexpr (MF) {
+      xrr[u] *= KCONST;
+      xri[u] *= KCONST;
+    }
+    ar[u] = ai[u] = 0.0;
+  }
+  double px = 0.0, py[2], pz[4], qx = 0.0;
+  const double *pr = nullptr, *pc = nullptr;
+  if constexpr (MF) {
+    pr = a.cs.rpts + 12 * (uint64_t)b.r;
+    pc = a.cs.cpts + 12 * (uint64_t)b.c;
+    px = pr[la >> 1];
+    qx = pc[lb >> 1];
+#pragma unroll
+    for (int u = 0; u < 2; u++) py[u] = pr[4 + 2 * (la & 1) + u];
+#pragma unroll
+    for (int u = 0; u < 4; u++) pz[u] = pr[8 + u];
+  }
+  double colr = 0.0, coli = 0.0;  // the lane's column of the block
+#pragma unroll 1
+  for (int q = 0; q < NPASS; q++) {
+    double xcr[CW], xci[CW], cr[CW], ci[CW];
+#pragma unroll
+    for (int v = 0; v < CW; v++) {
+      xci[v] = 0.0;
+      ld<C>(a.xt, in_c + 8 * lb + CW * q + v, xcr[v], xci[v]);
+      if constexpr (MF) {
+        xcr[v] *= KCONST;
+        xci[v] *= KCONST;
+      }
+      cr[v] = ci[v] = 0.0;
+    }
+    auto add = [&](int u, int v, double sr, double si) {
+      if constexpr (ADJ) si = -si;
+      ar[u] = fma(sr, xcr[v], ar[u]);
+      cr[v] = fma(sr, xrr[u], cr[v]);
+      if constexpr (C) {
+        ar[u] = fma(-si, xci[v], ar[u]);
+        ai[u] = fma(sr, xci[v], fma(si, xcr[v], ai[u]));
+        cr[v] = fma(-si, xri[u], cr[v]);
+        ci[v] = fma(sr, xri[u], fma(si, xrr[u], ci[v]));
+      }
+    };
+    if constexpr (MF) {
+      const double d0 = px - qx;
+#pragma unroll
+      for (int vy = 0; vy < CW / 4; vy++) {
+        const double qy = pc[4 + 2 * (lb & 1) + (CW == 4 ? q : vy)];
+        double dxy[2];
+#pragma unroll
+        for (int uy = 0; uy < 2; uy++) {
+          const double d1 = py[uy] - qy;
+          dxy[uy] = fma(d1, d1, d0 * d0);
+        }
+#pragma unroll
+        for (int vz = 0; vz < 4; vz++) {
+          const double qz = pc[8 + vz];
+#pragma unroll
+          for (int u = 0; u < 8; u++) {
+            const double d2 = pz[u & 3] - qz;
+            const double r2 = fma(d2, d2, dxy[u >> 2]);
+            // (the kernel constant is in the inputs)
+            const double rs = cpl_rsqrt(r2);
+            if constexpr (C) {
+              const double r = r2 * rs;
+              double amp = rs;
+              if constexpr (DAMP) amp *= h2hip::exp_cw(a.cs.kdamp * r);
+              double sn, cs;
+              h2hip::sincos_cw(a.cs.kr * r, sn, cs);
+              add(u, 4 * vy + vz, amp * cs, amp * sn);
+            } else {
+              add(u, 4 * vy + vz, rs, 0.0);
+            }
+          }
+        }
+      }
+    } else {
+      const dbl2 *S = (const dbl2 *)(a.S + (C ? 2 : 1) * b.soff);
+#pragma unroll
+      for (int v0 = 0; v0 < CW; v0 += 4) {
+        constexpr int L = C ? 8 : 4;  // loads per column
+        dbl2 m[4][L];
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+#pragma unroll
+          for (int u = 0; u < L; u++) {
+            const uint32_t j = 8 * lb + CW * q + v0 + v;
+            m[v][u] = __builtin_nontemporal_load(
+                S + (C ? 64 * j + la + 8 * u : 32 * j + la + 8 * u));
+          }
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+#pragma unroll
+          for (int u = 0; u < L; u++) {
+            if constexpr (C) {
+              add(u, v0 + v, m[v][u].x, m[v][u].y);
+            } else {
+              add(2 * u, v0 + v, m[v][u].x, 0.0);
+              add(2 * u + 1, v0 + v, m[v][u].y, 0.0);
+            }
+          }
+      }
+    }
+    // sums of the pass's columns over the lanes la: lane bits 3 to 5 pick
+    // the column (CW = 4: bits 3 and 4, and bit 5 the pass)
+    const double sr = column_sum<CW>(cr, lane);
+    const double si = C ? column_sum<CW>(ci, lane) : 0.0;
+    if (NPASS == 1 || (lane >> 5) == q) {
+      colr = sr;
+      coli = si;
+    }
+  }
+  // sums of the rows over the lanes lb: lane bits 0 to 2 pick the row
+  h2hip::bfly_step<4>(ar, lane);
+  h2hip::bfly_step<2>(ar, lane);
+  h2hip::bfly_step<1>(ar, lane);
+  if constexpr (C) {
+    h2hip::bfly_step<4>(ai, lane);
+    h2hip::bfly_step<2>(ai, lane);
+    h2hip::bfly_step<1>(ai, lane);
+  }
+  atomic_add<C>(a.yt, out_r + row(lb), ar[0], ai[0]);
+  atomic_add<C>(a.yt, out_c + 8 * lb + la, colr, coli);
 }
 
 // Self-adjoint product from the lower block triangle (row and column
@@ -2266,11 +2538,15 @@ void launch(const VecSet &vs, const h2hip_h2matrix *H, double *xt, double *yt,
   const bool twg = trans && !symm && !tv && H->maxrank <= 64 &&
                    H->maxleaf <= 64;
   // flat, not symmetric: the near blocks run in the upward launch (not for
-  // the workgroup adjoint blocks)
-  const bool fuse = flat && !symm && !twg && H->nnear > 0 &&
-                    !in.items.empty();
+  // the workgroup adjoint blocks of several vectors or fixed-order sums)
+  const bool fuse = flat && !symm && (!twg || (NV == 1 && !ord)) &&
+                    H->nnear > 0 && !in.items.empty();
   const int cm = C ? 2 : 1;
   const bool mf = H->cpl_recompute && !symm;
+  // one vector, order-4 interpolation couplings (read or computed) in
+  // mirrored pairs: each value once for a block and its mirror
+  const bool pairs64 = NV == 1 && !symm && !ord && !tv && H->pairs_on &&
+                       H->npair && H->cpl_known && H->cpl.m == 4;
   // view: the transposed blocks, whose rows are the column side's
   auto coupling_args = [&](bool view = false) {
     CNArgs c;
@@ -2399,6 +2675,25 @@ void launch(const VecSet &vs, const h2hip_h2matrix *H, double *xt, double *yt,
                          cnr);
     c.nnear = 0;
   }
+  if constexpr (NV == 1) {
+    if (pairs64) {
+      const dim3 gp((H->npair + WPB - 1) / WPB);
+      const PairD *pl = H->d_pairs.p;
+      const bool damp = C && mf && H->cpl.kdamp != 0.0;
+      auto go = [&](auto adj) {
+        constexpr bool ADJ = decltype(adj)::value;
+        auto k = !mf ? couple_pairs64<C, false, ADJ, false>
+                 : C && damp ? couple_pairs64<C, true, ADJ, C != 0>
+                             : couple_pairs64<C, true, ADJ, false>;
+        hipLaunchKernelGGL(k, gp, dim3(NT), 0, st, c, pl, H->npair);
+      };
+      if (trans)
+        go(std::true_type{});
+      else
+        go(std::false_type{});
+      c.nfar = 0;  // the near blocks (if any are left) as below
+    }
+  }
   if (twg) {
     // stored couplings and near blocks: one workgroup each; computed
     // couplings: the wave path for the far blocks, workgroups for the near
@@ -2447,16 +2742,14 @@ void launch(const VecSet &vs, const h2hip_h2matrix *H, double *xt, double *yt,
         hipLaunchKernelGGL((couple_near<C, true, NV>), gc, dim3(NT), 0, st,
                            c);
     } else if (mf) {
-      // symmetric structure, order-4 or -5 couplings, one vector, far
-      // blocks only: each value once for a block and its mirror
+      // symmetric structure, order-5 couplings, one vector, far blocks
+      // only: each value once for a block and its mirror
       bool paired = false;
       if constexpr (NV == 1)
-        paired = H->pairs_on && H->npair && c.nnear == 0 && !ord;
+        paired = H->pairs_on && H->npair && H->cpl.m == 5 && c.nfar > 0 &&
+                 c.nnear == 0 && !ord;
       const dim3 gp((H->npair + WPB - 1) / WPB);
-      if (paired && H->cpl.m == 4)
-        hipLaunchKernelGGL((couple_mf_pairs<C, 4>), gp, dim3(NT), 0, st, c,
-                           (const PairD *)H->d_pairs.p, H->npair);
-      else if (paired)
+      if (paired)
         hipLaunchKernelGGL((couple_mf_pairs<C, 5>), gp, dim3(NT), 0, st, c,
                            (const PairD *)H->d_pairs.p, H->npair);
       else if (ord)
@@ -3328,7 +3621,7 @@ int h2hip_h2matrix_interp_couplings(h2hip_h2matrix *H, int kernel,
       symmetric = b.r != b.c && it != key.end() && it->first == mirror;
       if (b.r > b.c)
         pairs.push_back(PairD{b.r, b.c, rnodes[b.r].coef, cnodes[b.c].coef,
-                              rnodes[b.c].coef, cnodes[b.r].coef});
+                              rnodes[b.c].coef, cnodes[b.r].coef, b.soff});
     }
     if (symmetric && !pairs.empty()) {
       H2HIP_CHECK(H->d_pairs.upload(pairs.data(), pairs.size()));

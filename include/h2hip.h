@@ -260,14 +260,15 @@ int h2hip_h2matrix_set_adjoint_storage(h2hip_h2matrix *H, int keep);
  * v_mfma_f64_16x16x4_f64 per coupling block.  Other products, computed
  * couplings and reproducible mode keep the vector kernels. */
 int h2hip_h2matrix_set_mfma(h2hip_h2matrix *H, int on);
-/* Couplings computed in the product (coupling mode 1) of an order-4 or -5
- * interpolation matrix (Laplace or Helmholtz) whose row and column boxes
- * have the same points and whose admissible blocks come in mirrored pairs
- * (r, c) / (c, r), as for the operators of one mesh: the one-vector
- * forward product evaluates each coupling value once for both blocks of a
- * pair (on = 1, the default; no counterpart in the reference).
- * Reproducible mode, adjoint and batched products keep one evaluation per
- * block. */
+/* Couplings of an order-4 or -5 interpolation matrix (Laplace or Helmholtz)
+ * whose row and column boxes have the same points and whose admissible
+ * blocks come in mirrored pairs (r, c) / (c, r), as for the operators of one
+ * mesh: the one-vector products evaluate each coupling value once for both
+ * blocks of a pair (on = 1, the default; no counterpart in the reference):
+ * order 4, read (h2hip_h2matrix_interp_couplings) or computed in the
+ * product (coupling mode 1), forward and adjoint; order 5, computed,
+ * forward.  Reproducible mode, batched products and the adjoint from kept
+ * transposes keep one evaluation per block. */
 int h2hip_h2matrix_set_coupling_pairs(h2hip_h2matrix *H, int on);
 /* The number of mirrored pairs found by h2hip_h2matrix_interp_couplings
  * (0: the structure is not symmetric, or not order 4 or 5; -1: H null). */
@@ -351,8 +352,9 @@ int h2hip_addeval_amatrix(const double *alpha, int is_complex, int trans,
                           uint32_t rows, uint32_t cols, const void *A,
                           uint64_t ld, const void *x, void *y, void *stream);
 
-/* Bytes one product y += alpha H x reads in the current schedule and
- * coupling mode: near field, couplings (0 when computed), bases (the
+/* Bytes of one product y += alpha H x in the current schedule and coupling
+ * mode (the couplings of both blocks of a mirrored pair, though one is
+ * read): near field, couplings (0 when computed), bases (the
  * blocks W_a|_l of both sides with the flat transforms, else leaf and
  * transfer matrices). */
 int h2hip_h2matrix_bytes(const h2hip_h2matrix *H, uint64_t *out3);

@@ -1,0 +1,65 @@
+"""Mirrored coupling pairs and the one-wave adjoint near blocks of the H2
+product (needs a GPU).
+
+The default products evaluate each coupling value of an order-4 matrix once
+for a block and its mirror, read or computed, forward and adjoint, and the
+adjoint reads each near block once.  The reproducible products use neither
+and are the reference here: the same values summed in another order, a few
+thousand terms, 1e-13 of the largest entry.  With the pairs switched off the
+general kernels run.  Leaves of 100 DOFs make blocks larger than the wave's
+64 x 64, leaves of 3 small ones.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("clf", [64, 100, 3])
+@pytest.mark.parametrize("kern,layer,basis,k", [
+    (0, 0, 1, 0.0), (0, 1, 1, 0.0), (0, 2, 0, 0.0), (1, 0, 0, 3.0),
+    (1, 1, 0, 2.0 + 0.5j), (1, 2, 1, 2.0)])
+def test_pairs_and_adjoint_match_general_kernels(kern, layer, basis, k, clf):
+    import h2lib_amd as h
+    from h2lib_amd import geometry as G
+    from h2lib_amd.h2matrix import H2Matrix
+    if clf == 3 and (kern, layer) not in ((0, 1), (1, 1)):
+        pytest.skip("small leaves: one real and one complex case")
+    mesh = G.sphere({3: 6, 64: 14, 100: 26}[clf])
+    gr = h.Surface3d(mesh.x, mesh.t, mesh.n, mesh.g)
+    op = h.Bem3d(gr, kern, layer, 2, 4, basis, basis,
+                 alpha=0.5 if layer else 0.0, k=k)
+    rt = G.ClusterTree(mesh, basis, clf)
+    bt = G.BlockTree(rt, rt, 2.0, 0)
+    H = H2Matrix(op, mesh, rt, rt, bt, 4)
+    H.set_schedule(2)
+    assert H.coupling_pairs() > 0
+    rng = np.random.default_rng(2)
+    x = rng.standard_normal(H.n)
+    if kern:
+        x = x + 1j * rng.standard_normal(H.n)
+    d_x = h.DeviceArray.from_host(x.astype(H.dtype))
+    d_y = h.DeviceArray(H.n, H.dtype)
+    alpha = 0.75 - 0.5j if kern else 0.75
+
+    def product(trans):
+        d_y.zero()
+        H.addeval(alpha, d_x, d_y, trans=trans)
+        return d_y.download()
+
+    try:
+        for mode in (0, 1):
+            H.set_coupling_mode(mode)
+            for trans in (False, True):
+                h.set_reproducible(True)
+                want = product(trans)
+                h.set_reproducible(False)
+                for pairs in (1, 0):
+                    H.set_coupling_pairs(pairs)
+                    for _ in range(2):  # coefficients cleared in between
+                        got = product(trans)
+                        err = np.abs(got - want).max() / np.abs(want).max()
+                        assert err < 1e-13, (mode, trans, pairs, err)
+                H.set_coupling_pairs(1)
+    finally:
+        h.set_reproducible(True)
