@@ -1275,13 +1275,14 @@ __device__ __forceinline__ double column_sum(double (&v)[CW], int lane) {
 typedef double dbl2 __attribute__((ext_vector_type(2)));
 
 template <int C, bool MF, bool ADJ, bool DAMP>
-__global__ __launch_bounds__(NT) void couple_pairs64(
-    CNArgs a, const PairD *__restrict__ pairs, uint32_t npair) {
+__device__ __forceinline__ void couple_pairs64_dev(
+    const CNArgs &a, const PairD *__restrict__ pairs, uint32_t npair,
+    uint32_t block) {
   constexpr double KCONST = 0.0795774715459476679;
   // columns per pass: complex computed values leave registers for 4
   constexpr int CW = C ? 4 : 8, NPASS = 8 / CW;
-  const uint32_t w = __builtin_amdgcn_readfirstlane(
-      blockIdx.x * WPB + (threadIdx.x >> 6));
+  const uint32_t w =
+      __builtin_amdgcn_readfirstlane(block * WPB + (threadIdx.x >> 6));
   if (w >= npair) return;  // uniform over the wave; no block barrier
   const int lane = threadIdx.x & 63, la = lane >> 3, lb = lane & 7;
   const PairD b = pairs[w];
@@ -1421,6 +1422,37 @@ __global__ __launch_bounds__(NT) void couple_pairs64(
   }
   atomic_add<C>(a.yt, out_r + row(lb), ar[0], ai[0]);
   atomic_add<C>(a.yt, out_c + 8 * lb + la, colr, coli);
+}
+
+// (complex computed values: three waves per SIMD, 168 registers instead of
+// the 170 to 174 the compiler would take, which allow two)
+template <int C, bool MF, bool ADJ, bool DAMP>
+__global__ __launch_bounds__(NT, C && MF ? 3 : 1) void couple_pairs64(
+    CNArgs a, const PairD *__restrict__ pairs, uint32_t npair) {
+  couple_pairs64_dev<C, MF, ADJ, DAMP>(a, pairs, npair, blockIdx.x);
+}
+
+// The computed complex couplings and the near blocks (a.nfar = 0) of a
+// forward product in one launch, their workgroups interleaved: the couplings
+// are bound by VALU issue and the near blocks by memory.  pb workgroups of
+// pairs, nb of near blocks.  Not for real couplings, which are short enough
+// that the upward launch hides more of the near blocks (2048 triangles 18.7
+// -> 19.8 us, 32768 triangles the same).
+template <bool DAMP>
+__global__ __launch_bounds__(NT, 3) void couple_pairs64_near(
+    CNArgs a, const PairD *__restrict__ pairs, uint32_t npair, uint32_t pb,
+    uint32_t nb) {
+  __shared__ double xs_all[WPB * 2 * MAXRANK];
+  // near blocks before workgroup b: floor(b nb / (pb + nb))
+  const uint32_t b = blockIdx.x;
+  const uint32_t n0 = (uint32_t)((uint64_t)b * nb / (pb + nb));
+  const uint32_t n1 = (uint32_t)((uint64_t)(b + 1) * nb / (pb + nb));
+  if (n1 == n0)  // uniform over the block
+    couple_pairs64_dev<1, true, false, DAMP>(a, pairs, npair, b - n0);
+  else
+    couple_near_dev<1, false, 1, false, false, true>(
+        a, n0 * WPB + (threadIdx.x >> 6),
+        xs_all + (threadIdx.x >> 6) * 2 * MAXRANK);
 }
 
 // Self-adjoint product from the lower block triangle (row and column
@@ -2537,16 +2569,23 @@ void launch(const VecSet &vs, const h2hip_h2matrix *H, double *xt, double *yt,
   // (couple_trans_wg)
   const bool twg = trans && !symm && !tv && H->maxrank <= 64 &&
                    H->maxleaf <= 64;
-  // flat, not symmetric: the near blocks run in the upward launch (not for
-  // the workgroup adjoint blocks of several vectors or fixed-order sums)
-  const bool fuse = flat && !symm && (!twg || (NV == 1 && !ord)) &&
-                    H->nnear > 0 && !in.items.empty();
   const int cm = C ? 2 : 1;
   const bool mf = H->cpl_recompute && !symm;
   // one vector, order-4 interpolation couplings (read or computed) in
   // mirrored pairs: each value once for a block and its mirror
   const bool pairs64 = NV == 1 && !symm && !ord && !tv && H->pairs_on &&
                        H->npair && H->cpl_known && H->cpl.m == 4;
+  // the near blocks of a flat, not symmetric product run with the computed
+  // complex pairs or in the upward launch (not the workgroup adjoint blocks
+  // of several vectors or fixed-order sums).  With the pairs where these are
+  // at least eight rounds of the 768 resident workgroups: 131072 triangles
+  // 758 -> 657 us; at 32768 (two and a half rounds) the last round's pairs
+  // run alone, 190 -> 204 us.
+  const bool pairs_near = C && pairs64 && mf && flat && !trans &&
+                          H->nnear > 0 && H->npair >= 8 * 768 * WPB;
+  const bool fuse = flat && !symm && !pairs_near &&
+                    (!twg || (NV == 1 && !ord)) && H->nnear > 0 &&
+                    !in.items.empty();
   // view: the transposed blocks, whose rows are the column side's
   auto coupling_args = [&](bool view = false) {
     CNArgs c;
@@ -2687,10 +2726,20 @@ void launch(const VecSet &vs, const h2hip_h2matrix *H, double *xt, double *yt,
                              : couple_pairs64<C, true, ADJ, false>;
         hipLaunchKernelGGL(k, gp, dim3(NT), 0, st, c, pl, H->npair);
       };
-      if (trans)
+      if (pairs_near) {
+        CNArgs cn = c;
+        cn.nfar = 0;
+        const uint32_t nb = (c.nnear + WPB - 1) / WPB;
+        hipLaunchKernelGGL(damp ? couple_pairs64_near<true>
+                                : couple_pairs64_near<false>,
+                           dim3(gp.x + nb), dim3(NT), 0, st, cn, pl, H->npair,
+                           gp.x, nb);
+        c.nnear = 0;
+      } else if (trans) {
         go(std::true_type{});
-      else
+      } else {
         go(std::false_type{});
+      }
       c.nfar = 0;  // the near blocks (if any are left) as below
     }
   }
