@@ -31,6 +31,25 @@ __device__ __forceinline__ void sincos_poly(double r, double &s, double &c) {
   c = fma(r2, pc, 1.0);
 }
 
+// sin and cos of |r| <= 0.255, as sincos_poly with S and C of degree 3 (they
+// miss sin and cos by 1.0e-17 and 1.4e-19 before the coefficients are
+// rounded).
+__device__ __forceinline__ void sincos_poly_tiny(double r, double &s,
+                                                 double &c) {
+  const double r2 = r * r;
+  double ps = 2.751519574989631e-06;
+  ps = fma(ps, r2, -0.0001984124490180426);
+  ps = fma(ps, r2, 0.008333333327309867);
+  ps = fma(ps, r2, -0.16666666666661845);
+  s = fma(r * r2, ps, r);
+  double pc = -2.752053385775909e-07;
+  pc = fma(pc, r2, 2.4801564162277738e-05);
+  pc = fma(pc, r2, -0.001388888888282356);
+  pc = fma(pc, r2, 0.0416666666666612);
+  pc = fma(pc, r2, -0.5);
+  c = fma(r2, pc, 1.0);
+}
+
 // sin and cos of x: Cody and Waite's reduction by pi/2 in three parts
 // (n the integer next to 2x / pi, r = x - n pi/2 with fused products) to |r| <= pi/4,
 // then sincos_poly (Taylor polynomials of degree 17 and 16, which the code

@@ -189,6 +189,12 @@ int launch_helmholtz_slp_sp(int rb, int cb, uint32_t q, const KArgs &a,
 int launch_helmholtz_dlp_sp(int rb, int cb, uint32_t q, const KArgs &a,
                             uint32_t ntiles, const SPair *sp,
                             const uint32_t *ncls, hipStream_t stream);
+int launch_helmholtz_slp_tp(int rb, int cb, uint32_t q, const KArgs &a,
+                            uint32_t ntiles, const SPair *sp,
+                            const uint32_t *ncls, hipStream_t stream);
+int launch_helmholtz_dlp_tp(int rb, int cb, uint32_t q, const KArgs &a,
+                            uint32_t ntiles, const SPair *sp,
+                            const uint32_t *ncls, hipStream_t stream);
 
 }  // namespace nf
 }  // namespace h2hip

@@ -764,16 +764,21 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
   uint32_t ncls[4];
   for (int c = 0; c < 4; c++) ncls[c] = (uint32_t)P->pairs[c];
   // FP64 Helmholtz kernels without argument reduction: real k, and the phase
-  // varies by at most pi/4 over two edges (|r - r0| <= 2 h within a pair of
-  // triangles, r <= 2 h in a pair with common vertices)
-  const bool small = a.mp == 0 && a.ki == 0.0 &&
-                     std::fabs(a.kr) * 2.0 * s->hmax <= 0.25 * M_PI;
+  // varies by at most pi/4 (1/4: shorter polynomials still) over two edges
+  // (|r - r0| <= 2 h within a pair of triangles, r <= 2 h in a pair with
+  // common vertices)
+  const double phase = std::fabs(a.kr) * 2.0 * s->hmax;
+  const bool real64 = a.mp == 0 && a.ki == 0.0;
+  const bool tiny = real64 && phase <= 0.25;
+  const bool small = real64 && phase <= 0.25 * M_PI;
   auto launch = op->kernel != H2HIP_HELMHOLTZ ? nullptr
                 : op->layer == H2HIP_SLP
-                    ? (small ? nf::launch_helmholtz_slp_sp
-                             : nf::launch_helmholtz_slp)
-                    : (small ? nf::launch_helmholtz_dlp_sp
-                             : nf::launch_helmholtz_dlp);
+                    ? (tiny    ? nf::launch_helmholtz_slp_tp
+                       : small ? nf::launch_helmholtz_slp_sp
+                               : nf::launch_helmholtz_slp)
+                    : (tiny    ? nf::launch_helmholtz_dlp_tp
+                       : small ? nf::launch_helmholtz_dlp_sp
+                               : nf::launch_helmholtz_dlp);
   const int rc =
       launch ? launch(op->rb, op->cb, op->q, a, ntiles, P->d_spairs, ncls,
                       stream)

@@ -41,18 +41,20 @@ constexpr uint32_t SING_ALL = 32768;
 // around a reference distance within any other pair (real k, 2 |k| h <= pi/4
 // with the longest edge h): no argument reduction per evaluation, and no
 // damping, whose exponential breaks up the evaluations of a pair.
+// K_HELM_*_TP: the same for 2 |k| h <= 1/4 with shorter polynomials.
 enum {
   K_LAP_SLP = 0,
   K_LAP_DLP = 1,
   K_HELM_SLP = 2,
   K_HELM_DLP = 3,
   K_HELM_SLP_SP = 4,
-  K_HELM_DLP_SP = 5
+  K_HELM_DLP_SP = 5,
+  K_HELM_SLP_TP = 6,
+  K_HELM_DLP_TP = 7
 };
-constexpr bool is_dlp(int ker) {
-  return ker == K_LAP_DLP || ker == K_HELM_DLP || ker == K_HELM_DLP_SP;
-}
+constexpr bool is_dlp(int ker) { return ker & 1; }
 constexpr bool small_phase(int ker) { return ker >= K_HELM_SLP_SP; }
+constexpr bool tiny_phase(int ker) { return ker >= K_HELM_SLP_TP; }
 
 // 1/sqrt(x): hardware estimate and one third-order correction
 // y (1 + e/2 + 3 e^2/8), e = 1 - x y^2.  Positive finite x only (x = 0
@@ -100,7 +102,9 @@ __device__ __forceinline__ void kcore(double r2, double kr, double ki,
     const double r = r2 * rs;
     g = is_dlp(KER) ? rs * rs * rs : rs;
     double s, c;
-    if constexpr (small_phase(KER)) {
+    if constexpr (tiny_phase(KER)) {
+      h2hip::sincos_poly_tiny(fma(kr, r, -ph0), s, c);
+    } else if constexpr (small_phase(KER)) {
       h2hip::sincos_poly(fma(kr, r, -ph0), s, c);
     } else {
       if (ki != 0.0) g *= exp(ki * r);
@@ -387,6 +391,17 @@ __device__ __forceinline__ void pair_sums(
           g1 = g * fma(dx, n1[0], fma(dy, n1[1], dz * n1[2]));
           if constexpr (TWO)
             g2 = g * fma(dx, n2[0], fma(dy, n2[1], dz * n2[2]));
+        }
+        if constexpr (CPLX && !BR && !BC) {
+          // one weight for both parts: one product less per value
+          const double w1 = W[i] * g1, w2 = W[i] * g2;
+          Ure[0] = fma(w1, fr, Ure[0]);
+          Uim[0] = fma(w1, fi, Uim[0]);
+          if constexpr (TWO) {
+            Vre[0] = fma(w2, fr, Vre[0]);
+            Vim[0] = fma(w2, fi, Vim[0]);
+          }
+          continue;
         }
 #pragma unroll
         for (int l = 0; l < NR; l++) {
@@ -1006,7 +1021,9 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
   // = A m, so the element matrix A M A^T is formed once after the sum.
   // kernel values at the difference d (FP64; mixed precision: d in FP64,
   // the value in FP32)
-  auto value = [&](const double *d, double (&vre)[ND], double (&vim)[ND]) {
+  // w: the weight, one product with both parts of a complex value
+  auto value = [&](const double *d, double w, double (&vre)[ND],
+                   double (&vim)[ND]) {
     if constexpr (MP) {
       const float dx = (float)d[0], dy = (float)d[1], dz = (float)d[2];
       float g, fr, fi;
@@ -1018,8 +1035,8 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
         float v = g;
         if constexpr (DLP)
           v *= fmaf(dx, (float)n[0], fmaf(dy, (float)n[1], dz * (float)n[2]));
-        vre[z] = CPLX ? fr * v : v;
-        vim[z] = CPLX ? fi * v : 0.0f;
+        vre[z] = w * (CPLX ? fr * v : v);
+        vim[z] = CPLX ? w * (fi * v) : 0.0;
       }
     } else {
       double g, fr, fi;
@@ -1031,6 +1048,7 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
         double v = g;
         if constexpr (DLP)
           v *= fma(d[0], n[0], fma(d[1], n[1], d[2] * n[2]));
+        v *= w;
         vre[z] = CPLX ? fr * v : v;
         vim[z] = CPLX ? fi * v : 0.0;
       }
@@ -1043,10 +1061,10 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
       d[k] = fma(-F2[k], sy,
                  fma(-F1[k], ty, fma(E2[k], sx, fma(E1[k], tx, D0[k]))));
     double vre[ND], vim[ND];
-    value(d, vre, vim);
+    value(d, wq, vre, vim);
     double ure[NR], uim[NR];
-    ure[0] = wq * vre[0];
-    uim[0] = wq * vim[0];
+    ure[0] = vre[0];
+    uim[0] = vim[0];
     if constexpr (BR) {
       ure[1] = ure[0] * tx;
       ure[2] = ure[0] * sx;
@@ -1131,17 +1149,17 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
               d2[d] = fma(c2[d], e2, t2[d]);
             }
             double v1r[ND], v1i[ND], v2r[ND], v2i[ND];
-            value(d1, v1r, v1i);
-            value(d2, v2r, v2i);
+            value(d1, w, v1r, v1i);
+            value(d2, w, v2r, v2i);
 #pragma unroll
             for (int z = 0; z < ND; z++) {
-              const double u1r = w * v1r[z], u2r = w * v2r[z];
+              const double u1r = v1r[z], u2r = v2r[z];
               U0r[z] += u1r;
               U2r[z] = fma(u1r, e2, U2r[z]);
               V0r[z] += u2r;
               V2r[z] = fma(u2r, e2, V2r[z]);
               if constexpr (CPLX) {
-                const double u1i = w * v1i[z], u2i = w * v2i[z];
+                const double u1i = v1i[z], u2i = v2i[z];
                 U0i[z] += u1i;
                 U2i[z] = fma(u1i, e2, U2i[z]);
                 V0i[z] += u2i;
@@ -1231,12 +1249,12 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
                 dd[d] = fma(cq, pq, bs[m][d]);
               }
               double vr[ND], vi[ND];
-              value(dd, vr, vi);
-              const double ur = w * vr[0];
+              value(dd, w, vr, vi);
+              const double ur = vr[0];
               W0r[m] += ur;
               W1r[m] = fma(ur, pq, W1r[m]);
               if constexpr (CPLX) {
-                const double ui = w * vi[0];
+                const double ui = vi[0];
                 W0i[m] += ui;
                 W1i[m] = fma(ui, pq, W1i[m]);
               }
@@ -1318,18 +1336,18 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
               // (single layer) or to its negative (double layer)
               double vr[ND], vi[ND];
               if (m < 3) {
-                value(dv[m], vr, vi);
+                value(dv[m], w, vr, vi);
                 pr[m] = vr[0];
                 pi[m] = vi[0];
               } else {
                 vr[0] = DLP ? -pr[m - 3] : pr[m - 3];
                 vi[0] = DLP ? -pi[m - 3] : pi[m - 3];
               }
-              const double ur = w * vr[0];
+              const double ur = vr[0];
               W0r[m] += ur;
               W1r[m] = fma(ur, bb, W1r[m]);
               if constexpr (CPLX) {
-                const double ui = w * vi[0];
+                const double ui = vi[0];
                 W0i[m] += ui;
                 W1i[m] = fma(ui, bb, W1i[m]);
               }

@@ -1,0 +1,15 @@
+// Near-field kernels of the Helmholtz single layer potential on
+// surfaces whose triangles are very short against the wave length (FP64).
+#include "nf_device.h"
+
+namespace h2hip {
+namespace nf {
+
+int launch_helmholtz_slp_tp(int rb, int cb, uint32_t q, const KArgs &a,
+                            uint32_t ntiles, const SPair *sp,
+                            const uint32_t *ncls, hipStream_t stream) {
+  return launch_family<K_HELM_SLP_TP>(rb, cb, q, a, ntiles, sp, ncls, stream);
+}
+
+}  // namespace nf
+}  // namespace h2hip

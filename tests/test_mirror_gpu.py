@@ -35,9 +35,10 @@ def run(h, plan, op, schedule):
     return out.download()
 
 
-# wave numbers on both sides of the small-phase bound 2 |k| h <= pi/4 (k = 1.3
-# and 1.31 on this mesh, h = 0.3015), and a damped one
-@pytest.mark.parametrize("kern,k", [(0, 0.0), (1, 1.3), (1, 1.31),
+# wave numbers below the tiny-phase bound 2 |k| h <= 1/4 (k = 0.41 on this mesh,
+# h = 0.3015) and on both sides of the small-phase bound pi/4 (k = 1.3
+# and 1.31), and a damped one
+@pytest.mark.parametrize("kern,k", [(0, 0.0), (1, 0.41), (1, 1.3), (1, 1.31),
                                     (1, 1.3 + 0.5j)])
 @pytest.mark.parametrize("layer", [0, 1, 2])
 @pytest.mark.parametrize("basis", [0, 1])
