@@ -725,6 +725,11 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
   a.are = op->layer != H2HIP_SLP ? op->alpha[0] : 0.0;
   a.aim = op->layer != H2HIP_SLP ? op->alpha[1] : 0.0;
   a.adj = op->layer == H2HIP_ADLP;
+  // given normals that are not perpendicular to the triangles: the general
+  // FP64 double layer kernels (no mirrored or fused tiles)
+  a.plane = s->plane;
+  const bool general =
+      op->layer != H2HIP_SLP && op->precision == 0 && !s->plane;
   for (int i = 0; i < 9; i++) a.mass[i] = op->mass[i];
   a.far = far;
   a.out = (double *)d_out;
@@ -732,7 +737,7 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
   a.tlist = nullptr;
   // mirrored tiles in the launches per rule class of the plan's own order
   const bool mir = !P->mirlist.empty() && !P->sorted && !P->persistent &&
-                   !P->fused && !far;
+                   !P->fused && !far && !general;
   a.mirlist = P->d_mirlist;
   a.nmir = mir ? (uint32_t)P->mirlist.size() : 0;
   a.nmain3 = P->nmain[CLS_IDENTICAL];
@@ -756,7 +761,7 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
     a.split = (uint32_t)std::max<uint64_t>(
         1, std::min<uint64_t>({(1024 + run - 1) / run, pairs / 512, 64}));
   }
-  if (P->fused && !far && op->q == 2 && op->q2 == 4) {
+  if (P->fused && !far && op->q == 2 && op->q2 == 4 && !general) {
     a.tiles = P->d_tiles_f.p;
     a.tlist = P->d_tpairs.p;
   }
@@ -1033,6 +1038,17 @@ int h2hip_surface_create(h2hip_surface **out, uint32_t vertices,
       h2 = std::max(h2, d0 * d0 + d1 * d1 + d2 * d2);
     }
   s->hmax = std::sqrt(h2);
+  if (n && g)
+    for (uint32_t i = 0; i < triangles && s->plane; i++)
+      for (int l = 0; l < 3; l++) {
+        const double *p = &s->x[3 * s->t[3 * i + l]];
+        const double *q = &s->x[3 * s->t[3 * i + (l + 1) % 3]];
+        const double e[3] = {q[0] - p[0], q[1] - p[1], q[2] - p[2]};
+        const double *m = &s->n[3 * i];
+        const double ne = e[0] * m[0] + e[1] * m[1] + e[2] * m[2];
+        if (!(ne * ne <= 1e-24 * (e[0] * e[0] + e[1] * e[1] + e[2] * e[2])))
+          s->plane = false;
+      }
   // triangles of each vertex, in decreasing triangle order as the
   // reference's prepend-built lists
   s->v2t_ptr.assign(vertices + 1, 0);

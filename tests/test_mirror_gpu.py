@@ -97,3 +97,34 @@ def test_unpaired_and_repeated_blocks_keep_single_tiles(basis, sphere8):
         for b, (ro, r, co, c) in enumerate(blocks):
             ref = orc.nearfield(ix[ro:ro + r], ix[co:co + c])
             assert rel_block_err(plan.block(got, b), ref) < 1e-12, b
+
+
+@pytest.mark.parametrize("kern,k", [(0, 0.0), (1, 2.0)])
+@pytest.mark.parametrize("layer", [1, 2])
+@pytest.mark.parametrize("basis", [0, 1])
+def test_given_normals_that_are_not_perpendicular(kern, k, layer, basis,
+                                                  sphere8):
+    """A surface may be given any normals; the double layers' kernels take
+    them as they are: <x - y, n> of every point."""
+    import h2lib_amd as h
+    x, t = sphere8["x"], sphere8["t"]
+    plain = h.Surface3d(x, t)
+    tilt = plain.n + 0.1 * np.roll(plain.n, 1, axis=1)
+    dofs = plain.vertices if basis else plain.triangles
+    rng = np.random.default_rng(8)
+    ridx = rng.permutation(dofs).astype(np.uint32)
+    blocks = mirrored_blocks((64, 9))
+    vals = []
+    # <d, n> is linear in n: the entries of the tilted normals are those of
+    # the true ones plus a tenth of those of the rolled ones (which are not
+    # perpendicular either)
+    for nn in (plain.n, np.roll(plain.n, 1, axis=1), tilt):
+        gr = h.Surface3d(x, t, nn, plain.g)
+        op = h.Bem3d(gr, kern, layer, 2, 4, basis, basis, alpha=0.0, k=k)
+        plan = h.NearfieldPlan(gr, basis, basis, ridx, ridx, blocks)
+        vals.append([run(h, plan, op, s) for s in ((0, 0, 0), (0, 1, 0),
+                                                   (0, 0, 1))])
+    for a, b, c in zip(*vals):
+        # (cancellation in the rolled entries: their scale bounds the error)
+        scale = max(np.abs(b).max(), np.abs(a).max())
+        assert np.abs(c - (a + 0.1 * b)).max() < 1e-13 * scale
