@@ -572,7 +572,12 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
            (uint64_t)tiles[y].nrsup * tiles[y].ncsup;
   });
   P->tiles.resize(tiles.size());
-  for (size_t i = 0; i < order.size(); i++) P->tiles[i] = tiles[order[i]];
+  // place[i]: where the i-th tile in block order went
+  std::vector<uint32_t> place(tiles.size());
+  for (size_t i = 0; i < order.size(); i++) {
+    P->tiles[i] = tiles[order[i]];
+    place[order[i]] = (uint32_t)i;
+  }
   tiles.clear();
   if (mirrors) {
     std::vector<uint64_t> key(order.size());
@@ -585,7 +590,6 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
   struct SPart {
     std::vector<SPair> by_cls[4];
     size_t nmain[4] = {0, 0, 0, 0};  // pairs to evaluate (mirrored tiles)
-    uint64_t pairs0 = 0;
   };
   const uint32_t ntiles = (uint32_t)P->tiles.size();
   const bool mir = !P->mirlist.empty();
@@ -598,49 +602,92 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
     const uint32_t m = P->tiles[q.tile].mirror;
     return m == q.tile ? (q.cls == CLS_IDENTICAL || q.r < q.c) : q.tile < m;
   };
-  std::vector<SPart> sparts(
-      std::max(1u, std::min<unsigned>(plan_threads(P->supp.size()), ntiles)));
-  parallel_ranges(ntiles, (unsigned)sparts.size(),
+  auto push = [&](SPart &W, uint32_t ti, uint32_t r, uint32_t c,
+                  const uint32_t *rv, const uint32_t *cv) {
+    SPair q;
+    q.tile = ti;
+    q.r = (uint16_t)r;
+    q.c = (uint16_t)c;
+    q.cls = (uint16_t)classify(rv, cv, q.perm);
+    W.by_cls[q.cls].push_back(q);
+    if (mir && is_main(q)) W.nmain[q.cls]++;
+  };
+  // Constant basis: a block's triangles are its DOFs, so its pairs are found
+  // in one pass over its rows and go to the tiles they fall into (a pass per
+  // tile looked up every row once for each tile of its row of tiles: 32
+  // times for a 2048 x 2048 block).  Linear basis: per tile.
+  const bool by_block = !rb && !cb;
+  const uint32_t nunits = by_block ? nblocks : ntiles;
+  std::vector<uint32_t> tile0;
+  if (by_block) {
+    tile0.resize(nblocks);
+    uint32_t t0 = 0;
+    for (uint32_t b = 0; b < nblocks; b++) {
+      tile0[b] = t0;
+      t0 += (blocks[4 * b + 1] + tile - 1) / tile *
+            ((blocks[4 * b + 3] + tile - 1) / tile);
+    }
+  }
+  std::vector<SPart> sparts(std::max(
+      1u, std::min<unsigned>(plan_threads(by_block ? dofs : P->supp.size()),
+                             nunits)));
+  for (const Tile &T : P->tiles) P->pairs[0] += (uint64_t)T.nrsup * T.ncsup;
+  parallel_ranges(nunits, (unsigned)sparts.size(),
                   [&](unsigned t, uint32_t lo, uint32_t hi) {
     SPart &W = sparts[t];
     std::vector<int32_t> cpos(s->nt, -1), cnext;
     std::vector<uint32_t> met;  // row that last met the triangle at c
-    for (uint32_t ti = lo; ti < hi; ti++) {
-      const Tile &T = P->tiles[ti];
-      W.pairs0 += (uint64_t)T.nrsup * T.ncsup;
-      // the first column position of each triangle; the further positions
-      // of a triangle that the column indices repeat (constant basis)
-      // chained behind it in increasing order
-      cnext.assign(T.ncsup, -1);
-      met.assign(T.ncsup, 0);
-      for (uint32_t c = T.ncsup; c-- > 0;) {
-        const uint32_t tri = P->supp[T.csup + c].tri;
+    // the pairs of nr row triangles with nc column triangles; the first
+    // column position of each triangle, the further positions of a triangle
+    // that the column indices repeat (constant basis) chained behind it in
+    // increasing order
+    auto search = [&](uint32_t nr, uint32_t nc, auto row, auto col,
+                      auto found) {
+      cnext.assign(nc, -1);
+      met.assign(nc, 0);
+      for (uint32_t c = nc; c-- > 0;) {
+        const uint32_t tri = col(c);
         cnext[c] = cpos[tri];
         cpos[tri] = (int32_t)c;
       }
-      for (uint32_t r = 0; r < T.nrsup; r++) {
-        const Supp &sr = P->supp[T.rsup + r];
+      for (uint32_t r = 0; r < nr; r++) {
+        const uint32_t *rv = &s->t[3 * row(r)];
         for (int l = 0; l < 3; l++) {
-          const uint32_t v = sr.v[l];
+          const uint32_t v = rv[l];
           for (uint32_t p = s->v2t_ptr[v]; p < s->v2t_ptr[v + 1]; p++) {
             const uint32_t tri = s->v2t[p];
             if (cpos[tri] < 0 || met[cpos[tri]] == r + 1) continue;
             met[cpos[tri]] = r + 1;
-            for (int32_t c = cpos[tri]; c >= 0; c = cnext[c]) {
-              SPair q;
-              q.tile = ti;
-              q.r = (uint16_t)r;
-              q.c = (uint16_t)c;
-              q.cls =
-                  (uint16_t)classify(sr.v, P->supp[T.csup + c].v, q.perm);
-              W.by_cls[q.cls].push_back(q);
-              if (mir && is_main(q)) W.nmain[q.cls]++;
-            }
+            for (int32_t c = cpos[tri]; c >= 0; c = cnext[c])
+              found(r, (uint32_t)c, rv, &s->t[3 * tri]);
           }
         }
       }
-      for (uint32_t c = 0; c < T.ncsup; c++)
-        cpos[P->supp[T.csup + c].tri] = -1;
+      for (uint32_t c = 0; c < nc; c++) cpos[col(c)] = -1;
+    };
+    for (uint32_t u = lo; u < hi; u++) {
+      if (by_block) {
+        const uint32_t *ri = ridx_all + blocks[4 * u];
+        const uint32_t *ci = cidx_all + blocks[4 * u + 2];
+        const uint32_t tc = (blocks[4 * u + 3] + tile - 1) / tile;
+        search(
+            blocks[4 * u + 1], blocks[4 * u + 3],
+            [&](uint32_t r) { return ri[r]; },
+            [&](uint32_t c) { return ci[c]; },
+            [&](uint32_t r, uint32_t c, const uint32_t *rv,
+                const uint32_t *cv) {
+              const uint32_t k = r / tile * tc + c / tile;
+              push(W, place[tile0[u] + k], r % tile, c % tile, rv, cv);
+            });
+      } else {
+        const Tile &T = P->tiles[u];
+        search(
+            T.nrsup, T.ncsup,
+            [&](uint32_t r) { return P->supp[T.rsup + r].tri; },
+            [&](uint32_t c) { return P->supp[T.csup + c].tri; },
+            [&](uint32_t r, uint32_t c, const uint32_t *rv,
+                const uint32_t *cv) { push(W, u, r, c, rv, cv); });
+      }
     }
   });
   // where each part's pairs go: the class lists (identical, edge, vertex)
@@ -649,7 +696,6 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
   const unsigned np = (unsigned)sparts.size();
   std::vector<size_t> cdst(4 * (size_t)np), odst(4 * (size_t)np);
   size_t nsp = 0;
-  for (auto &W : sparts) P->pairs[0] += W.pairs0;
   for (int c = 3; c >= 1; c--) {
     // mirrored tiles: the pairs to evaluate first, then the others
     size_t nmain = 0;
@@ -816,8 +862,10 @@ struct CbCtx {
   DevBuf<unsigned char> out;
   void *stage = nullptr;
   size_t stage_cap = 0;
+  std::vector<hipEvent_t> ev;  // pieces of a large output (copy_out)
   bool busy = false;
   ~CbCtx() {
+    for (hipEvent_t e : ev) (void)hipEventDestroy(e);
     if (stage) (void)hipHostFree(stage);
     if (st) (void)hipStreamDestroy(st);
   }
@@ -857,43 +905,93 @@ namespace {
 
 constexpr int CB_CONTEXTS = 4;
 
-// Copies the packed column-major blocks of `stage` into their host
-// windows (block b: ld[b], written in the block's storage orientation),
-// split over a few threads for large copies.
-void scatter_blocks(const unsigned char *stage, const uint64_t *off,
-                    const uint32_t *blocks, const uint8_t *ntr,
-                    void *const *dst, const size_t *ld, size_t nblocks,
-                    size_t es) {
-  auto one = [&](size_t b) {
+// Copies bytes [lo, hi) of the packed column-major blocks of `stage` into
+// their host windows (block b: ld[b], written in the block's storage
+// orientation).
+void scatter_range(const unsigned char *stage, const uint64_t *off,
+                   const uint32_t *blocks, const uint8_t *ntr,
+                   void *const *dst, const size_t *ld, size_t nblocks,
+                   size_t es, size_t lo, size_t hi) {
+  // the block that holds byte lo: the last that starts at or before it
+  size_t b = std::upper_bound(off, off + nblocks, lo / es) - off;
+  for (b = b ? b - 1 : 0; b < nblocks && es * off[b] < hi; b++) {
     const uint32_t rows = blocks[4 * b + 1], cols = blocks[4 * b + 3];
-    const size_t wr = ntr[b] ? cols : rows, wc = ntr[b] ? rows : cols;
-    const unsigned char *src = stage + es * off[b];
+    const size_t wr = es * (ntr[b] ? cols : rows), wc = ntr[b] ? rows : cols;
+    const size_t b0 = es * off[b];
+    const size_t from = std::max(lo, b0) - b0, to = std::min(hi - b0, wr * wc);
     unsigned char *d = (unsigned char *)dst[b];
-    if (ld[b] == wr) {
-      std::memcpy(d, src, es * wr * wc);
-    } else {
-      for (size_t j = 0; j < wc; j++)
-        std::memcpy(d + es * j * ld[b], src + es * j * wr, es * wr);
+    if (es * ld[b] == wr) {
+      if (to > from) std::memcpy(d + from, stage + b0 + from, to - from);
+      continue;
+    }
+    for (size_t p = from; p < to;) {
+      const size_t j = p / wr, i = p - j * wr, n = std::min(to - p, wr - i);
+      std::memcpy(d + es * ld[b] * j + i, stage + b0 + p, n);
+      p += n;
+    }
+  }
+}
+
+// Device output -> pinned staging memory -> host windows.  Small outputs in
+// one piece; larger ones in pieces of 2 MB, all copies queued at once, each
+// piece scattered when its event has passed, by a few threads: the copy into
+// the caller's memory waited for the transfer and was longer (2048 x 2048
+// real entries with the plan and the kernels: 2.60 -> 1.35 ms, of which the
+// search of the pairs by blocks took some 0.5 ms).
+int copy_out(CbCtx &C, const uint64_t *off, const uint32_t *blocks,
+             const uint8_t *ntr, void *const *dst, const size_t *ld,
+             size_t nblocks, size_t es, size_t bytes) {
+  const unsigned char *stage = (const unsigned char *)C.stage;
+  constexpr size_t PIECE = (size_t)2 << 20;
+  const size_t np = (bytes + PIECE - 1) / PIECE;
+  if (np <= 1) {
+    H2HIP_CHECK(hipMemcpyAsync(C.stage, C.out.p, bytes,
+                               hipMemcpyDeviceToHost, C.st));
+    H2HIP_CHECK(hipStreamSynchronize(C.st));
+    scatter_range(stage, off, blocks, ntr, dst, ld, nblocks, es, 0, bytes);
+    return H2HIP_OK;
+  }
+  while (C.ev.size() < std::min<size_t>(np, 64)) {
+    hipEvent_t e;
+    H2HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    C.ev.push_back(e);
+  }
+  const size_t groups = C.ev.size() < np ? C.ev.size() : np;
+  const size_t per = (np + groups - 1) / groups * PIECE;
+  const size_t ng = (bytes + per - 1) / per;
+  for (size_t g = 0; g < ng; g++) {
+    const size_t lo = g * per, n = std::min(per, bytes - lo);
+    H2HIP_CHECK(hipMemcpyAsync((unsigned char *)C.stage + lo, C.out.p + lo, n,
+                               hipMemcpyDeviceToHost, C.st));
+    H2HIP_CHECK(hipEventRecord(C.ev[g], C.st));
+  }
+  int device = 0;
+  H2HIP_CHECK(hipGetDevice(&device));
+  std::atomic<size_t> next{0};
+  std::atomic<int> bad{0};
+  auto work = [&]() {
+    (void)hipSetDevice(device);
+    for (size_t g; (g = next.fetch_add(1)) < ng;) {
+      if (hipEventSynchronize(C.ev[g]) != hipSuccess) {
+        bad = 1;
+        return;
+      }
+      scatter_range(stage, off, blocks, ntr, dst, ld, nblocks, es, g * per,
+                    std::min(bytes, (g + 1) * per));
     }
   };
-  uint64_t bytes = 0;
-  for (size_t b = 0; b < nblocks; b++)
-    bytes += (uint64_t)blocks[4 * b + 1] * blocks[4 * b + 3];
-  bytes *= es;
-  const unsigned hw = std::max(1u, std::min(16u,
-                                            std::thread::hardware_concurrency()));
-  const unsigned nt = bytes < (16u << 20) ? 1u : hw;
-  if (nt <= 1 || nblocks < 2) {
-    for (size_t b = 0; b < nblocks; b++) one(b);
-    return;
-  }
-  std::atomic<size_t> next{0};
+  const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
+  const unsigned nt = (unsigned)std::min<size_t>({ng, hw, bytes >> 23, 8});
   std::vector<std::thread> pool;
-  for (unsigned t = 0; t < nt; t++)
-    pool.emplace_back([&]() {
-      for (size_t b; (b = next.fetch_add(1)) < nblocks;) one(b);
-    });
+  for (unsigned t = 1; t < nt; t++) pool.emplace_back(work);
+  work();
   for (auto &th : pool) th.join();
+  H2HIP_CHECK(hipStreamSynchronize(C.st));
+  if (bad) {
+    set_error("h2hip_nearfield: copy to the host failed");
+    return H2HIP_EDEVICE;
+  }
+  return H2HIP_OK;
 }
 
 // Plans, computes and writes one group of blocks (one rule) through a
@@ -926,12 +1024,8 @@ int run_blocks(const h2hip_op *op, CbCtx &C, int far,
     rc = execute(op, &C.plan, far, C.out.p, C.st);
   }
   if (rc != H2HIP_OK) return rc;
-  H2HIP_CHECK(hipMemcpyAsync(C.stage, C.out.p, bytes, hipMemcpyDeviceToHost,
-                             C.st));
-  H2HIP_CHECK(hipStreamSynchronize(C.st));
-  scatter_blocks((const unsigned char *)C.stage, C.plan.off.data(), blocks,
-                 ntr, dst, ld, nblocks, es);
-  return H2HIP_OK;
+  return copy_out(C, C.plan.off.data(), blocks, ntr, dst, ld, nblocks, es,
+                  bytes);
 }
 
 // A free callback context of op (waits while all are busy).
