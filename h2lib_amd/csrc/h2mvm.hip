@@ -555,6 +555,15 @@ __device__ __forceinline__ void dot_row(const double *__restrict__ M,
   }
 }
 
+// Place of input j of vector v in a wave's LDS slice: one vector as (re, im)
+// pairs; several with the vectors of an input next to each other (real
+// matrices without imaginary parts), so that a wave's broadcast reads take
+// two values at a time.  Eight vectors, 32768 triangles: NVTIME.
+template <int C, int NV>
+__device__ __forceinline__ uint32_t lx(uint32_t v, uint32_t j) {
+  return NV == 1 ? 2 * j : C ? 2 * (j * NV + v) : j * NV + v;
+}
+
 // ar/ai[v] += sum_j M[base + j sj] x_v[j] over n columns for NV vectors in
 // LDS (complex pairs when C; CONJ: the conjugate of M; NTL: non-temporal
 // loads): B columns' entries are loaded together, the last batch with its
@@ -585,8 +594,8 @@ __device__ __forceinline__ void dot_cols_nv(const double *__restrict__ M,
         const double sr = mr[u], si = CONJ ? -mi[u] : mi[u];
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-          const double xr = xs[v * 2 * XR + 2 * j];
-          const double xi = xs[v * 2 * XR + 2 * j + 1];
+          const double xr = xs[lx<C, NV>(v, j)];
+          const double xi = xs[lx<C, NV>(v, j) + 1];
           ar[v] = fma(sr, xr, ar[v]);
           if constexpr (C) {
             ar[v] = fma(-si, xi, ar[v]);
@@ -671,8 +680,8 @@ __device__ __forceinline__ void mf_laplace4(const double *p3,
         const double sr = KCONST * cpl_rsqrt(fma(d2, d2, s1));
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-          ar[v] = fma(sr, xs[v * 2 * XR + 2 * j], ar[v]);
-          if constexpr (C) ai[v] = fma(sr, xs[v * 2 * XR + 2 * j + 1], ai[v]);
+          ar[v] = fma(sr, xs[lx<C, NV>(v, j)], ar[v]);
+          if constexpr (C) ai[v] = fma(sr, xs[lx<C, NV>(v, j) + 1], ai[v]);
         }
       }
     }
@@ -770,8 +779,8 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
       const uint32_t v = e / in.rank, j = e - v * in.rank;
       double xr = 0.0, xi = 0.0;
       if (v < a.v.nv) ld<C>(a.xt + v * a.cstride, in.coef + j, xr, xi);
-      xs[v * 2 * XR + 2 * j] = xr;
-      xs[v * 2 * XR + 2 * j + 1] = xi;
+      xs[lx<C, NV>(v, j)] = xr;
+      if constexpr (C || NV == 1) xs[lx<C, NV>(v, j) + 1] = xi;
     }
     // the wave reads what its own lanes wrote: LDS keeps the order of
     // one wave's accesses, the compiler must not move them
@@ -808,8 +817,8 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
               si = -si;
 #pragma unroll
               for (int v = 0; v < NV; v++) {
-                const double xr = xs[v * 2 * XR + 2 * j];
-                const double xi = xs[v * 2 * XR + 2 * j + 1];
+                const double xr = xs[lx<C, NV>(v, j)];
+                const double xi = xs[lx<C, NV>(v, j) + 1];
                 ar[v] = fma(sr, xr, ar[v]);
                 if constexpr (C) {
                   ar[v] = fma(-si, xi, ar[v]);
@@ -841,8 +850,8 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
                         a.cs.kdamp, sr, si);
 #pragma unroll
               for (int v = 0; v < NV; v++) {
-                const double xr = xs[v * 2 * XR + 2 * j];
-                const double xi = xs[v * 2 * XR + 2 * j + 1];
+                const double xr = xs[lx<C, NV>(v, j)];
+                const double xi = xs[lx<C, NV>(v, j) + 1];
                 ar[v] = fma(sr, xr, ar[v]);
                 if constexpr (C) {
                   ar[v] = fma(-si, xi, ar[v]);
@@ -896,8 +905,8 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
     const uint32_t v = e / nin, j = e - v * nin;
     double xr = 0.0, xi = 0.0;
     if (v < a.v.nv) ld<C>(a.v.x[v], iidx[j], xr, xi);
-    xs[v * 2 * XR + 2 * j] = xr;
-    xs[v * 2 * XR + 2 * j + 1] = xi;
+    xs[lx<C, NV>(v, j)] = xr;
+    if constexpr (C || NV == 1) xs[lx<C, NV>(v, j) + 1] = xi;
   }
   __builtin_amdgcn_wave_barrier();
   for (uint32_t i = lane; i < nout; i += 64) {
@@ -933,7 +942,7 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
 template <int C, bool TRANS, int NV, bool MF = false, bool ORD = false>
 __global__ __launch_bounds__(NT) void couple_near(CNArgs a) {
   constexpr int XS = NV * 2 * (NV == 1 ? MAXRANK : 64);  // per wave
-  __shared__ double xs_all[WPB * XS];
+  __shared__ alignas(16) double xs_all[WPB * XS];
   couple_near_dev<C, TRANS, NV, MF, ORD>(
       a, blockIdx.x * WPB + (threadIdx.x >> 6),
       xs_all + (threadIdx.x >> 6) * XS);
@@ -1432,6 +1441,123 @@ __global__ __launch_bounds__(NT, C && MF ? 3 : 1) void couple_pairs64(
   couple_pairs64_dev<C, MF, ADJ, DAMP>(a, pairs, npair, blockIdx.x);
 }
 
+// Mirrored pairs for several vectors: the lane's sub-block of S (complex:
+// half of its columns at a time) is read or computed once into registers,
+// then each vector's sums are formed with it as above.  Products at 32768
+// triangles (Laplace), 2 / 4 / 8 vectors: read couplings 87 / 101 / 145 ->
+// 68 / 87 / 132 us, their adjoint 197 / 208 / 334 -> 95 / 114 / 178 us,
+// computed 61 / 79 / 133 -> 58 / 78 / 124 us (there the output atomics are
+// most of the time).
+template <int C, bool MF, bool ADJ, bool DAMP>
+__global__ __launch_bounds__(NT, C && !DAMP ? 1 : 2) void couple_pairs64_nv(
+    CNArgs a, const PairD *__restrict__ pairs, uint32_t npair) {
+  constexpr double KCONST = 0.0795774715459476679;
+  constexpr int CW = C ? 4 : 8, NPASS = 8 / CW;
+  const uint32_t w =
+      __builtin_amdgcn_readfirstlane(blockIdx.x * WPB + (threadIdx.x >> 6));
+  if (w >= npair) return;  // uniform over the wave; no block barrier
+  const int lane = threadIdx.x & 63, la = lane >> 3, lb = lane & 7;
+  const PairD b = pairs[w];
+  const uint64_t out_r = ADJ ? b.in_r : b.out_r, in_r = ADJ ? b.out_r : b.in_r;
+  const uint64_t out_c = ADJ ? b.in_c : b.out_c, in_c = ADJ ? b.out_c : b.in_c;
+  auto row = [&](int u) {
+    return MF ? 8 * la + u
+              : C ? la + 8 * u : 2 * la + (u & 1) + 16 * (u >> 1);
+  };
+#pragma unroll 1
+  for (int q = 0; q < NPASS; q++) {
+    double sr[8][CW], si[C ? 8 : 1][C ? CW : 1];
+    if constexpr (MF) {
+      const double *pr = a.cs.rpts + 12 * (uint64_t)b.r;
+      const double *pc = a.cs.cpts + 12 * (uint64_t)b.c;
+      const double d0 = pr[la >> 1] - pc[lb >> 1];
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+#pragma unroll
+        for (int v = 0; v < CW; v++) {
+          const double d1 = pr[4 + 2 * (la & 1) + (u >> 2)] -
+                            pc[4 + 2 * (lb & 1) + (CW == 4 ? q : v >> 2)];
+          const double d2 = pr[8 + (u & 3)] - pc[8 + (v & 3)];
+          const double r2 = fma(d2, d2, fma(d1, d1, d0 * d0));
+          const double rs = cpl_rsqrt(r2);
+          if constexpr (C) {
+            const double r = r2 * rs;
+            double amp = KCONST * rs;
+            if constexpr (DAMP) amp *= h2hip::exp_cw(a.cs.kdamp * r);
+            double sn, cs;
+            h2hip::sincos_cw(a.cs.kr * r, sn, cs);
+            sr[u][v] = amp * cs;
+            si[u][v] = ADJ ? -(amp * sn) : amp * sn;
+          } else {
+            sr[u][v] = KCONST * rs;
+          }
+        }
+    } else {
+      const dbl2 *S = (const dbl2 *)(a.S + (C ? 2 : 1) * b.soff);
+#pragma unroll
+      for (int v = 0; v < CW; v++)
+#pragma unroll
+        for (int u = 0; u < (C ? 8 : 4); u++) {
+          const uint32_t j = 8 * lb + CW * q + v;
+          const dbl2 m = __builtin_nontemporal_load(
+              S + (C ? 64 * j + la + 8 * u : 32 * j + la + 8 * u));
+          if constexpr (C) {
+            sr[u][v] = m.x;
+            si[u][v] = ADJ ? -m.y : m.y;
+          } else {
+            sr[2 * u][v] = m.x;
+            sr[2 * u + 1][v] = m.y;
+          }
+        }
+    }
+#pragma unroll 1
+    for (uint32_t k = 0; k < a.v.nv; k++) {
+      const double *xt = a.xt + k * a.cstride;
+      double *yt = a.yt + k * a.cstride;
+      double xr[8], xi[8], cr[CW], ci[CW], ar[8], ai[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        xi[u] = 0.0;
+        ld<C>(xt, in_r + row(u), xr[u], xi[u]);
+        ar[u] = ai[u] = 0.0;
+      }
+#pragma unroll
+      for (int v = 0; v < CW; v++) {
+        double yr = 0.0, yi = 0.0;
+        ld<C>(xt, in_c + 8 * lb + CW * q + v, yr, yi);
+        double tr = 0.0, ti = 0.0;
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+          ar[u] = fma(sr[u][v], yr, ar[u]);
+          tr = fma(sr[u][v], xr[u], tr);
+          if constexpr (C) {
+            ar[u] = fma(-si[u][v], yi, ar[u]);
+            ai[u] = fma(sr[u][v], yi, fma(si[u][v], yr, ai[u]));
+            tr = fma(-si[u][v], xi[u], tr);
+            ti = fma(sr[u][v], xi[u], fma(si[u][v], xr[u], ti));
+          }
+        }
+        cr[v] = tr;
+        ci[v] = ti;
+      }
+      const double tr = column_sum<CW>(cr, lane);
+      const double ti = C ? column_sum<CW>(ci, lane) : 0.0;
+      h2hip::bfly_step<4>(ar, lane);
+      h2hip::bfly_step<2>(ar, lane);
+      h2hip::bfly_step<1>(ar, lane);
+      if constexpr (C) {
+        h2hip::bfly_step<4>(ai, lane);
+        h2hip::bfly_step<2>(ai, lane);
+        h2hip::bfly_step<1>(ai, lane);
+      }
+      atomic_add<C>(yt, out_r + row(lb), ar[0], ai[0]);
+      // (CW = 4: lanes l and l ^ 32 hold the same column)
+      if (NPASS == 1 || lane < 32)
+        atomic_add<C>(yt, out_c + 8 * lb + CW * q + (la & (CW - 1)), tr, ti);
+    }
+  }
+}
+
 // The computed complex couplings and the near blocks (a.nfar = 0) of a
 // forward product in one launch, their workgroups interleaved: the couplings
 // are bound by VALU issue and the near blocks by memory.  pb workgroups of
@@ -1712,8 +1838,8 @@ __device__ __forceinline__ void dot_strided_nv(const double *__restrict__ M,
     for (int u = 0; u < B; u++)
 #pragma unroll
       for (int v = 0; v < NV; v++) {
-        ar[v] = fma(m[u], xs[v * 2 * XR + 2 * (i + u)], ar[v]);
-        if constexpr (C) ai[v] = fma(m[u], xs[v * 2 * XR + 2 * (i + u) + 1], ai[v]);
+        ar[v] = fma(m[u], xs[lx<C, NV>(v, i + u)], ar[v]);
+        if constexpr (C) ai[v] = fma(m[u], xs[lx<C, NV>(v, i + u) + 1], ai[v]);
       }
   }
   if (i < n) {
@@ -1729,9 +1855,9 @@ __device__ __forceinline__ void dot_strided_nv(const double *__restrict__ M,
       if ((uint32_t)u < rem) {
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-          ar[v] = fma(m[u], xs[v * 2 * XR + 2 * (i + u)], ar[v]);
+          ar[v] = fma(m[u], xs[lx<C, NV>(v, i + u)], ar[v]);
           if constexpr (C)
-            ai[v] = fma(m[u], xs[v * 2 * XR + 2 * (i + u) + 1], ai[v]);
+            ai[v] = fma(m[u], xs[lx<C, NV>(v, i + u) + 1], ai[v]);
         }
       }
   }
@@ -1784,8 +1910,8 @@ __device__ __forceinline__ void fwd_flat_dev(const FlatArgs &a, uint32_t blk,
     const uint32_t v = e / sz, i = e - v * sz;
     double xr = 0.0, xi = 0.0;
     if (v < a.v.nv) ld<C>(a.v.x[v], a.idx[L.off + i], xr, xi);
-    xs[v * 2 * XR + 2 * i] = xr;
-    xs[v * 2 * XR + 2 * i + 1] = xi;
+    xs[lx<C, NV>(v, i)] = xr;
+    if constexpr (C || NV == 1) xs[lx<C, NV>(v, i) + 1] = xi;
   }
   // the wave reads what its own lanes wrote: LDS keeps the order of one
   // wave's accesses, the compiler must not move them
@@ -1816,7 +1942,7 @@ __device__ __forceinline__ void fwd_flat_dev(const FlatArgs &a, uint32_t blk,
 template <int C, int K, int NV, bool ORD = false>
 __global__ __launch_bounds__(NT) void fwd_flat(FlatArgs a) {
   constexpr int XS = NV * 2 * (NV == 1 ? MAXRANK : 64);
-  __shared__ double xs_all[WPB * XS];
+  __shared__ alignas(16) double xs_all[WPB * XS];
   fwd_flat_dev<C, K, NV, ORD>(a, blockIdx.x, gridDim.x,
                               xs_all + (threadIdx.x >> 6) * XS);
 }
@@ -1829,7 +1955,7 @@ template <int C, int K, int NV, bool ORD = false, bool TRANS = false>
 __global__ __launch_bounds__(NT) void fwd_flat_near(FlatArgs a, CNArgs c,
                                                     uint32_t fb) {
   constexpr int XS = NV * 2 * (NV == 1 ? MAXRANK : 64);
-  __shared__ double xs_all[WPB * XS];
+  __shared__ alignas(16) double xs_all[WPB * XS];
   double *xs = xs_all + (threadIdx.x >> 6) * XS;
   if (blockIdx.x < fb)  // uniform over the block
     fwd_flat_dev<C, K, NV, ORD>(a, blockIdx.x, fb, xs);
@@ -1929,7 +2055,7 @@ __global__ __launch_bounds__(NT) void back_flat_ord(FlatArgs a,
                                                     const uint32_t *ibeg,
                                                     uint32_t nleaves) {
   constexpr int XR = NV == 1 ? MAXRANK : 64;
-  __shared__ double ys_all[WPB][NV * 2 * XR];
+  __shared__ alignas(16) double ys_all[WPB][NV * 2 * XR];
   // the input coefficients xt, zero for the next product whatever its mode
   flat_zero(a, blockIdx.x, gridDim.x);
   const uint32_t l = blockIdx.x * WPB + (threadIdx.x >> 6);
@@ -1954,8 +2080,8 @@ __global__ __launch_bounds__(NT) void back_flat_ord(FlatArgs a,
       const uint32_t v = e / k, j = e - v * k;
       double yr = 0.0, yi = 0.0;
       if (v < a.v.nv) ld<C>(a.yt + v * a.cstride, A.coef + j, yr, yi);
-      ys[v * 2 * XR + 2 * j] = yr;
-      ys[v * 2 * XR + 2 * j + 1] = yi;
+      ys[lx<C, NV>(v, j)] = yr;
+      if constexpr (C || NV == 1) ys[lx<C, NV>(v, j) + 1] = yi;
     }
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
@@ -1990,7 +2116,7 @@ __global__ __launch_bounds__(NT) void back_flat_ord(FlatArgs a,
 template <int C, int K, int NV>
 __global__ __launch_bounds__(NT) void back_flat(FlatArgs a) {
   constexpr int XR = NV == 1 ? MAXRANK : 64;
-  __shared__ double ys_all[WPB][NV * 2 * XR];
+  __shared__ alignas(16) double ys_all[WPB][NV * 2 * XR];
   flat_zero(a, blockIdx.x, gridDim.x);  // the input coefficients xt, for
                                         // the next product
   const uint32_t w = blockIdx.x * WPB + (threadIdx.x >> 6);
@@ -2005,8 +2131,8 @@ __global__ __launch_bounds__(NT) void back_flat(FlatArgs a) {
     const uint32_t v = e / k, j = e - v * k;
     double yr = 0.0, yi = 0.0;
     if (v < a.v.nv) ld<C>(a.yt + v * a.cstride, A.coef + j, yr, yi);
-    ys[v * 2 * XR + 2 * j] = yr;
-    ys[v * 2 * XR + 2 * j + 1] = yi;
+    ys[lx<C, NV>(v, j)] = yr;
+    if constexpr (C || NV == 1) ys[lx<C, NV>(v, j) + 1] = yi;
   }
   __builtin_amdgcn_wave_barrier();
   for (uint32_t i = lane; i < sz; i += 64) {
@@ -2571,17 +2697,22 @@ void launch(const VecSet &vs, const h2hip_h2matrix *H, double *xt, double *yt,
                    H->maxleaf <= 64;
   const int cm = C ? 2 : 1;
   const bool mf = H->cpl_recompute && !symm;
-  // one vector, order-4 interpolation couplings (read or computed) in
-  // mirrored pairs: each value once for a block and its mirror
-  const bool pairs64 = NV == 1 && !symm && !ord && !tv && H->pairs_on &&
-                       H->npair && H->cpl_known && H->cpl.m == 4;
+  // order-4 interpolation couplings (read or computed) in mirrored pairs:
+  // each value once for a block and its mirror
+  // (several vectors keep the matrix cores where they are asked for; more
+  // than four complex vectors with read couplings, forward, keep a wave per
+  // block: 259 us against 279 for eight at 12800 triangles)
+  const bool pairs64 = !symm && !ord && !tv && H->pairs_on && H->npair &&
+                       H->cpl_known && H->cpl.m == 4 &&
+                       (NV == 1 || C || mf || !H->cpl_mfma || trans) &&
+                       !(C && NV > 4 && !mf && !trans);
   // the near blocks of a flat, not symmetric product run with the computed
   // complex pairs or in the upward launch (not the workgroup adjoint blocks
   // of several vectors or fixed-order sums).  With the pairs where these are
   // at least eight rounds of the 768 resident workgroups: 131072 triangles
   // 758 -> 657 us; at 32768 (two and a half rounds) the last round's pairs
   // run alone, 190 -> 204 us.
-  const bool pairs_near = C && pairs64 && mf && flat && !trans &&
+  const bool pairs_near = C && NV == 1 && pairs64 && mf && flat && !trans &&
                           H->nnear > 0 && H->npair >= 8 * 768 * WPB;
   const bool fuse = flat && !symm && !pairs_near &&
                     (!twg || (NV == 1 && !ord)) && H->nnear > 0 &&
@@ -2742,6 +2873,22 @@ void launch(const VecSet &vs, const h2hip_h2matrix *H, double *xt, double *yt,
       }
       c.nfar = 0;  // the near blocks (if any are left) as below
     }
+  } else if (pairs64) {
+    const dim3 gp((H->npair + WPB - 1) / WPB);
+    const PairD *pl = H->d_pairs.p;
+    const bool damp = C && mf && H->cpl.kdamp != 0.0;
+    auto go = [&](auto adj) {
+      constexpr bool ADJ = decltype(adj)::value;
+      auto k = !mf ? couple_pairs64_nv<C, false, ADJ, false>
+               : C && damp ? couple_pairs64_nv<C, true, ADJ, C != 0>
+                           : couple_pairs64_nv<C, true, ADJ, false>;
+      hipLaunchKernelGGL(k, gp, dim3(NT), 0, st, c, pl, H->npair);
+    };
+    if (trans)
+      go(std::true_type{});
+    else
+      go(std::false_type{});
+    c.nfar = 0;
   }
   if (twg) {
     // stored couplings and near blocks: one workgroup each; computed

@@ -263,12 +263,13 @@ int h2hip_h2matrix_set_mfma(h2hip_h2matrix *H, int on);
 /* Couplings of an order-4 or -5 interpolation matrix (Laplace or Helmholtz)
  * whose row and column boxes have the same points and whose admissible
  * blocks come in mirrored pairs (r, c) / (c, r), as for the operators of one
- * mesh: the one-vector products evaluate each coupling value once for both
- * blocks of a pair (on = 1, the default; no counterpart in the reference):
- * order 4, read (h2hip_h2matrix_interp_couplings) or computed in the
- * product (coupling mode 1), forward and adjoint; order 5, computed,
- * forward.  Reproducible mode, batched products and the adjoint from kept
- * transposes keep one evaluation per block. */
+ * mesh: the products use each coupling value once for both blocks of a pair
+ * (on = 1, the default; no counterpart in the reference): order 4, read
+ * (h2hip_h2matrix_interp_couplings) or computed in the product (coupling
+ * mode 1), forward and adjoint, of one or several vectors; order 5,
+ * computed, forward, one vector.  Reproducible mode, the adjoint from kept
+ * transposes, products on matrix cores and forward products of more than
+ * four complex vectors with read couplings keep one evaluation per block. */
 int h2hip_h2matrix_set_coupling_pairs(h2hip_h2matrix *H, int on);
 /* The number of mirrored pairs found by h2hip_h2matrix_interp_couplings
  * (0: the structure is not symmetric, or not order 4 or 5; -1: H null). */

@@ -65,6 +65,55 @@ def test_pairs_and_adjoint_match_general_kernels(kern, layer, basis, k, clf):
         h.set_reproducible(True)
 
 
+@pytest.mark.parametrize("kern,layer,basis,k", [
+    (0, 0, 1, 0.0), (0, 1, 1, 0.0), (1, 0, 0, 3.0), (1, 1, 0, 2.0 + 0.5j)])
+@pytest.mark.parametrize("nvec", [2, 3, 8])
+def test_batched_pairs_match_general_kernels(kern, layer, basis, k, nvec):
+    """Several vectors: the pairs' values used for all of them, and the
+    vectors' layout in the other kernels."""
+    import h2lib_amd as h
+    from h2lib_amd import geometry as G
+    from h2lib_amd.h2matrix import H2Matrix
+    mesh = G.sphere(13)
+    gr = h.Surface3d(mesh.x, mesh.t, mesh.n, mesh.g)
+    op = h.Bem3d(gr, kern, layer, 2, 4, basis, basis,
+                 alpha=0.5 if layer else 0.0, k=k)
+    rt = G.ClusterTree(mesh, basis, 60)
+    bt = G.BlockTree(rt, rt, 2.0, 0)
+    H = H2Matrix(op, mesh, rt, rt, bt, 4)
+    H.set_schedule(2)
+    assert H.coupling_pairs() > 0
+    rng = np.random.default_rng(5)
+    d_x = [h.DeviceArray.from_host((rng.standard_normal(H.n) + (
+        1j * rng.standard_normal(H.n) if kern else 0.0)).astype(H.dtype))
+        for _ in range(nvec)]
+    d_y = [h.DeviceArray(H.n, H.dtype) for _ in range(nvec)]
+    alphas = [0.5 + 0.25 * v for v in range(nvec)]
+
+    def product(trans):
+        for y in d_y:
+            y.zero()
+        H.addeval_batch(alphas, d_x, d_y, trans=trans)
+        return np.array([y.download() for y in d_y])
+
+    try:
+        for mode in (0, 1):
+            H.set_coupling_mode(mode)
+            for trans in (False, True):
+                h.set_reproducible(True)
+                want = product(trans)
+                h.set_reproducible(False)
+                for pairs in (1, 0):
+                    H.set_coupling_pairs(pairs)
+                    for _ in range(2):
+                        err = np.abs(product(trans) - want).max(1)
+                        assert (err < 1e-13 * np.abs(want).max(1)).all(), (
+                            mode, trans, pairs, err)
+                H.set_coupling_pairs(1)
+    finally:
+        h.set_reproducible(True)
+
+
 def test_large_helmholtz_product_runs_near_blocks_with_the_pairs():
     """At 131072 triangles the near blocks share the launch of the computed
     couplings."""
