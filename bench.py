@@ -889,7 +889,7 @@ def bench_dirichlet(h, mesh, args, stream):
         "operator_build_s": build_s,
         "couplings_in_solves": modes,
         "matvec": {
-            "kernels": ("fwd_flat_near + couple_near + back_flat (Laplace "
+            "kernels": ("fwd_flat_near + couple_pairs64 + back_flat (Laplace "
                         "SLP)" if best == 2 else
                         "fwd_up (+ fwd_level) + couple_near + down_back "
                         "(Laplace SLP)"),
@@ -1176,9 +1176,10 @@ def main():
         names = []
         for k in (0, 1):
             if schedule == "per_class":
-                names.append("nf_regular_kernel<%d, 1, 1, 2, 0>" % k)
-                names += ["nf_singular_kernel<%d, 1, 1, %d, 4, false>" %
-                          (k, c) for c in (1, 2, 3)]
+                names.append("nf_pair_kernel<%d, 1, 2, 0>" % k)
+                names += ["nf_singular_kernel<%d, 1, 1, %d, 4, false, %s, "
+                          "true>" % (k, c, "false" if c == 2 else "true")
+                          for c in (1, 2, 3)]
             elif schedule == "fused":
                 names.append("nf_fused_kernel<%d, 1, 1, 2, 0>" % k)
             else:
@@ -1197,9 +1198,10 @@ def main():
         names = []
         for k in (0, 1):
             if schedule == "per_class":
-                names.append("nf_regular_kernel<%d, 1, 1, 2, 0>" % k)
-                names += ["nf_singular_kernel<%d, 1, 1, %d, 4, false>" %
-                          (k, c) for c in (1, 2, 3)]
+                names.append("nf_pair_kernel<%d, 1, 2, 0>" % k)
+                names += ["nf_singular_kernel<%d, 1, 1, %d, 4, false, %s, "
+                          "true>" % (k, c, "false" if c == 2 else "true")
+                          for c in (1, 2, 3)]
             elif schedule == "fused":
                 names.append("nf_fused_kernel<%d, 1, 1, 2, 0>" % k)
             else:

@@ -558,7 +558,8 @@ __device__ __forceinline__ void dot_row(const double *__restrict__ M,
 // Place of input j of vector v in a wave's LDS slice: one vector as (re, im)
 // pairs; several with the vectors of an input next to each other (real
 // matrices without imaginary parts), so that a wave's broadcast reads take
-// two values at a time.  Eight vectors, 32768 triangles: NVTIME.
+// two values at a time.  Eight vectors, 32768 triangles, with the pairs'
+// kernel for several vectors: stored 145 -> 132 us, adjoint 334 -> 178 us.
 template <int C, int NV>
 __device__ __forceinline__ uint32_t lx(uint32_t v, uint32_t j) {
   return NV == 1 ? 2 * j : C ? 2 * (j * NV + v) : j * NV + v;

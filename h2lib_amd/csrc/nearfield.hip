@@ -17,6 +17,7 @@
 #include <thread>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <numeric>
 #include <unordered_map>
 
@@ -771,8 +772,9 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
   a.are = op->layer != H2HIP_SLP ? op->alpha[0] : 0.0;
   a.aim = op->layer != H2HIP_SLP ? op->alpha[1] : 0.0;
   a.adj = op->layer == H2HIP_ADLP;
-  // given normals that are not perpendicular to the triangles: the general
-  // FP64 double layer kernels (no mirrored or fused tiles)
+  // given normals that are not perpendicular to the triangles, or a surface
+  // that folds back on itself: the FP64 double layer kernels with a product
+  // <d, n> per value (no mirrored or fused tiles)
   a.plane = s->plane;
   const bool general =
       op->layer != H2HIP_SLP && op->precision == 0 && !s->plane;
@@ -983,7 +985,12 @@ int copy_out(CbCtx &C, const uint64_t *off, const uint32_t *blocks,
   const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
   const unsigned nt = (unsigned)std::min<size_t>({ng, hw, bytes >> 23, 8});
   std::vector<std::thread> pool;
-  for (unsigned t = 1; t < nt; t++) pool.emplace_back(work);
+  try {
+    pool.reserve(nt);
+    for (unsigned t = 1; t < nt; t++) pool.emplace_back(work);
+  } catch (const std::exception &) {
+    // no more threads: those started and this one do all pieces
+  }
   work();
   for (auto &th : pool) th.join();
   H2HIP_CHECK(hipStreamSynchronize(C.st));
@@ -1049,6 +1056,28 @@ void give_context(const h2hip_op *op, CbCtx *c) {
     c->busy = false;
   }
   op->cb_cv.notify_one();
+}
+
+// Whether two triangles with a common vertex have opposite normals (to 18
+// degrees): the surface folds back on itself there, as the finer cylinder
+// meshes do.  Where the folded sheets overlap, <x - y, n> is zero up to the
+// rounding of the points, which 1/r^3 magnifies: forming it from anything
+// but the difference x - y moves such entries by up to 1e-9 of the largest
+// (cylinder, 46240 triangles; 8e-13 in the norm of all entries).
+bool folds(const h2hip_surface &s) {
+  for (uint32_t v = 0; v < s.nv; v++)
+    for (uint32_t p = s.v2t_ptr[v]; p < s.v2t_ptr[v + 1]; p++) {
+      const double *a = &s.n[3 * s.v2t[p]];
+      for (uint32_t q = p + 1; q < s.v2t_ptr[v + 1]; q++) {
+        const double *b = &s.n[3 * s.v2t[q]];
+        const double ab = a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
+        if (ab < 0.0 &&
+            ab * ab > 0.9 * (a[0] * a[0] + a[1] * a[1] + a[2] * a[2]) *
+                          (b[0] * b[0] + b[1] * b[1] + b[2] * b[2]))
+          return true;
+      }
+    }
+  return false;
 }
 
 }  // namespace
@@ -1155,6 +1184,7 @@ int h2hip_surface_create(h2hip_surface **out, uint32_t vertices,
       const uint32_t v = t[3 * i + l];
       s->v2t[s->v2t_ptr[v] + fill[v]++] = i;
     }
+  s->plane = s->plane && !folds(*s);
   int rc = H2HIP_OK;
   if (s->d_x.upload(s->x.data(), s->x.size()) != hipSuccess ||
       s->d_t.upload(s->t.data(), s->t.size()) != hipSuccess ||

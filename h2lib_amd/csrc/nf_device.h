@@ -253,7 +253,7 @@ __device__ __forceinline__ void kahan_add(float &s, float &c, float x) {
 // change sign).  S1[l][k] sums the kernel of one order: single layers the
 // kernel, double layers sg A or, wantB, sg B.  TWO: both orders at once, S1
 // with A and S2 with B, which share the difference, its length and the
-// phase.  FP64 and normals perpendicular to the triangles (a.plane): A does
+// phase.  FP64 and a.plane (normals perpendicular to the triangles): A does
 // not depend on b nor B on i, so A is a factor of the row point and B of the
 // column point and no value takes a product of vectors (double layer, linear
 // basis, 32768 triangles: 1011 -> 945 us).
@@ -261,7 +261,9 @@ __device__ __forceinline__ void kahan_add(float &s, float &c, float x) {
 // 2 mixed with FP32 accumulation throughout, the outer sums compensated
 // (Kahan); TWO is for MP 0 and single layers with MP 1 (S2 is not set: the
 // single layers are symmetric).
-template <int KER, int BR, int BC, int Q, int MP, bool TWO>
+// PL_: a.plane where the launch knows it (0, 1), -1 where it is looked up (a
+// kernel with both ways takes the registers of the larger, up to 220).
+template <int KER, int BR, int BC, int Q, int MP, bool TWO, int PL_>
 __device__ __forceinline__ void pair_sums(
     const KArgs &a, uint32_t tt, uint32_t ts, const double (&nt)[3],
     const double (&ns)[3], bool wantB, double sg,
@@ -376,6 +378,10 @@ __device__ __forceinline__ void pair_sums(
     }
     auto sums = [&](auto plane) {
       constexpr bool PL = DLP && decltype(plane)::value;
+      // (the Helmholtz double layer with argument reduction and a product per
+      // value: 127 VGPRs instead of 220; folded cylinder of 46240 triangles,
+      // constant basis, 2.33 -> 2.11 ms)
+      constexpr int UB = KER == K_HELM_DLP && !PL ? 1 : QQ;
       // the factors of the points and, without them, the normal of <d, n>
       double fi_[QQ], fb_[QQ], n1[3];
 #pragma unroll
@@ -396,7 +402,7 @@ __device__ __forceinline__ void pair_sums(
 #pragma unroll
         for (int d = 0; d < 3; d++) n1[d] = sg * (wantB ? -nt[d] : ns[d]);
       }
-#pragma unroll
+#pragma unroll UB
       for (int b = 0; b < QQ; b++) {
         const double qx = Ps[3 * b], qy = Ps[3 * b + 1], qz = Ps[3 * b + 2];
         double Ure[NR], Uim[NR], Vre[NR], Vim[NR];
@@ -464,7 +470,12 @@ __device__ __forceinline__ void pair_sums(
         }
       }
     };
-    if (!DLP || TWO || a.plane)  // uniform; TWO only with plane normals
+    // (TWO only with plane normals)
+    if constexpr (!DLP || TWO || PL_ == 1)
+      sums(std::true_type{});
+    else if constexpr (PL_ == 0)
+      sums(std::false_type{});
+    else if (a.plane)  // uniform
       sums(std::true_type{});
     else
       sums(std::false_type{});
@@ -506,8 +517,9 @@ constexpr bool paired(int ker, int rb, int cb, int mp) {
 // The same sums for the entry (row triangle rt, column triangle ct).  The
 // constant basis evaluates a pair of triangles in one order, the smaller
 // number first, whichever of the two entries asks: both entries then have
-// the same bits in every schedule.
-template <int KER, int BR, int BC, int Q, int MP>
+// the same bits in every schedule (not PL = 0, whose tiles have no mirrors:
+// there a wave's lanes read the same column triangle, not each its own).
+template <int KER, int BR, int BC, int Q, int MP, int PL>
 __device__ __forceinline__ void entry_sums(
     const KArgs &a, uint32_t rt, uint32_t ct,
     double (&Sre)[BR ? 3 : 1][BC ? 3 : 1],
@@ -516,7 +528,7 @@ __device__ __forceinline__ void entry_sums(
   // The reference's lc far integrator maps the first rule coordinates onto
   // the column triangle (Library/bem3d.c:2637-2649); kept as is.
   const bool sw =
-      CC ? paired(KER, 0, 0, MP) && rt > ct : (BR && !BC) && a.far;
+      CC ? PL != 0 && paired(KER, 0, 0, MP) && rt > ct : (BR && !BC) && a.far;
   const uint32_t tt = sw ? ct : rt, ts = sw ? rt : ct;
   // n_y belongs to the column triangle, the adjoint's -n_x to the row
   // triangle; d changes sign with the order except in the lc far rule
@@ -529,7 +541,7 @@ __device__ __forceinline__ void entry_sums(
   }
   double dre[BR ? 3 : 1][BC ? 3 : 1], dim[BR ? 3 : 1][BC ? 3 : 1];
   // (only the normal of the one order is read)
-  pair_sums<KER, BR, BC, Q, MP, false>(a, tt, ts, nv, nv, wantB,
+  pair_sums<KER, BR, BC, Q, MP, false, PL>(a, tt, ts, nv, nv, wantB,
                                        !CC && sw ? -1.0 : 1.0, Sre, Sim, dre,
                                        dim);
 }
@@ -545,7 +557,8 @@ __device__ __forceinline__ void tile_singular(const KArgs &a, const Tile &T,
 // vertices (tlist + T.sbeg, T.ns[c] per class) before the tile is stored,
 // so they add into the LDS accumulator instead of the output (constant
 // basis: the regular pass leaves their entries to the singular pass).
-template <int KER, int BR, int BC, int Q, int MP, bool FUSED = false>
+template <int KER, int BR, int BC, int Q, int MP, bool FUSED = false,
+          int PL = -1>
 __device__ __forceinline__ void regular_tile(const KArgs &a, uint32_t tile,
                                              const SPair *tlist = nullptr,
                                              uint32_t slice = 0,
@@ -602,7 +615,7 @@ __device__ __forceinline__ void regular_tile(const KArgs &a, uint32_t tile,
     double f2 = 0.0;
     if (!shared) {
       f2 = pair_factor<CC>(a, sr.tri, sc.tri);
-      entry_sums<KER, BR, BC, Q, MP>(a, sr.tri, sc.tri, Sre, Sim);
+      entry_sums<KER, BR, BC, Q, MP, PL>(a, sr.tri, sc.tri, Sre, Sim);
     }
     if constexpr (CC) {
       // entry (r, c) of the tile; pairs with common vertices are stored as
@@ -668,10 +681,14 @@ __device__ __forceinline__ void regular_tile(const KArgs &a, uint32_t tile,
   }
 }
 
-template <int KER, int BR, int BC, int Q, int MP>
-__global__ __launch_bounds__(NTHREADS) void nf_regular_kernel(KArgs a) {
-  regular_tile<KER, BR, BC, Q, MP>(a, blockIdx.x / a.split, nullptr,
-                                   blockIdx.x % a.split, a.split);
+// (The Helmholtz double layer with argument reduction takes 220 VGPRs, two
+// waves per SIMD, where it is free to.)
+template <int KER, int BR, int BC, int Q, int MP, int PL>
+__global__ __launch_bounds__(NTHREADS,
+                             KER == K_HELM_DLP && Q == 2 && MP == 0 ? 3 : 1)
+void nf_regular_kernel(KArgs a) {
+  regular_tile<KER, BR, BC, Q, MP, false, PL>(a, blockIdx.x / a.split, nullptr,
+                                              blockIdx.x % a.split, a.split);
 }
 
 // Two mirrored tiles per workgroup: tile T = (rows R, columns C) and its
@@ -783,7 +800,7 @@ __global__ __launch_bounds__(pair_threads(KER, B),
           ns[d] = a.n[3 * ts + d];
         }
       }
-      pair_sums<KER, B, B, Q, MP, DLP>(a, tt, ts, nt, ns, false, 1.0, S1re,
+      pair_sums<KER, B, B, Q, MP, DLP, 1>(a, tt, ts, nt, ns, false, 1.0, S1re,
                                        S1im, S2re, S2im);
     } else {
 #pragma unroll
@@ -889,7 +906,7 @@ __global__ __launch_bounds__(NTHREADS) void nf_regular_persistent(
 template <int KER, int BR, int BC, int Q, int MP>
 __global__ __launch_bounds__(NTHREADS) void nf_fused_kernel(
     KArgs a, const SPair *__restrict__ tlist) {
-  regular_tile<KER, BR, BC, Q, MP, true>(a, blockIdx.x, tlist);
+  regular_tile<KER, BR, BC, Q, MP, true, 1>(a, blockIdx.x, tlist);
 }
 
 template <int KER, int BR, int BC, int Q, int MP>
@@ -903,7 +920,7 @@ __global__ __launch_bounds__(NTHREADS) void nf_fused_persistent(
     const uint32_t t = cur;
     __syncthreads();
     if (t >= ntiles) break;
-    regular_tile<KER, BR, BC, Q, MP, true>(a, t, tlist);
+    regular_tile<KER, BR, BC, Q, MP, true, 1>(a, t, tlist);
   }
 }
 
@@ -1002,8 +1019,11 @@ __device__ __forceinline__ V sel3(const V (&v)[3], int i) {
 // other when the triangles are exchanged, so the exchanged pair has the
 // same points and the same moments, of the kernel with the other normal
 // (single layer: the same values).  The edge rule has no such symmetry.
+//
+// PL: the normals are perpendicular to the triangles and no triangles fold
+// back on each other (a.plane), so <d, n> may be formed from them.
 template <int KER, int BR, int BC, int CLS, int Q2, bool MP, bool MIR,
-          class Sink>
+          bool PL, class Sink>
 __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
                                               const SPair &P, int sub,
                                               Sink &&sink) {
@@ -1136,13 +1156,12 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
     }
   };
 
-  // The rules of order 4 take the normals as perpendicular to the triangles
-  // (the launches see to it): the double layers vanish on identical
+  // PL, the rules of order 4: the double layers vanish on identical
   // triangles, whose differences lie in their plane, and on a common edge
   // <d, n> is one coordinate of the other triangle's point times a constant.
   // (Vertex pairs keep the products: the same there takes more registers,
   // 222 -> 254 us for the double layer at 32768 triangles.)
-  constexpr bool PLANE = DLP && !MP && Q2 > 0;
+  constexpr bool PLANE = DLP && !MP && Q2 > 0 && PL;
   auto dot = [](const double (&u)[3], const double (&v)[3]) {
     return fma(u[0], v[0], fma(u[1], v[1], u[2] * v[2]));
   };
@@ -1594,7 +1613,8 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
 // (the regular kernel has stored the tiles before).
 // MIR: the list holds one of each two exchanged pairs; the other's entry is
 // added into the mirror tile.
-template <int KER, int BR, int BC, int CLS, int Q2, bool MP, bool MIR>
+template <int KER, int BR, int BC, int CLS, int Q2, bool MP, bool MIR,
+          bool PL>
 __device__ __forceinline__ void singular_list(const KArgs &a,
                                               const SPair *__restrict__ list,
                                               uint32_t npairs,
@@ -1609,7 +1629,7 @@ __device__ __forceinline__ void singular_list(const KArgs &a,
   // identical triangles of a diagonal tile have no exchanged pair
   const bool mir =
       MIR && !(CLS == CLS_IDENTICAL && T.mirror == P.tile);
-  singular_pair<KER, BR, BC, CLS, Q2, MP, MIR>(
+  singular_pair<KER, BR, BC, CLS, Q2, MP, MIR, PL>(
       a, T, P, sub,
       [&](uint32_t lr, uint32_t lc, double vre, double vim, double vre2,
           double vim2) {
@@ -1635,10 +1655,12 @@ __device__ __forceinline__ void singular_list(const KArgs &a,
       });
 }
 
-template <int KER, int BR, int BC, int CLS, int Q2, bool MP, bool MIR>
+template <int KER, int BR, int BC, int CLS, int Q2, bool MP, bool MIR,
+          bool PL>
 __global__ __launch_bounds__(NTHREADS) void nf_singular_kernel(
     KArgs a, const SPair *__restrict__ list, uint32_t npairs) {
-  singular_list<KER, BR, BC, CLS, Q2, MP, MIR>(a, list, npairs, blockIdx.x);
+  singular_list<KER, BR, BC, CLS, Q2, MP, MIR, PL>(a, list, npairs,
+                                                   blockIdx.x);
 }
 
 // The three classes (order 4) in one launch: identical pairs in the first
@@ -1648,19 +1670,20 @@ __global__ __launch_bounds__(NTHREADS) void nf_singular_kernel(
 // us, its launches 33 -> 20; 2048 triangles, constant basis: 25 -> 16 us;
 // 2028 triangles, linear, 30000 pairs: 40 -> 35 us); the registers are
 // those of the largest class, so long lists keep a launch per class.
-template <int KER, int BR, int BC, bool MP, bool MIR>
+template <int KER, int BR, int BC, bool MP, bool MIR, bool PL>
 __global__ __launch_bounds__(NTHREADS) void nf_singular_all(
     KArgs a, const SPair *__restrict__ l3, uint32_t n3,
     const SPair *__restrict__ l2, uint32_t n2, const SPair *__restrict__ l1,
     uint32_t n1, uint32_t b3, uint32_t b2) {
   const uint32_t b = blockIdx.x;
   if (b < b3)
-    singular_list<KER, BR, BC, CLS_IDENTICAL, 4, MP, MIR && BR != 0>(a, l3, n3,
-                                                                    b);
+    singular_list<KER, BR, BC, CLS_IDENTICAL, 4, MP, MIR && BR != 0, PL>(
+        a, l3, n3, b);
   else if (b < b3 + b2)
-    singular_list<KER, BR, BC, CLS_EDGE, 4, MP, false>(a, l2, n2, b - b3);
+    singular_list<KER, BR, BC, CLS_EDGE, 4, MP, false, PL>(a, l2, n2, b - b3);
   else
-    singular_list<KER, BR, BC, CLS_VERTEX, 4, MP, MIR>(a, l1, n1, b - b3 - b2);
+    singular_list<KER, BR, BC, CLS_VERTEX, 4, MP, MIR, PL>(a, l1, n1,
+                                                           b - b3 - b2);
 }
 
 // The pairs with common vertices of one tile and one rule class, by the
@@ -1679,7 +1702,7 @@ __device__ __forceinline__ void tile_singular(const KArgs &a, const Tile &T,
   for (uint32_t p0 = 0; p0 < n; p0 += NTHREADS / 16) {
     const uint32_t w = p0 + row;
     if (w >= n) continue;  // uniform per row of 16 lanes
-    singular_pair<KER, BR, BC, CLS, Q2, MP, false>(
+    singular_pair<KER, BR, BC, CLS, Q2, MP, false, true>(
         a, T, list[w], sub,
         [&](uint32_t lr, uint32_t lc, double vre, double vim, double,
             double) {
@@ -1743,23 +1766,24 @@ int launch_bases_p(uint32_t q, const KArgs &a, uint32_t ntiles,
                  n1 = ncls[CLS_VERTEX];
   // order 4, all classes: one launch while every pair has its lanes at once
   // (SING_ALL), else one per class
-  auto singular4 = [&](auto mir, uint32_t c3, uint32_t c1) {
+  auto singular4 = [&](auto mir, auto plane, uint32_t c3, uint32_t c1) {
     constexpr bool MIR = decltype(mir)::value;
+    constexpr bool PL = decltype(plane)::value;
     if (c3 + n2 + c1 <= SING_ALL) {
       auto nb = [](uint32_t n) { return (n + PPB - 1) / PPB; };
       if (c3 + n2 + c1)
-        hipLaunchKernelGGL((nf_singular_all<KER, BR, BC, SMP, MIR>),
+        hipLaunchKernelGGL((nf_singular_all<KER, BR, BC, SMP, MIR, PL>),
                            dim3(nb(c3) + nb(n2) + nb(c1)), dim3(NTHREADS), 0,
                            stream, a, sp, c3, sp + n3, n2, sp + n3 + n2, c1,
                            nb(c3), nb(n2));
       return;
     }
     singular(nf_singular_kernel<KER, BR, BC, CLS_IDENTICAL, 4, SMP,
-                                MIR && BR != 0>,
+                                MIR && BR != 0, PL>,
              sp, c3);
-    singular(nf_singular_kernel<KER, BR, BC, CLS_EDGE, 4, SMP, false>,
+    singular(nf_singular_kernel<KER, BR, BC, CLS_EDGE, 4, SMP, false, PL>,
              sp + n3, n2);
-    singular(nf_singular_kernel<KER, BR, BC, CLS_VERTEX, 4, SMP, MIR>,
+    singular(nf_singular_kernel<KER, BR, BC, CLS_VERTEX, 4, SMP, MIR, PL>,
              sp + n3 + n2, c1);
   };
   if ((BR || BC) && a.split > 1) {
@@ -1779,10 +1803,11 @@ int launch_bases_p(uint32_t q, const KArgs &a, uint32_t ntiles,
                            dim3(pair_threads(KER, BR)), 0, stream, a,
                            a.mirlist);
       else
-        hipLaunchKernelGGL((nf_regular_kernel<KER, BR, BC, 2, MP>),
+        hipLaunchKernelGGL((nf_regular_kernel<KER, BR, BC, 2, MP, 1>),
                            dim3(ntiles * a.split), dim3(NTHREADS), 0, stream,
                            a);
-      singular4(std::true_type{}, BR ? a.nmain3 : n3, a.nmain1);
+      singular4(std::true_type{}, std::true_type{}, BR ? a.nmain3 : n3,
+                a.nmain1);
       return H2HIP_OK;
     }
   }
@@ -1810,25 +1835,33 @@ int launch_bases_p(uint32_t q, const KArgs &a, uint32_t ntiles,
   } else if (ntiles) {
     void (*reg)(KArgs) = nullptr;
     switch (q) {
-      case 1: reg = nf_regular_kernel<KER, BR, BC, 1, MP>; break;
-      case 2: reg = nf_regular_kernel<KER, BR, BC, 2, MP>; break;
-      case 3: reg = nf_regular_kernel<KER, BR, BC, 3, MP>; break;
-      case 4: reg = nf_regular_kernel<KER, BR, BC, 4, MP>; break;
+      case 1: reg = nf_regular_kernel<KER, BR, BC, 1, MP, -1>; break;
+      case 2: reg = nf_regular_kernel<KER, BR, BC, 2, MP, 1>; break;
+      case 3: reg = nf_regular_kernel<KER, BR, BC, 3, MP, -1>; break;
+      case 4: reg = nf_regular_kernel<KER, BR, BC, 4, MP, -1>; break;
       default: return H2HIP_EINVAL;
     }
+    if constexpr (MP == 0 && is_dlp(KER))
+      if (q == 2 && !a.plane) reg = nf_regular_kernel<KER, BR, BC, 2, MP, 0>;
     hipLaunchKernelGGL(reg, dim3(ntiles * a.split), dim3(NTHREADS), 0, stream,
                        a);
   }
   if (a.far) return H2HIP_OK;
-  if (a.q2 == 4 && (a.plane || MP || !is_dlp(KER))) {
-    singular4(std::false_type{}, n3, n1);
+  if (a.q2 == 4) {
+    if constexpr (MP == 0 && is_dlp(KER)) {
+      if (!a.plane) {
+        singular4(std::false_type{}, std::false_type{}, n3, n1);
+        return H2HIP_OK;
+      }
+    }
+    singular4(std::false_type{}, std::true_type{}, n3, n1);
     return H2HIP_OK;
   }
-  singular(nf_singular_kernel<KER, BR, BC, CLS_IDENTICAL, 0, SMP, false>, sp,
+  singular(nf_singular_kernel<KER, BR, BC, CLS_IDENTICAL, 0, SMP, false, true>, sp,
            n3);
-  singular(nf_singular_kernel<KER, BR, BC, CLS_EDGE, 0, SMP, false>, sp + n3,
+  singular(nf_singular_kernel<KER, BR, BC, CLS_EDGE, 0, SMP, false, true>, sp + n3,
            n2);
-  singular(nf_singular_kernel<KER, BR, BC, CLS_VERTEX, 0, SMP, false>,
+  singular(nf_singular_kernel<KER, BR, BC, CLS_VERTEX, 0, SMP, false, true>,
            sp + n3 + n2, n1);
   return H2HIP_OK;
 }

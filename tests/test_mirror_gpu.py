@@ -128,3 +128,52 @@ def test_given_normals_that_are_not_perpendicular(kern, k, layer, basis,
         # (cancellation in the rolled entries: their scale bounds the error)
         scale = max(np.abs(b).max(), np.abs(a).max())
         assert np.abs(c - (a + 0.1 * b)).max() < 1e-13 * scale
+
+
+@pytest.mark.parametrize("kern,k", [(0, 0.0), (1, 2.0)])
+@pytest.mark.parametrize("layer", [1, 2])
+@pytest.mark.parametrize("basis", [0, 1])
+@pytest.mark.parametrize("perm", [(0, 2, 1), (2, 1, 0), (1, 0, 2)])
+def test_folded_sheets_take_differences(kern, k, layer, basis, perm):
+    """Two coplanar sheets folded at an edge, 1e-6 apart within their plane:
+    quadrature points nearly coincide (for one of the orders of the vertices)
+    and the double layers are rounding noise.  Formed from x - y, <x - y, n>
+    stays linear in n to the rounding of one product of vectors, a few 1e-16
+    of the values with normals in the plane; from a triangle's plane it is
+    off by 1e-16 h / r of them, 1e-10."""
+    import h2lib_amd as h
+    m = 6
+    q, _ = np.linalg.qr(np.random.default_rng(2).normal(size=(3, 3)))
+    grid = np.array([(i / m, j / m, 0.0) for i in range(m + 1)
+                     for j in range(m + 1)])
+    x = np.concatenate([grid, grid + [0.0, 1e-6, 0.0]]) @ q.T
+    nv = len(grid)
+    t = []
+    for i in range(m):
+        for j in range(m):
+            a = i * (m + 1) + j
+            b, c, d = a + m + 1, a + m + 2, a + 1
+            t += [(a, b, c), (a, c, d)]
+    # the second sheet's vertices on the fold i = m are the first's
+    back = np.where(np.arange(nv) >= m * (m + 1), np.arange(nv),
+                    np.arange(nv) + nv)
+    t = np.array(t, dtype=np.uint32)
+    t = np.concatenate([t, back[t][:, perm]]).astype(np.uint32)
+    used = np.unique(t)
+    t = np.searchsorted(used, t).astype(np.uint32)
+    x = np.ascontiguousarray(x[used])
+    plain = h.Surface3d(x, t)
+    assert np.allclose(plain.n[0], -plain.n[len(t) // 2])
+    roll = np.roll(plain.n, 1, axis=1)
+    dofs = plain.vertices if basis else plain.triangles
+    idx = np.random.default_rng(8).permutation(dofs).astype(np.uint32)
+    blocks = mirrored_blocks((64, 13))
+    vals = []
+    for nn in (plain.n, roll, plain.n + 0.1 * roll):
+        gr = h.Surface3d(x, t, nn, plain.g)
+        op = h.Bem3d(gr, kern, layer, 2, 4, basis, basis, alpha=0.0, k=k)
+        plan = h.NearfieldPlan(gr, basis, basis, idx, idx, blocks)
+        vals.append([run(h, plan, op, s) for s in ((0, 0, 0), (0, 1, 0),
+                                                   (0, 0, 1))])
+    for a, b, c in zip(*vals):
+        assert np.abs(c - (a + 0.1 * b)).max() < 1e-13 * np.abs(b).max()
