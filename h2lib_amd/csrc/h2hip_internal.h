@@ -301,10 +301,13 @@ struct h2hip_nfplan {
   h2hip::SPair *d_spairs = nullptr;
   uint32_t *d_mirlist = nullptr;
   // schedule: tiles in decreasing order of their pair count, and the
-  // persistent regular kernel with its tile counter
+  // persistent regular kernel with its tile counter.  The sorted order has
+  // device lists of its own, made when it is first set and kept: kernels of
+  // earlier executions may still read the plan's own lists on streams that
+  // nothing here waits for.
   int sorted = 0, persistent = 0;
-  std::vector<h2hip::Tile> tiles0;    // plan order, kept once sorted
-  std::vector<h2hip::SPair> spairs0;
+  h2hip::DevBuf<h2hip::Tile> d_tiles_s;
+  h2hip::DevBuf<h2hip::SPair> d_spairs_s;
   h2hip::DevBuf<uint32_t> d_counter;
   // fused schedule: tiles by decreasing total work (regular and singular
   // evaluations) and the singular pairs grouped by tile

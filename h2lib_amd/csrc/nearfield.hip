@@ -348,8 +348,11 @@ int build_plan(h2hip_nfplan *P, const h2hip_surface *s, int rb, int cb,
   P->supp.clear();
   P->fix.clear();
   P->spairs.clear();
-  // a fused schedule is set again for the new plan
+  // a schedule is set again for the new plan
+  P->sorted = 0;
   P->fused = 0;
+  P->d_tiles_s.release();
+  P->d_spairs_s.release();
   P->d_tiles_f.release();
   P->d_tpairs.release();
   for (auto &c : P->pairs) c = 0;
@@ -751,7 +754,8 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
   if (P->tiles.empty()) return H2HIP_OK;
   const h2hip_surface *s = op->s;
   nf::KArgs a;
-  a.tiles = P->d_tiles;
+  a.tiles = P->sorted ? P->d_tiles_s.p : P->d_tiles;
+  const SPair *const spairs = P->sorted ? P->d_spairs_s.p : P->d_spairs;
   a.supp = P->d_supp;
   a.x = s->d_x.p;
   a.n = s->d_n.p;
@@ -833,10 +837,9 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
                        : small ? nf::launch_helmholtz_dlp_sp
                                : nf::launch_helmholtz_dlp);
   const int rc =
-      launch ? launch(op->rb, op->cb, op->q, a, ntiles, P->d_spairs, ncls,
-                      stream)
+      launch ? launch(op->rb, op->cb, op->q, a, ntiles, spairs, ncls, stream)
              : nf::launch_laplace(op->layer, op->rb, op->cb, op->q, a, ntiles,
-                                  P->d_spairs, ncls, stream);
+                                  spairs, ncls, stream);
   if (rc != H2HIP_OK) {
     set_error("unsupported regular quadrature order (1..4 supported)");
     return rc;
@@ -1475,10 +1478,7 @@ int h2hip_nfplan_set_tile(h2hip_nfplan *p, uint32_t tile) {
                      (uint32_t)p->in_cidx.size(), p->nblocks,
                      p->in_blocks.data(), 0);
   }
-  // the new tiles are in plan order: the schedule is applied again
-  p->sorted = 0;
-  p->tiles0.clear();
-  p->spairs0.clear();
+  // the schedule is applied again
   int rc2 = h2hip_nfplan_set_schedule(p, sorted, persistent);
   if (rc2 == H2HIP_OK) rc2 = h2hip_nfplan_set_fused(p, fused);
   return rc != H2HIP_OK ? rc : rc2;
@@ -1503,40 +1503,29 @@ int h2hip_nfplan_set_schedule(h2hip_nfplan *p, int sorted, int persistent) {
   }
   if (persistent && !p->d_counter.p)
     H2HIP_CHECK(p->d_counter.alloc(1));
-  p->persistent = persistent;
-  if (sorted == p->sorted) return H2HIP_OK;
-  if (sorted) {
+  if (sorted && !p->d_tiles_s.p && !p->tiles.empty()) {
     // tiles by decreasing number of support pairs (the regular work), the
     // singular pairs renumbered to follow their tiles
-    p->tiles0 = p->tiles;
-    p->spairs0 = p->spairs;
     const size_t nt = p->tiles.size();
     std::vector<uint32_t> perm(nt), pos(nt);
     for (size_t i = 0; i < nt; i++) perm[i] = (uint32_t)i;
     std::stable_sort(perm.begin(), perm.end(), [&](uint32_t x, uint32_t y) {
-      const uint64_t cx = (uint64_t)p->tiles0[x].nrsup * p->tiles0[x].ncsup;
-      const uint64_t cy = (uint64_t)p->tiles0[y].nrsup * p->tiles0[y].ncsup;
+      const uint64_t cx = (uint64_t)p->tiles[x].nrsup * p->tiles[x].ncsup;
+      const uint64_t cy = (uint64_t)p->tiles[y].nrsup * p->tiles[y].ncsup;
       return cx > cy;
     });
+    std::vector<Tile> tiles(nt);
     for (size_t i = 0; i < nt; i++) {
-      p->tiles[i] = p->tiles0[perm[i]];
+      tiles[i] = p->tiles[perm[i]];
+      tiles[i].mirror = NO_MIRROR;  // (mirrors belong to the plan's order)
       pos[perm[i]] = (uint32_t)i;
     }
-    for (auto &T : p->tiles)
-      if (T.mirror != NO_MIRROR) T.mirror = pos[T.mirror];
-    for (auto &sp : p->spairs) sp.tile = pos[sp.tile];
-  } else {
-    p->tiles = p->tiles0;
-    p->spairs = p->spairs0;
+    std::vector<SPair> spairs = p->spairs;
+    for (auto &sp : spairs) sp.tile = pos[sp.tile];
+    H2HIP_CHECK(p->d_spairs_s.upload(spairs.data(), spairs.size()));
+    H2HIP_CHECK(p->d_tiles_s.upload(tiles.data(), tiles.size()));
   }
-  if (!p->tiles.empty())
-    H2HIP_CHECK(hipMemcpy(p->d_tiles, p->tiles.data(),
-                          sizeof(Tile) * p->tiles.size(),
-                          hipMemcpyHostToDevice));
-  if (!p->spairs.empty())
-    H2HIP_CHECK(hipMemcpy(p->d_spairs, p->spairs.data(),
-                          sizeof(SPair) * p->spairs.size(),
-                          hipMemcpyHostToDevice));
+  p->persistent = persistent;
   p->sorted = sorted;
   return H2HIP_OK;
 }

@@ -176,8 +176,9 @@ int h2hip_nfplan_offsets(const h2hip_nfplan *p, uint64_t *off);
  * entries are the same bit for bit).  sorted = 1 orders the tiles
  * by decreasing regular work (longest first); persistent = 1 runs the
  * regular kernel as a persistent grid of resident workgroups that take
- * tiles from a device counter.  Not thread-safe against concurrent
- * executions of the same plan. */
+ * tiles from a device counter.  Executions queued before the call keep the
+ * schedule they were queued with (each order has device lists of its own).
+ * Not thread-safe against concurrent executions of the same plan. */
 int h2hip_nfplan_set_schedule(h2hip_nfplan *p, int sorted, int persistent);
 /* Fused tiles (no counterpart in the reference): fused = 1 evaluates each
  * tile's pairs with common vertices in the tile's own workgroup, added into

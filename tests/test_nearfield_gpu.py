@@ -262,6 +262,38 @@ def test_schedules_give_identical_entries(sorted_tiles, persistent, fused,
                 assert err < 1e-14, (name, mode, err)
 
 
+def test_schedule_set_while_executions_are_queued():
+    # a schedule set without waiting for the stream does not reach the
+    # executions queued before it: they and the later ones give the entries
+    # of the plan's order (constant basis: the same bits)
+    import h2lib_amd as h
+    from h2lib_amd import geometry as G
+    mesh = G.sphere(32)
+    gr = h.Surface3d(mesh.x, mesh.t, mesh.n, mesh.g)
+    op = h.Bem3d(gr, 0, 1, 2, 4, 0, 0, alpha=0.5)
+    rt = G.ClusterTree(mesh, 0, 40)
+    bt = G.BlockTree(rt, rt, 2.0, 0)
+    # one block without its mirror, so that no schedule pairs tiles
+    plan = h.NearfieldPlan(gr, 0, 0, rt.idx, rt.idx,
+                           bt.near_block_list()[:-1])
+    stream = h.Stream()
+    outs = [h.DeviceArray(plan.entries, op.dtype) for _ in range(7)]
+    for out in outs:
+        out.fill_nan()
+    plan.execute(op, outs[0].ptr, stream.handle)
+    stream.sync()
+    want = outs[0].download()
+    for _ in range(20):  # the device is busy when the first change comes
+        plan.execute(op, outs[0].ptr, stream.handle)
+    for out, schedule in zip(outs[1:], [(1, 0), (0, 0), (1, 1), (0, 1),
+                                        (1, 0), (0, 0)]):
+        plan.set_schedule(*schedule)
+        plan.execute(op, out.ptr, stream.handle)
+    stream.sync()
+    for out in outs[1:]:
+        assert np.array_equal(out.download(), want)
+
+
 @pytest.mark.parametrize("tile", [32, 24, 8])
 def test_tile_edges_give_identical_entries(tile, sphere8):
     # a plan cut into smaller tiles gives the entries of the 64-DOF tiles
