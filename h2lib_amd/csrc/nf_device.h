@@ -517,8 +517,9 @@ constexpr bool paired(int ker, int rb, int cb, int mp) {
 // The same sums for the entry (row triangle rt, column triangle ct).  The
 // constant basis evaluates a pair of triangles in one order, the smaller
 // number first, whichever of the two entries asks: both entries then have
-// the same bits in every schedule (not PL = 0, whose tiles have no mirrors:
-// there a wave's lanes read the same column triangle, not each its own).
+// the same bits in every schedule.  Not the FP64 double layers without
+// a.plane, whose tiles have no mirrors, in any schedule: there a wave's lanes
+// read the same column triangle, not each its own.
 template <int KER, int BR, int BC, int Q, int MP, int PL>
 __device__ __forceinline__ void entry_sums(
     const KArgs &a, uint32_t rt, uint32_t ct,
@@ -527,8 +528,10 @@ __device__ __forceinline__ void entry_sums(
   constexpr bool CC = (BR == 0) && (BC == 0);
   // The reference's lc far integrator maps the first rule coordinates onto
   // the column triangle (Library/bem3d.c:2637-2649); kept as is.
-  const bool sw =
-      CC ? PL != 0 && paired(KER, 0, 0, MP) && rt > ct : (BR && !BC) && a.far;
+  const bool plane =
+      PL == 1 || (PL == -1 && (!is_dlp(KER) || a.plane));  // uniform
+  const bool sw = CC ? plane && paired(KER, 0, 0, MP) && rt > ct
+                     : (BR && !BC) && a.far;
   const uint32_t tt = sw ? ct : rt, ts = sw ? rt : ct;
   // n_y belongs to the column triangle, the adjoint's -n_x to the row
   // triangle; d changes sign with the order except in the lc far rule

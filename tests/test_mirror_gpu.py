@@ -177,3 +177,30 @@ def test_folded_sheets_take_differences(kern, k, layer, basis, perm):
                                                    (0, 0, 1))])
     for a, b, c in zip(*vals):
         assert np.abs(c - (a + 0.1 * b)).max() < 1e-13 * np.abs(b).max()
+
+
+@pytest.mark.parametrize("kern,k", [(0, 0.0), (1, 0.05), (1, 6.0),
+                                    (1, 2.0 + 0.5j)])
+@pytest.mark.parametrize("layer", [1, 2])
+@pytest.mark.parametrize("surface", ["folded", "tilted"])
+def test_constant_basis_bits_in_every_schedule(kern, k, layer, surface,
+                                               sphere8):
+    """Surfaces whose double layers take <x - y, n> per value: the entries of
+    the constant basis have the same bits in every schedule there too."""
+    import h2lib_amd as h
+    from h2lib_amd import geometry as G
+    if surface == "folded":
+        mesh = G.cylinder(10)
+        gr = h.Surface3d(mesh.x, mesh.t, mesh.n, mesh.g)
+    else:
+        plain = h.Surface3d(sphere8["x"], sphere8["t"])
+        gr = h.Surface3d(sphere8["x"], sphere8["t"],
+                         plain.n + 0.1 * np.roll(plain.n, 1, axis=1),
+                         plain.g)
+    idx = np.random.default_rng(5).permutation(gr.triangles).astype(np.uint32)
+    blocks = mirrored_blocks((64, 63, 130))
+    plan = h.NearfieldPlan(gr, 0, 0, idx, idx, blocks)
+    op = h.Bem3d(gr, kern, layer, 2, 4, 0, 0, alpha=0.5, k=k)
+    want = run(h, plan, op, (0, 0, 0))
+    for schedule in ((1, 0, 0), (0, 1, 0), (1, 1, 0), (0, 0, 1), (0, 1, 1)):
+        assert np.array_equal(run(h, plan, op, schedule), want), schedule
