@@ -555,14 +555,19 @@ __device__ __forceinline__ void dot_row(const double *__restrict__ M,
   }
 }
 
-// Place of input j of vector v in a wave's LDS slice: one vector as (re, im)
-// pairs; several with the vectors of an input next to each other (real
-// matrices without imaginary parts), so that a wave's broadcast reads take
-// two values at a time.  Eight vectors, 32768 triangles, with the pairs'
-// kernel for several vectors: stored 145 -> 132 us, adjoint 334 -> 178 us.
-template <int C, int NV>
+// Place of input j of vector v in a wave's LDS slice: (re, im) pairs, vector
+// after vector; several vectors of a real matrix that is read (not MF) with
+// the vectors of an input next to each other and without imaginary parts, so
+// that a wave's broadcast reads take two values at a time.  Eight vectors,
+// 32768 triangles, with the pairs' kernel for several vectors: stored 145 ->
+// 132 us, adjoint 334 -> 178 us.  (Complex values are read in pairs anyway,
+// and the vectors next to each other put a wave's writes into one bank: eight
+// vectors, 20000 triangles, read couplings, 387 us so against 360; computed
+// values hide the reads: order 3, four vectors, 85 us so against 80.)
+template <int C, int NV, bool MF = false>
 __device__ __forceinline__ uint32_t lx(uint32_t v, uint32_t j) {
-  return NV == 1 ? 2 * j : C ? 2 * (j * NV + v) : j * NV + v;
+  constexpr uint32_t XR = 64;  // inputs per vector where NV > 1
+  return NV == 1 ? 2 * j : C || MF ? 2 * (v * XR + j) : j * NV + v;
 }
 
 // ar/ai[v] += sum_j M[base + j sj] x_v[j] over n columns for NV vectors in
@@ -570,7 +575,7 @@ __device__ __forceinline__ uint32_t lx(uint32_t v, uint32_t j) {
 // loads): B columns' entries are loaded together, the last batch with its
 // indices past n repeating the last column, before their products, which
 // run in column order.
-template <int C, int NV, int XR, bool NTL, bool CONJ>
+template <int C, int NV, int XR, bool NTL, bool CONJ, bool MF = false>
 __device__ __forceinline__ void dot_cols_nv(const double *__restrict__ M,
                                             uint64_t base, uint64_t sj,
                                             uint32_t n, const double *xs,
@@ -595,8 +600,8 @@ __device__ __forceinline__ void dot_cols_nv(const double *__restrict__ M,
         const double sr = mr[u], si = CONJ ? -mi[u] : mi[u];
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-          const double xr = xs[lx<C, NV>(v, j)];
-          const double xi = xs[lx<C, NV>(v, j) + 1];
+          const double xr = xs[lx<C, NV, MF>(v, j)];
+          const double xi = xs[lx<C, NV, MF>(v, j) + 1];
           ar[v] = fma(sr, xr, ar[v]);
           if constexpr (C) {
             ar[v] = fma(-si, xi, ar[v]);
@@ -681,8 +686,8 @@ __device__ __forceinline__ void mf_laplace4(const double *p3,
         const double sr = KCONST * cpl_rsqrt(fma(d2, d2, s1));
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-          ar[v] = fma(sr, xs[lx<C, NV>(v, j)], ar[v]);
-          if constexpr (C) ai[v] = fma(sr, xs[lx<C, NV>(v, j) + 1], ai[v]);
+          ar[v] = fma(sr, xs[lx<C, NV, true>(v, j)], ar[v]);
+          if constexpr (C) ai[v] = fma(sr, xs[lx<C, NV, true>(v, j) + 1], ai[v]);
         }
       }
     }
@@ -780,8 +785,8 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
       const uint32_t v = e / in.rank, j = e - v * in.rank;
       double xr = 0.0, xi = 0.0;
       if (v < a.v.nv) ld<C>(a.xt + v * a.cstride, in.coef + j, xr, xi);
-      xs[lx<C, NV>(v, j)] = xr;
-      if constexpr (C || NV == 1) xs[lx<C, NV>(v, j) + 1] = xi;
+      xs[lx<C, NV, MF>(v, j)] = xr;
+      if constexpr (C || NV == 1) xs[lx<C, NV, MF>(v, j) + 1] = xi;
     }
     // the wave reads what its own lanes wrote: LDS keeps the order of
     // one wave's accesses, the compiler must not move them
@@ -818,8 +823,8 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
               si = -si;
 #pragma unroll
               for (int v = 0; v < NV; v++) {
-                const double xr = xs[lx<C, NV>(v, j)];
-                const double xi = xs[lx<C, NV>(v, j) + 1];
+                const double xr = xs[lx<C, NV, MF>(v, j)];
+                const double xi = xs[lx<C, NV, MF>(v, j) + 1];
                 ar[v] = fma(sr, xr, ar[v]);
                 if constexpr (C) {
                   ar[v] = fma(-si, xi, ar[v]);
@@ -851,8 +856,8 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
                         a.cs.kdamp, sr, si);
 #pragma unroll
               for (int v = 0; v < NV; v++) {
-                const double xr = xs[lx<C, NV>(v, j)];
-                const double xi = xs[lx<C, NV>(v, j) + 1];
+                const double xr = xs[lx<C, NV, MF>(v, j)];
+                const double xi = xs[lx<C, NV, MF>(v, j) + 1];
                 ar[v] = fma(sr, xr, ar[v]);
                 if constexpr (C) {
                   ar[v] = fma(-si, xi, ar[v]);
@@ -866,7 +871,7 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
         dot_row<C, true>(a.S + (C ? 2 : 1) * (b.soff + i), r.rank, in.rank,
                          xs, ar[0], ai[0]);
       } else {
-        dot_cols_nv<C, NV, XR, true, TRANS>(
+        dot_cols_nv<C, NV, XR, true, TRANS, MF>(
             a.S, b.soff + (TRANS ? (uint64_t)i * r.rank : (uint64_t)i),
             TRANS ? 1 : r.rank, in.rank, xs, ar, ai);
       }
@@ -906,8 +911,8 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
     const uint32_t v = e / nin, j = e - v * nin;
     double xr = 0.0, xi = 0.0;
     if (v < a.v.nv) ld<C>(a.v.x[v], iidx[j], xr, xi);
-    xs[lx<C, NV>(v, j)] = xr;
-    if constexpr (C || NV == 1) xs[lx<C, NV>(v, j) + 1] = xi;
+    xs[lx<C, NV, MF>(v, j)] = xr;
+    if constexpr (C || NV == 1) xs[lx<C, NV, MF>(v, j) + 1] = xi;
   }
   __builtin_amdgcn_wave_barrier();
   for (uint32_t i = lane; i < nout; i += 64) {
@@ -922,7 +927,7 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
         dot_row<C>(a.N + (C ? 2 : 1) * (b.noff + i), b.rows, nin, xs, ar[0],
                    ai[0]);
     } else {
-      dot_cols_nv<C, NV, XR, false, TRANS>(
+      dot_cols_nv<C, NV, XR, false, TRANS, MF>(
           a.N, b.noff + (TRANS ? (uint64_t)i * b.rows : (uint64_t)i),
           TRANS ? 1 : b.rows, nin, xs, ar, ai);
     }
