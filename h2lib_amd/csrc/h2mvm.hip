@@ -2680,6 +2680,41 @@ int build_side(h2hip_h2matrix::Side &S, uint32_t nnodes, const uint32_t *tree,
   return H2HIP_OK;
 }
 
+// The number of mirrored pairs from which the pairs' kernels (couple_pairs64,
+// couple_pairs64_nv) are the faster way: below, one wave per pair leaves
+// SIMDs idle that the general kernels fill (a wave per block, a workgroup per
+// adjoint block with twg).  Not flat: the near blocks, which share the
+// launch of the general kernels, take one of their own beside the pairs'.
+// Measured at 98 to 8800 pairs (spheres of 968 to 32768 triangles, real: R,
+// complex: Z; us, general / pairs):
+//   flat, read: one vector 98 R 18 / 21, 662 R 23 / 23, 910 R 26 / 25,
+//     384 Z 24 / 28, 674 Z 34 / 32; several: 98 R 29 / 25 (two), 6 R 37 / 42
+//     (eight), 112 Z 44 / 47 and 244 Z 50 / 49 (four)
+//   flat, read, adjoint: 98 R 17 / 20 (one), 22 / 33 (four), 300 R 24 / 21
+//     (one), 27 / 28 (two); 244 Z 24 / 26 and 384 Z 32 / 28 (one), 384 Z 41 /
+//     44 and 674 Z 53 / 53 (two), 384 Z 96 / 99 (eight)
+//   flat, computed: one vector never slower; several 300 R 41 / 44 (eight),
+//     1109 R 38 / 40 (four), 1578 R 72 / 64 (eight); 112 Z 41 / 33 (two)
+//   not flat, read: 910 R 67 / 71, 1578 R 90 / 89, 3063 R 111 / 102, 2414 Z
+//     228 / 232 (four), 2950 Z 272 / 261; adjoint: as flat with twg
+//   not flat, computed: real 3063 91 / 92, 8816 121 / 121; 384 Z 100 / 104
+//     and 674 Z 128 / 128 (two), 8816 Z 537 / 548 (four); adjoint 98 R 58 /
+//     60 (four), 300 R 103 / 107 (eight)
+template <int C, int NV>
+uint32_t pairs_from(bool flat, bool trans, bool mf, bool twg) {
+  constexpr uint32_t NEVER = ~0u;
+  if (!flat && !trans) {
+    if (!mf) return 2048;
+    return !C || NV > 2 ? NEVER : NV == 2 ? 640 : 0;
+  }
+  if (mf) {
+    if (C || (NV == 1 && (flat || twg))) return 0;
+    return flat ? 1536 : !twg ? NEVER : 640;
+  }
+  if (trans) return C && (NV == 8 || (flat && NV == 2)) ? 640 : 256;
+  return NV == 1 ? 640 : C && NV == 4 ? 256 : 64;
+}
+
 template <int C, int K, int NV>
 void launch(const VecSet &vs, const h2hip_h2matrix *H, double *xt, double *yt,
             hipStream_t st, bool trans, bool symm = false) {
@@ -2704,25 +2739,28 @@ void launch(const VecSet &vs, const h2hip_h2matrix *H, double *xt, double *yt,
   const int cm = C ? 2 : 1;
   const bool mf = H->cpl_recompute && !symm;
   // order-4 interpolation couplings (read or computed) in mirrored pairs:
-  // each value once for a block and its mirror
-  // (several vectors keep the matrix cores where they are asked for; more
+  // each value once for a block and its mirror, where there are enough of
+  // them (several vectors keep the matrix cores where they are asked for; more
   // than four complex vectors with read couplings, forward, keep a wave per
   // block: 259 us against 279 for eight at 12800 triangles)
   const bool pairs64 = !symm && !ord && !tv && H->pairs_on && H->npair &&
                        H->cpl_known && H->cpl.m == 4 &&
+                       H->npair >= pairs_from<C, NV>(flat, trans, mf, twg) &&
                        (NV == 1 || C || mf || !H->cpl_mfma || trans) &&
                        !(C && NV > 4 && !mf && !trans);
   // the near blocks of a flat, not symmetric product run with the computed
   // complex pairs or in the upward launch (not the workgroup adjoint blocks
-  // of several vectors or fixed-order sums).  With the pairs where these are
+  // of several vectors, fixed-order sums or few real blocks: 196 far blocks
+  // 16.4 -> 16.9 us).  With the pairs where these are
   // at least eight rounds of the 768 resident workgroups: 131072 triangles
   // 758 -> 657 us; at 32768 (two and a half rounds) the last round's pairs
   // run alone, 190 -> 204 us.
   const bool pairs_near = C && NV == 1 && pairs64 && mf && flat && !trans &&
                           H->nnear > 0 && H->npair >= 8 * 768 * WPB;
   const bool fuse = flat && !symm && !pairs_near &&
-                    (!twg || (NV == 1 && !ord)) && H->nnear > 0 &&
-                    !in.items.empty();
+                    (!twg || (NV == 1 && !ord &&
+                              (pairs64 || C || H->nfar >= 512))) &&
+                    H->nnear > 0 && !in.items.empty();
   // view: the transposed blocks, whose rows are the column side's
   auto coupling_args = [&](bool view = false) {
     CNArgs c;

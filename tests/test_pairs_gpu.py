@@ -144,3 +144,54 @@ def test_large_helmholtz_product_runs_near_blocks_with_the_pairs():
         h.set_reproducible(True)
     for got in out[1:]:
         assert np.abs(got - out[0]).max() < 1e-13 * np.abs(out[0]).max()
+
+
+@pytest.mark.parametrize("schedule", [2, 0])
+@pytest.mark.parametrize("kern,layer,basis,k", [
+    (0, 0, 1, 0.0), (0, 1, 1, 0.0), (1, 0, 0, 3.0), (1, 1, 0, 2.0 + 0.5j)])
+def test_many_pairs_match_general_kernels(kern, layer, basis, k, schedule):
+    """Enough pairs for the pairs' kernels at every number of vectors, read
+    and computed, forward and adjoint (fewer keep the general kernels: the
+    tests above)."""
+    import h2lib_amd as h
+    from h2lib_amd import geometry as G
+    from h2lib_amd.h2matrix import H2Matrix
+    mesh = G.sphere(20)
+    gr = h.Surface3d(mesh.x, mesh.t, mesh.n, mesh.g)
+    op = h.Bem3d(gr, kern, layer, 2, 4, basis, basis,
+                 alpha=0.5 if layer else 0.0, k=k)
+    rt = G.ClusterTree(mesh, basis, 12)
+    bt = G.BlockTree(rt, rt, 2.0, 0)
+    H = H2Matrix(op, mesh, rt, rt, bt, 4)
+    H.set_schedule(schedule)
+    assert H.coupling_pairs() >= 2048
+    rng = np.random.default_rng(9)
+    d_x = [h.DeviceArray.from_host((rng.standard_normal(H.n) + (
+        1j * rng.standard_normal(H.n) if kern else 0.0)).astype(H.dtype))
+        for _ in range(8)]
+    d_y = [h.DeviceArray(H.n, H.dtype) for _ in range(8)]
+    alphas = [0.5 + 0.25 * v for v in range(8)]
+
+    def product(nv, trans):
+        for y in d_y[:nv]:
+            y.zero()
+        if nv == 1:
+            H.addeval(alphas[0], d_x[0], d_y[0], trans=trans)
+        else:
+            H.addeval_batch(alphas[:nv], d_x[:nv], d_y[:nv], trans=trans)
+        return np.array([y.download() for y in d_y[:nv]])
+
+    try:
+        for mode in (0, 1):
+            H.set_coupling_mode(mode)
+            for trans in (False, True):
+                h.set_reproducible(True)
+                want = product(8, trans)
+                h.set_reproducible(False)
+                for nv in (1, 2, 4, 8):
+                    for _ in range(2):
+                        err = np.abs(product(nv, trans) - want[:nv]).max(1)
+                        assert (err < 1e-13 * np.abs(want[:nv]).max(1)
+                                ).all(), (mode, trans, nv, err)
+    finally:
+        h.set_reproducible(True)
