@@ -770,8 +770,10 @@ __device__ __forceinline__ void near_adjoint64(const CNArgs &a,
 // xs: the wave's LDS slice of NV * 2 * XR doubles.  PF: near blocks of one
 // vector load their first columns before the input gather (more registers;
 // used where the launch holds only near blocks).
+// A64 (adjoint of one vector): near blocks of at most 64 x 64 by
+// near_adjoint64, whose registers the larger ones' loop would pay for too.
 template <int C, bool TRANS, int NV, bool MF = false, bool ORD = false,
-          bool PF = false>
+          bool PF = false, bool A64 = true>
 __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
                                                 double *xs) {
   constexpr int XR = NV == 1 ? MAXRANK : 64;  // inputs per LDS vector
@@ -889,7 +891,7 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
   const uint32_t nb = w - a.nfar;
   if (nb >= a.nnear) return;
   const NearD b = a.near[nb];
-  if constexpr (TRANS && NV == 1 && !ORD && !MF) {
+  if constexpr (TRANS && NV == 1 && !ORD && !MF && A64) {
     if (b.rows <= 64 && b.cols <= 64) {
       near_adjoint64<C>(a, b, lane);
       return;
@@ -1957,7 +1959,8 @@ __global__ __launch_bounds__(NT) void fwd_flat(FlatArgs a) {
 // after them, in one launch: the near blocks do not wait for the
 // coefficients, so they fill the device while the short upward items run.
 // TRANS: the adjoint product (near blocks N^*).
-template <int C, int K, int NV, bool ORD = false, bool TRANS = false>
+template <int C, int K, int NV, bool ORD = false, bool TRANS = false,
+          bool A64 = true>
 __global__ __launch_bounds__(NT) void fwd_flat_near(FlatArgs a, CNArgs c,
                                                     uint32_t fb) {
   constexpr int XS = NV * 2 * (NV == 1 ? MAXRANK : 64);
@@ -1966,7 +1969,7 @@ __global__ __launch_bounds__(NT) void fwd_flat_near(FlatArgs a, CNArgs c,
   if (blockIdx.x < fb)  // uniform over the block
     fwd_flat_dev<C, K, NV, ORD>(a, blockIdx.x, fb, xs);
   else
-    couple_near_dev<C, TRANS, NV, false, ORD, true>(
+    couple_near_dev<C, TRANS, NV, false, ORD, true, A64>(
         c, (blockIdx.x - fb) * WPB + (threadIdx.x >> 6), xs);
 }
 
@@ -2453,6 +2456,7 @@ struct h2hip_h2matrix {
   bool cpl_known = false;
   int cpl_recompute = 0;
   uint32_t maxleaf = 0, maxrank = 0;  // over both sides
+  uint32_t near64 = 0;  // near blocks of at most 64 x 64
   // schedule of the transforms: 0 one upward launch with counters (the
   // last son computes its father), 1 one upward launch per height above
   // the leaves and twigs, 2 flat transforms (products y += alpha H x of
@@ -2700,6 +2704,9 @@ int build_side(h2hip_h2matrix::Side &S, uint32_t nnodes, const uint32_t *tree,
 //   not flat, computed: real 3063 91 / 92, 8816 121 / 121; 384 Z 100 / 104
 //     and 674 Z 128 / 128 (two), 8816 Z 537 / 548 (four); adjoint 98 R 58 /
 //     60 (four), 300 R 103 / 107 (eight)
+//   leaves of more than 64 DOFs (not twg), adjoint: read 4608 triangles R 66
+//     / 46, not flat 91 / 80; computed, not flat, 4608 triangles Z 99 / 108,
+//     20000 triangles R 121 / 127, Z 305 / 296 and (leaves up to 128) 295 / 306
 template <int C, int NV>
 uint32_t pairs_from(bool flat, bool trans, bool mf, bool twg) {
   constexpr uint32_t NEVER = ~0u;
@@ -2708,10 +2715,12 @@ uint32_t pairs_from(bool flat, bool trans, bool mf, bool twg) {
     return !C || NV > 2 ? NEVER : NV == 2 ? 640 : 0;
   }
   if (mf) {
-    if (C || (NV == 1 && (flat || twg))) return 0;
-    return flat ? 1536 : !twg ? NEVER : 640;
+    if (!flat && !twg) return NEVER;
+    if (C || NV == 1) return 0;
+    return flat ? 1536 : 640;
   }
-  if (trans) return C && (NV == 8 || (flat && NV == 2)) ? 640 : 256;
+  if (trans)
+    return !twg ? 64 : C && (NV == 8 || (flat && NV == 2)) ? 640 : 256;
   return NV == 1 ? 640 : C && NV == 4 ? 256 : 64;
 }
 
@@ -2834,8 +2843,16 @@ void launch(const VecSet &vs, const h2hip_h2matrix *H, double *xt, double *yt,
                          0, st, fa, (const uint32_t *)in.d_it_ptr.p,
                          (const uint32_t *)in.d_it_ids.p, in.nnodes);
     } else if (fuse && ntrans) {
-      hipLaunchKernelGGL((fwd_flat_near<C, K, NV, false, true>), gf,
-                         dim3(NT), 0, st, fa, cn, fb);
+      // one vector, most blocks larger than 64 x 64: without near_adjoint64
+      // (20000 triangles, leaves of 78 DOFs, computed couplings: Laplace 84
+      // us with it, 77 without, Helmholtz 240 and 216)
+      constexpr bool A64 = NV > 1;
+      if (NV == 1 && H->near64 < H->nnear / 2)
+        hipLaunchKernelGGL((fwd_flat_near<C, K, NV, false, true, A64>), gf,
+                           dim3(NT), 0, st, fa, cn, fb);
+      else
+        hipLaunchKernelGGL((fwd_flat_near<C, K, NV, false, true>), gf,
+                           dim3(NT), 0, st, fa, cn, fb);
     } else if (fuse) {
       hipLaunchKernelGGL((fwd_flat_near<C, K, NV, false, false>), gf,
                          dim3(NT), 0, st, fa, cn, fb);
@@ -3477,6 +3494,7 @@ int h2hip_h2matrix_create(h2hip_h2matrix **out, int is_complex,
     const NodeD &r = H->side[0].nodes[near[2 * b]];
     const NodeD &c = H->side[1].nodes[near[2 * b + 1]];
     H->near.push_back(NearD{r.off, r.size, c.off, c.size, no});
+    H->near64 += r.size <= 64 && c.size <= 64;
     no += (uint64_t)r.size * c.size;
   }
   for (uint32_t b = 0; b < nfar; b++) {
