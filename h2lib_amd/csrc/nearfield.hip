@@ -779,7 +779,10 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
   // given normals that are not perpendicular to the triangles, or a surface
   // that folds back on itself: the FP64 double layer kernels with a product
   // <d, n> per value (no mirrored or fused tiles)
-  a.plane = s->plane;
+  // (and the Laplace far rule: 12800 triangles, constant basis 112 -> 104 us,
+  // adjoint, linear basis 550 -> 506 us, linear rows and constant columns 318
+  // -> 257 us)
+  a.plane = s->plane && !(far && op->kernel != H2HIP_HELMHOLTZ);
   const bool general =
       op->layer != H2HIP_SLP && op->precision == 0 && !s->plane;
   for (int i = 0; i < 9; i++) a.mass[i] = op->mass[i];

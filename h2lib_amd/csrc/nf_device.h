@@ -1814,6 +1814,15 @@ int launch_bases_p(uint32_t q, const KArgs &a, uint32_t ntiles,
       return H2HIP_OK;
     }
   }
+  // Laplace adjoint double layer at other orders than 2: a product <d, n> per
+  // value, in a kernel without the points' factors, whose registers it would
+  // pay for (order 3, 12800 triangles, linear basis 3190 -> 2983 us, constant
+  // rows and linear columns 1684 -> 1502).  The double layer takes the
+  // factors in the kernel with both (2884 us; 3022 by products, 3625 with the
+  // factors alone, whose loads the compiler then holds in registers).
+  constexpr bool LDLP = KER == K_LAP_DLP && MP == 0;
+  KArgs ar = a;
+  if (LDLP && q != 2 && a.adj) ar.plane = 0;
   if (ntiles && a.counter) {
     void (*reg)(KArgs, uint32_t, uint32_t *) = nullptr;
     switch (q) {
@@ -1833,7 +1842,7 @@ int launch_bases_p(uint32_t q, const KArgs &a, uint32_t ntiles,
     const uint32_t resident = (uint32_t)std::max(1, per_cu) * (uint32_t)ncu;
     const uint32_t grid = std::min(ntiles, std::max(1u, resident));
     hipLaunchKernelGGL(zero_counter, dim3(1), dim3(1), 0, stream, a.counter);
-    hipLaunchKernelGGL(reg, dim3(grid), dim3(NTHREADS), 0, stream, a, ntiles,
+    hipLaunchKernelGGL(reg, dim3(grid), dim3(NTHREADS), 0, stream, ar, ntiles,
                        a.counter);
   } else if (ntiles) {
     void (*reg)(KArgs) = nullptr;
@@ -1846,6 +1855,12 @@ int launch_bases_p(uint32_t q, const KArgs &a, uint32_t ntiles,
     }
     if constexpr (MP == 0 && is_dlp(KER))
       if (q == 2 && !a.plane) reg = nf_regular_kernel<KER, BR, BC, 2, MP, 0>;
+    if constexpr (LDLP)
+      if (!ar.plane) switch (q) {
+          case 1: reg = nf_regular_kernel<KER, BR, BC, 1, MP, 0>; break;
+          case 3: reg = nf_regular_kernel<KER, BR, BC, 3, MP, 0>; break;
+          case 4: reg = nf_regular_kernel<KER, BR, BC, 4, MP, 0>; break;
+        }
     hipLaunchKernelGGL(reg, dim3(ntiles * a.split), dim3(NTHREADS), 0, stream,
                        a);
   }

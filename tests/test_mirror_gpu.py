@@ -204,3 +204,35 @@ def test_constant_basis_bits_in_every_schedule(kern, k, layer, surface,
     want = run(h, plan, op, (0, 0, 0))
     for schedule in ((1, 0, 0), (0, 1, 0), (1, 1, 0), (0, 0, 1), (0, 1, 1)):
         assert np.array_equal(run(h, plan, op, schedule), want), schedule
+
+
+@pytest.mark.parametrize("q,q2,far", [(2, 4, True), (1, 3, False),
+                                      (3, 5, False), (3, 4, True)])
+@pytest.mark.parametrize("layer", [1, 2])
+def test_laplace_bits_at_other_orders_and_far(q, q2, far, layer, sphere8):
+    """The Laplace double layers take <x - y, n> per value in the far rule and
+    (adjoint) at orders other than 2, in every schedule."""
+    import h2lib_amd as h
+    gr = h.Surface3d(sphere8["x"], sphere8["t"])
+    idx = np.random.default_rng(6).permutation(gr.triangles).astype(np.uint32)
+    blocks = mirrored_blocks((64, 65, 130))
+    plan = h.NearfieldPlan(gr, 0, 0, idx, idx, blocks)
+    op = h.Bem3d(gr, 0, layer, q, q2, 0, 0, alpha=0.5)
+    orc = OracleBem(0, layer, 0, 0, sphere8["x"], sphere8["t"], q=q, q2=q2,
+                    alpha=0.5)
+    stream = h.Stream()
+    outs = []
+    for schedule in ((0, 0, 0), (0, 1, 0), (1, 0, 1)):
+        plan.set_schedule(*schedule)
+        out = h.DeviceArray(plan.entries, op.dtype)
+        out.fill_nan()
+        plan.execute(op, out.ptr, stream.handle, far)
+        stream.sync()
+        outs.append(out.download())
+        # (the far rule of a triangle with itself is not a number)
+        assert np.array_equal(outs[0], outs[-1], equal_nan=far), schedule
+    for b, (ro, r, co, c) in enumerate(blocks):
+        if far and ro == co:
+            continue
+        ref = orc.nearfield(idx[ro:ro + r], idx[co:co + c], far=far)
+        assert rel_block_err(plan.block(outs[0], b), ref) < 1e-12, b
