@@ -1171,14 +1171,27 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
   if constexpr (PLANE && CLS == CLS_IDENTICAL) {
   } else if constexpr (Q2 > 0) {
     // order known at compile time (Q2^2 <= 16): one (k, l) per lane, the
-    // nodes in registers, the (i, j) loops unrolled
+    // nodes in registers, the (i, j) loops unrolled.  Not the Helmholtz
+    // double layer with argument reduction in FP64: its evaluations are long
+    // enough that 24 of them interleaved take up to 360 registers, one wave
+    // per SIMD, so its loops (two, six or three evaluations a turn) stay
+    // loops: 134 to 232 registers (constant basis), two to three waves.
+    // Cylinder of 46240 triangles (no mirrored tiles), constant / linear
+    // basis 2.54 -> 2.06 / 11.16 -> 10.19 ms (2.34 / 11.04 before the
+    // branch-free sine and cosine let the compiler interleave them), sphere of
+    // 3872, linear basis, k = 5, mirrored tiles 679 -> 617 us.
     static_assert(Q2 * Q2 <= 16, "one tensor index pair per lane");
+    constexpr bool LONG = KER == K_HELM_DLP && !MP;
+    constexpr int UN = LONG ? 1 : Q2;
     double gn[Q2], gw[Q2];
 #pragma unroll
     for (int i = 0; i < Q2; i++) {
       gn[i] = a.gauss[i];
       gw[i] = a.gauss[Q2 + i];
     }
+    // node and weight i, read again where the loop is not unrolled
+    auto node = [&](int i) { return LONG ? a.gauss[i] : gn[i]; };
+    auto weight = [&](int i) { return LONG ? a.gauss[Q2 + i] : gw[i]; };
     if (sub < Q2 * Q2) {
       const int k = sub / Q2, l = sub % Q2;
       const double gk = a.gauss[k], gl = a.gauss[l];
@@ -1206,10 +1219,10 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
           b2[d] = xi * fma(E2[d], e3, E1[d]);
           c2[d] = -xi * F2[d];
         }
-#pragma unroll
+#pragma unroll UN
         for (int i = 0; i < Q2; i++) {
-          const double e1 = gn[i];
-          const double wi1 = wkl * gw[i] * e1;
+          const double e1 = node(i);
+          const double wi1 = wkl * weight(i) * e1;
           double t1[3], t2[3];
 #pragma unroll
           for (int d = 0; d < 3; d++) {
@@ -1222,9 +1235,9 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
           for (int z = 0; z < ND; z++)
             U0r[z] = U0i[z] = U2r[z] = U2i[z] = V0r[z] = V0i[z] = V2r[z] =
                 V2i[z] = 0.0;
-#pragma unroll
+#pragma unroll UN
           for (int j = 0; j < Q2; j++) {
-            const double e2 = gn[j], w = wi1 * gw[j];
+            const double e2 = node(j), w = wi1 * weight(j);
             double d1[3], d2[3];
 #pragma unroll
             for (int d = 0; d < 3; d++) {
@@ -1324,9 +1337,9 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
           double W0r[6], W1r[6], W0i[6], W1i[6];
 #pragma unroll
           for (int m = 0; m < 6; m++) W0r[m] = W1r[m] = W0i[m] = W1i[m] = 0.0;
-#pragma unroll
+#pragma unroll UN
           for (int j = 0; j < Q2; j++) {
-            const double pq = p * gn[j], w = wi1 * gw[j];
+            const double pq = p * node(j), w = wi1 * weight(j);
 #pragma unroll
             for (int m = 0; m < 6; m++) {
               double dd[3];
@@ -1436,9 +1449,9 @@ __device__ __forceinline__ void singular_pair(const KArgs &a, const Tile &T,
           double W0r[6], W1r[6], W0i[6], W1i[6];
 #pragma unroll
           for (int m = 0; m < 6; m++) W0r[m] = W1r[m] = W0i[m] = W1i[m] = 0.0;
-#pragma unroll
+#pragma unroll UN
           for (int i = 0; i < Q2; i++) {
-            const double eta = gn[i], w = gw[i] * wj1;
+            const double eta = node(i), w = weight(i) * wj1;
             const double bb = x1 * (1.0 - eta);
             double dv[3][3], pr[3], pi[3];
 #pragma unroll
