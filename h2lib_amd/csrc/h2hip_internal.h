@@ -151,7 +151,7 @@ struct KArgs {
   // adjoint double layer: the kernels of the double layer take -n_x (the
   // row triangle's normal) in place of n_y, <y - x, n_x> = <x - y, -n_x>
   int adj;
-  // the normals are perpendicular to their triangles (to 1e-12) and the
+  // the normals are perpendicular to their triangles (to rounding) and the
   // surface has no folds: the FP64 double layers then use that <d, n> is
   // constant along the triangle of n
   int plane;
@@ -210,7 +210,7 @@ struct h2hip_surface {
   std::vector<uint32_t> t;
   std::vector<uint32_t> v2t_ptr, v2t;  // triangles of each vertex
   double hmax = 0.0;                   // longest edge
-  bool plane = true;  // normals perpendicular to the triangles (to 1e-12)
+  bool plane = true;  // normals perpendicular to the triangles (to rounding)
                       // and no two triangles at a vertex folded together
   h2hip::DevBuf<double> d_x, d_n, d_g;
   h2hip::DevBuf<uint32_t> d_t;

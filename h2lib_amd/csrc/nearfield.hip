@@ -1167,17 +1167,23 @@ int h2hip_surface_create(h2hip_surface **out, uint32_t vertices,
       h2 = std::max(h2, d0 * d0 + d1 * d1 + d2 * d2);
     }
   s->hmax = std::sqrt(h2);
-  if (n && g)
-    for (uint32_t i = 0; i < triangles && s->plane; i++)
-      for (int l = 0; l < 3; l++) {
-        const double *p = &s->x[3 * s->t[3 * i + l]];
-        const double *q = &s->x[3 * s->t[3 * i + (l + 1) % 3]];
-        const double e[3] = {q[0] - p[0], q[1] - p[1], q[2] - p[2]};
-        const double *m = &s->n[3 * i];
-        const double ne = e[0] * m[0] + e[1] * m[1] + e[2] * m[2];
-        if (!(ne * ne <= 1e-24 * (e[0] * e[0] + e[1] * e[1] + e[2] * e[2])))
-          s->plane = false;
-      }
+  // Normals perpendicular to the triangles to rounding: 8 * 2^-52 of both
+  // lengths (unit normals formed from the edges are within 1.3 on spheres,
+  // cubes and cylinders; needles, whose normals have fewer digits, and
+  // normals from elsewhere may be further off and are taken as they are)
+  constexpr double PERP = 8.0 * 2.220446049250313e-16;
+  for (uint32_t i = 0; i < triangles && s->plane; i++)
+    for (int l = 0; l < 3; l++) {
+      const double *p = &s->x[3 * s->t[3 * i + l]];
+      const double *q = &s->x[3 * s->t[3 * i + (l + 1) % 3]];
+      const double e[3] = {q[0] - p[0], q[1] - p[1], q[2] - p[2]};
+      const double *m = &s->n[3 * i];
+      const double ne = e[0] * m[0] + e[1] * m[1] + e[2] * m[2];
+      if (!(ne * ne <= PERP * PERP *
+                           (e[0] * e[0] + e[1] * e[1] + e[2] * e[2]) *
+                           (m[0] * m[0] + m[1] * m[1] + m[2] * m[2])))
+        s->plane = false;
+    }
   // triangles of each vertex, in decreasing triangle order as the
   // reference's prepend-built lists
   s->v2t_ptr.assign(vertices + 1, 0);

@@ -236,3 +236,68 @@ def test_laplace_bits_at_other_orders_and_far(q, q2, far, layer, sphere8):
             continue
         ref = orc.nearfield(idx[ro:ro + r], idx[co:co + c], far=far)
         assert rel_block_err(plan.block(outs[0], b), ref) < 1e-12, b
+
+
+@pytest.mark.parametrize("kern,k", [(0, 0.0), (1, 0.1), (1, 5.0),
+                                    (1, 2.0 + 0.5j)])
+@pytest.mark.parametrize("layer", [1, 2])
+@pytest.mark.parametrize("basis", [0, 1])
+def test_fine_folded_cylinder_one_launch_per_class(kern, k, layer, basis):
+    """More than 32768 touching pairs on a folded surface: a launch per rule
+    class of the kernels with <x - y, n> per value.  A plan of a few of the
+    blocks takes the launch of all classes: the same entries (constant basis:
+    the same bits).  Where folded sheets lie in one plane the entries are
+    rounding noise, so the oracle's are compared on the scale of all."""
+    import h2lib_amd as h
+    from h2lib_amd import geometry as G
+    mesh = G.cylinder(22)
+    gr = h.Surface3d(mesh.x, mesh.t, mesh.n, mesh.g)
+    rt = G.ClusterTree(mesh, basis, 64)
+    bt = G.BlockTree(rt, rt, 2.0, 0)
+    blocks = bt.near_block_list()
+    plan = h.NearfieldPlan(gr, basis, basis, rt.idx, rt.idx, blocks)
+    op = h.Bem3d(gr, kern, layer, 2, 4, basis, basis, alpha=0.5, k=k)
+    assert plan.work(op)[1][1:].sum() > 32768
+    got = run(h, plan, op, (0, 0, 0))
+    scale = np.abs(got).max()
+    sel = np.random.default_rng(1).choice(len(blocks), 10, replace=False)
+    few = h.NearfieldPlan(gr, basis, basis, rt.idx, rt.idx, blocks[sel])
+    assert few.work(op)[1][1:].sum() <= 32768
+    part = run(h, few, op, (0, 0, 0))
+    orc = OracleBem(kern, layer, basis, basis, mesh.x, mesh.t, q=2, q2=4,
+                    alpha=0.5, k=k)
+    for i, b in enumerate(sel):
+        ro, r, co, c = (int(v) for v in blocks[b])
+        a = plan.block(got, b)
+        if basis == 0:
+            assert np.array_equal(few.block(part, i), a), b
+        else:
+            assert np.abs(few.block(part, i) - a).max() < 1e-14 * scale, b
+        ref = orc.nearfield(rt.idx[ro:ro + r], rt.idx[co:co + c])
+        assert np.abs(a - ref).max() < 1e-12 * scale, b
+
+
+@pytest.mark.parametrize("tilt", [3e-13, 1e-14])
+@pytest.mark.parametrize("kern,k", [(0, 0.0), (1, 2.0)])
+@pytest.mark.parametrize("layer", [1, 2])
+@pytest.mark.parametrize("basis", [0, 1])
+def test_given_normals_are_exact(tilt, kern, k, layer, basis, sphere8):
+    """Normals off the perpendicular by a little more than rounding are taken
+    as they are: <x - y, n> is linear in n.  Entries are sums of <d, n> / r^3
+    with a few roundings of |d| / r^3 each, which the in-plane normals' entries
+    have the size of: 16 * 2^-52 of their largest."""
+    import h2lib_amd as h
+    x, t = sphere8["x"], sphere8["t"]
+    plain = h.Surface3d(x, t)
+    roll = np.roll(plain.n, 1, axis=1)
+    dofs = plain.vertices if basis else plain.triangles
+    idx = np.random.default_rng(8).permutation(dofs).astype(np.uint32)
+    vals = []
+    for nn in (plain.n, roll, plain.n + tilt * roll):
+        gr = h.Surface3d(x, t, nn, plain.g)
+        op = h.Bem3d(gr, kern, layer, 2, 4, basis, basis, alpha=0.0, k=k)
+        plan = h.NearfieldPlan(gr, basis, basis, idx, idx,
+                               mirrored_blocks((64, 9)))
+        vals.append(run(h, plan, op, (0, 0, 0)))
+    a, b, c = vals
+    assert np.abs(c - (a + tilt * b)).max() < 16 * 2.0 ** -52 * np.abs(b).max()
