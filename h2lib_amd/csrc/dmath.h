@@ -88,14 +88,15 @@ __device__ __forceinline__ void sincos_cw(double x, double &s, double &c) {
 // and fused products, |r| <= 0.3466, the Taylor polynomial of degree 13 (the
 // first term left out is 4.2e-18 at most) and a scaling by 2^n.  Relative
 // error below 0.63 * 2^-52 (4e6 arguments against long-double expl, the same
-// operations in C).  No branches, for the damping of the coupling values
+// operations in C); NaN gives NaN.  No branches, for the damping of the coupling values
 // (the library's exponential breaks up the evaluations of a lane).
 __device__ __forceinline__ double exp_cw(double x) {
   constexpr double LOG2E = 1.4426950408889634;
   constexpr double L1 = 0.6931471805599453, L2 = 2.3190468138462996e-17;
   constexpr double MAGIC = 6755399441055744.0;
-  // beyond, the result is 0 or infinite
-  x = fmin(fmax(x, -1100.0), 1100.0);
+  // beyond, the result is 0 or infinite (selections, which keep a NaN)
+  x = x < -1100.0 ? -1100.0 : x;
+  x = x > 1100.0 ? 1100.0 : x;
   const double m = fma(x, LOG2E, MAGIC);
   const double n = m - MAGIC;
   double r = fma(-n, L1, x);

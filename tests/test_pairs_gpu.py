@@ -195,3 +195,42 @@ def test_many_pairs_match_general_kernels(kern, layer, basis, k, schedule):
                                 ).all(), (mode, trans, nv, err)
     finally:
         h.set_reproducible(True)
+
+
+@pytest.mark.parametrize("m", [4, 3])
+def test_nan_wave_number_reaches_every_coupling(m):
+    """A damping that is not a number gives couplings that are not (with the
+    near field zero, so that they alone decide)."""
+    import ctypes as C
+    import h2lib_amd as h
+    from h2lib_amd import geometry as G
+    from h2lib_amd.h2matrix import H2Matrix
+    mesh = G.sphere(12)
+    gr = h.Surface3d(mesh.x, mesh.t, mesh.n, mesh.g)
+    op = h.Bem3d(gr, 1, 0, 2, 4, 0, 0, k=complex(2.0, np.nan))
+    rt = G.ClusterTree(mesh, 0, 16)
+    bt = G.BlockTree(rt, rt, 2.0, 0)
+    H = H2Matrix(op, mesh, rt, rt, bt, m)
+    nb = bt.near_block_list().astype(np.int64)
+    near = np.zeros(int((nb[:, 1] * nb[:, 3]).sum()), dtype=H.dtype)
+    assert h.hip().h2hip_h2matrix_set_nearfield(
+        H._h, near.ctypes.data_as(C.c_void_p)) == 0
+    d_x = [h.DeviceArray.from_host(np.ones(H.n, dtype=H.dtype))] * 2
+    d_y = [h.DeviceArray(H.n, H.dtype) for _ in range(2)]
+    H.set_schedule(2)
+    try:
+        for mode in (0, 1):
+            H.set_coupling_mode(mode)
+            for rep in (False, True):
+                h.set_reproducible(rep)
+                for trans in (False, True):
+                    for y in d_y:
+                        y.zero()
+                    H.addeval_batch([1.0, 1.0], d_x, d_y, trans=trans)
+                    two = d_y[1].download()
+                    d_y[0].zero()
+                    H.addeval(1.0, d_x[0], d_y[0], trans=trans)
+                    for y in (two, d_y[0].download()):
+                        assert np.isnan(y).all(), (mode, rep, trans)
+    finally:
+        h.set_reproducible(True)
