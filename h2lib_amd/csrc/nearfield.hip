@@ -21,6 +21,7 @@
 #include <numeric>
 #include <unordered_map>
 
+#include "folds.h"
 #include "h2hip_internal.h"
 
 namespace h2hip {
@@ -1064,28 +1065,6 @@ void give_context(const h2hip_op *op, CbCtx *c) {
   op->cb_cv.notify_one();
 }
 
-// Whether two triangles with a common vertex have opposite normals (to 18
-// degrees): the surface folds back on itself there, as the finer cylinder
-// meshes do.  Where the folded sheets overlap, <x - y, n> is zero up to the
-// rounding of the points, which 1/r^3 magnifies: forming it from anything
-// but the difference x - y moves such entries by up to 1e-9 of the largest
-// (cylinder, 46240 triangles; 8e-13 in the norm of all entries).
-bool folds(const h2hip_surface &s) {
-  for (uint32_t v = 0; v < s.nv; v++)
-    for (uint32_t p = s.v2t_ptr[v]; p < s.v2t_ptr[v + 1]; p++) {
-      const double *a = &s.n[3 * s.v2t[p]];
-      for (uint32_t q = p + 1; q < s.v2t_ptr[v + 1]; q++) {
-        const double *b = &s.n[3 * s.v2t[q]];
-        const double ab = a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
-        if (ab < 0.0 &&
-            ab * ab > 0.9 * (a[0] * a[0] + a[1] * a[1] + a[2] * a[2]) *
-                          (b[0] * b[0] + b[1] * b[1] + b[2] * b[2]))
-          return true;
-      }
-    }
-  return false;
-}
-
 }  // namespace
 }  // namespace h2hip
 
@@ -1196,7 +1175,8 @@ int h2hip_surface_create(h2hip_surface **out, uint32_t vertices,
       const uint32_t v = t[3 * i + l];
       s->v2t[s->v2t_ptr[v] + fill[v]++] = i;
     }
-  s->plane = s->plane && !folds(*s);
+  s->plane = s->plane && !folds(vertices, s->v2t_ptr.data(), s->v2t.data(),
+                                s->n.data());
   int rc = H2HIP_OK;
   if (s->d_x.upload(s->x.data(), s->x.size()) != hipSuccess ||
       s->d_t.upload(s->t.data(), s->t.size()) != hipSuccess ||
