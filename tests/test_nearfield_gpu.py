@@ -152,6 +152,71 @@ def test_window_inside_larger_matrix(sphere8):
     assert np.all(big[mask] == 7.0)
 
 
+@pytest.mark.parametrize("name", ["lap_slp_cc", "helm_dlp_cc"])
+@pytest.mark.parametrize("ntrans", [0, 1])
+def test_large_windows_of_larger_matrices(name, ntrans):
+    # outputs of several pieces of 2 MB (8.6 and 17 MB, so more than one
+    # thread for the larger), which end inside columns, into windows: the
+    # same entries as without a window, and nothing beside it
+    import h2lib_amd as h
+    from h2lib_amd import geometry as G
+    kern, layer, br, bc, _, k = CASES[name]
+    mesh = G.sphere(16)
+    gr = h.Surface3d(mesh.x, mesh.t, mesh.n, mesh.g)
+    # (without the identity term, whose place depends on the block)
+    op = h.Bem3d(gr, kern, layer, 2, 4, br, bc, alpha=0.0, k=k)
+    idx = np.random.default_rng(3).permutation(gr.triangles)
+    rows, cols = 1237, 871
+    ridx, cidx = idx[:rows], idx[100:100 + cols]
+    want = op.nearfield(ridx, cidx, ntrans=ntrans)
+    assert want.nbytes > 4 << 21
+    wr, wc = want.shape
+    big = np.full((wr + 19, wc + 5), 7.0, dtype=op.dtype, order="F")
+    op.nearfield(ridx, cidx, ntrans=ntrans, N=big[6:6 + wr, 2:2 + wc])
+    assert np.array_equal(big[6:6 + wr, 2:2 + wc], want)
+    mask = np.ones(big.shape, dtype=bool)
+    mask[6:6 + wr, 2:2 + wc] = False
+    assert np.all(big[mask] == 7.0)
+    # small blocks in one piece
+    for r in (0, 640, 1200):
+        part = op.nearfield(ridx[r:r + 30], cidx, ntrans=ntrans)
+        assert np.array_equal(part, want[:, r:r + 30] if ntrans
+                              else want[r:r + 30])
+
+
+def test_deferred_blocks_across_pieces():
+    # recorded blocks of both orientations and all sizes, 13 MB together, so
+    # that pieces hold several blocks and blocks several pieces
+    import ctypes as C
+    import h2lib_amd as h
+    from h2lib_amd import geometry as G
+    mesh = G.sphere(16)
+    gr = h.Surface3d(mesh.x, mesh.t, mesh.n, mesh.g)
+    op = h.Bem3d(gr, 0, 1, 2, 4, 0, 0, alpha=0.5)
+    rng = np.random.default_rng(4)
+    idx = rng.permutation(gr.triangles).astype(np.uint32)
+    lib = h.hip()
+    blocks = []
+    for b, (r, c) in enumerate([(1, 1), (700, 900), (64, 3), (1, 2000),
+                                (130, 70), (900, 901), (2, 2), (333, 500)]):
+        ro = int(rng.integers(0, len(idx) - r + 1))
+        co = int(rng.integers(0, len(idx) - c + 1))
+        ntrans = b % 3 == 1
+        wr, wc = (c, r) if ntrans else (r, c)
+        big = np.full((wr + b, wc + 1), 7.0, order="F")
+        ri, ci = idx[ro:ro + r].copy(), idx[co:co + c].copy()
+        assert lib.h2hip_nearfield_defer(
+            op.handle, 0, ri.ctypes.data_as(C.c_void_p), r,
+            ci.ctypes.data_as(C.c_void_p), c, int(ntrans),
+            big.ctypes.data_as(C.c_void_p), C.c_size_t(wr + b)) == 0
+        blocks.append((ri, ci, ntrans, big, wr, wc))
+    assert lib.h2hip_nearfield_flush(op.handle) == 0
+    for ri, ci, ntrans, big, wr, wc in blocks:
+        want = op.nearfield(ri, ci, ntrans=ntrans)
+        assert np.array_equal(big[:wr, :wc], want), (wr, wc)
+        assert np.all(big[wr:] == 7.0) and np.all(big[:, wc:] == 7.0)
+
+
 @pytest.mark.parametrize("q,q2", [(1, 3), (3, 5), (4, 6)])
 def test_other_orders(q, q2, sphere4):
     for name in ("lap_slp_cc", "helm_dlp_ll", "lap_dlp_cl", "lap_adlp_lc"):

@@ -146,6 +146,37 @@ def test_large_helmholtz_product_runs_near_blocks_with_the_pairs():
         assert np.abs(got - out[0]).max() < 1e-13 * np.abs(out[0]).max()
 
 
+def test_large_damped_product_runs_near_blocks_with_the_pairs():
+    """The same with a complex wave number and a double layer."""
+    import h2lib_amd as h
+    from h2lib_amd import geometry as G
+    from h2lib_amd.h2matrix import H2Matrix
+    mesh = G.sphere(128)
+    gr = h.Surface3d(mesh.x, mesh.t, mesh.n, mesh.g)
+    op = h.new_dlp_helmholtz_bem3d(2.0 + 0.3j, gr, 2, 4, 0, 0, 0.5)
+    rt = G.ClusterTree(mesh, 0, 64)
+    bt = G.BlockTree(rt, rt, 2.0, 0)
+    H = H2Matrix(op, mesh, rt, rt, bt, 4)
+    H.set_schedule(2)
+    H.set_coupling_mode(1)
+    assert H.coupling_pairs() >= 8 * 768 * 4
+    rng = np.random.default_rng(6)
+    d_x = h.DeviceArray.from_host(rng.standard_normal(H.n) +
+                                  1j * rng.standard_normal(H.n))
+    d_y = h.DeviceArray(H.n, H.dtype)
+    out = []
+    try:
+        for rep in (True, False, False):
+            h.set_reproducible(rep)
+            d_y.zero()
+            H.addeval(0.5 + 0.25j, d_x, d_y)
+            out.append(d_y.download())
+    finally:
+        h.set_reproducible(True)
+    for got in out[1:]:
+        assert np.abs(got - out[0]).max() < 1e-13 * np.abs(out[0]).max()
+
+
 @pytest.mark.parametrize("schedule", [2, 0])
 @pytest.mark.parametrize("kern,layer,basis,k", [
     (0, 0, 1, 0.0), (0, 1, 1, 0.0), (1, 0, 0, 3.0), (1, 1, 0, 2.0 + 0.5j)])
