@@ -134,6 +134,9 @@ struct KArgs {
   const double *n;       // unit normals
   const double *g;       // Gram determinants
   const double *regpts;  // regular-rule points, 3 q^2 per triangle
+  // double layers: normal and mean of <p_i - p_0, n> over the regular points
+  // p_i, 4 per triangle
+  const double *regn;
   const double *regw;    // regular weights: w | phi0 w | phi1 w | phi2 w
   const double *gauss;   // Gauss-Legendre nodes and weights on [0, 1], q2 each
   // mixed precision only: offsets of the regular points from point 0 of
@@ -255,6 +258,7 @@ struct h2hip_op {
   h2hip::DevBuf<double> d_gauss;
   // regular rule: per-triangle points (3 * q * q doubles per triangle)
   h2hip::DevBuf<double> d_regpts;
+  h2hip::DevBuf<double> d_regn;  // nf::KArgs::regn (double layers)
   // mixed precision: regular points relative to point 0 of their triangle
   // and the regular weights, in FP32
   h2hip::DevBuf<float> d_regoff, d_regwf;

@@ -87,6 +87,20 @@ __global__ void regpts_kernel(const double *x, const uint32_t *t, uint32_t nt,
     pts[3 * (size_t)i + d] = A[d] * ca + B[d] * cb + C[d] * cc;
 }
 
+// Double layers: normal of each triangle and the mean of <p_i - p_0, n> over
+// its points p_i, zero but for their rounding
+__global__ void regn_kernel(const double *n, const double *pts, uint32_t nt,
+                            int qq, double *out) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nt) return;
+  const double *p = pts + 3 * (size_t)i * qq, *m = n + 3 * (size_t)i;
+  double s = 0.0;
+  for (int a = 1; a < qq; a++)
+    for (int d = 0; d < 3; d++) s = fma(p[3 * a + d] - p[d], m[d], s);
+  for (int d = 0; d < 3; d++) out[4 * (size_t)i + d] = m[d];
+  out[4 * (size_t)i + 3] = s / qq;
+}
+
 // 1/(4 pi) (Library/laplacebem3d.c:33)
 constexpr double KERNEL_CONST = 0.0795774715459476679;
 
@@ -762,6 +776,7 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
   a.n = s->d_n.p;
   a.g = s->d_g.p;
   a.regpts = op->d_regpts.p;
+  a.regn = op->d_regn.p;
   a.regw = op->d_regw.p;
   a.gauss = op->d_gauss.p;
   a.regoff = op->d_regoff.p;
@@ -777,13 +792,23 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
   a.are = op->layer != H2HIP_SLP ? op->alpha[0] : 0.0;
   a.aim = op->layer != H2HIP_SLP ? op->alpha[1] : 0.0;
   a.adj = op->layer == H2HIP_ADLP;
+  // FP64 Helmholtz kernels without argument reduction: real k, and the phase
+  // varies by at most pi/4 (1/4: shorter polynomials still) over two edges
+  // (|r - r0| <= 2 h within a pair of triangles, r <= 2 h in a pair with
+  // common vertices)
+  const double phase = std::fabs(a.kr) * 2.0 * s->hmax;
+  const bool real64 = a.mp == 0 && a.ki == 0.0;
+  const bool tiny = real64 && phase <= 0.25;
+  const bool small = real64 && phase <= 0.25 * M_PI;
   // given normals that are not perpendicular to the triangles, or a surface
   // that folds back on itself: the FP64 double layer kernels with a product
-  // <d, n> per value (no mirrored or fused tiles)
-  // (and the Laplace far rule: 12800 triangles, constant basis 112 -> 104 us,
-  // adjoint, linear basis 550 -> 506 us, linear rows and constant columns 318
-  // -> 257 us)
-  a.plane = s->plane && !(far && op->kernel != H2HIP_HELMHOLTZ);
+  // <d, n> per value (no mirrored or fused tiles); so in the far rule of the
+  // Laplace kernels (12800 triangles, constant basis 112 -> 104 us, adjoint,
+  // linear basis 550 -> 506 us, linear rows and constant columns 318 -> 257
+  // us) and of the constant-basis Helmholtz ones with argument reduction (268
+  // -> 244 us)
+  a.plane = s->plane && !(far && (op->kernel != H2HIP_HELMHOLTZ ||
+                                  (!small && !op->rb && !op->cb)));
   const bool general =
       op->layer != H2HIP_SLP && op->precision == 0 && !s->plane;
   for (int i = 0; i < 9; i++) a.mass[i] = op->mass[i];
@@ -824,14 +849,6 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
   const uint32_t ntiles = (uint32_t)P->tiles.size();
   uint32_t ncls[4];
   for (int c = 0; c < 4; c++) ncls[c] = (uint32_t)P->pairs[c];
-  // FP64 Helmholtz kernels without argument reduction: real k, and the phase
-  // varies by at most pi/4 (1/4: shorter polynomials still) over two edges
-  // (|r - r0| <= 2 h within a pair of triangles, r <= 2 h in a pair with
-  // common vertices)
-  const double phase = std::fabs(a.kr) * 2.0 * s->hmax;
-  const bool real64 = a.mp == 0 && a.ki == 0.0;
-  const bool tiny = real64 && phase <= 0.25;
-  const bool small = real64 && phase <= 0.25 * M_PI;
   auto launch = op->kernel != H2HIP_HELMHOLTZ ? nullptr
                 : op->layer == H2HIP_SLP
                     ? (tiny    ? nf::launch_helmholtz_slp_tp
@@ -1260,7 +1277,9 @@ int h2hip_op_create(h2hip_op **out, const h2hip_surface *s, int kernel,
       op->d_regw.upload(op->regw.data(), op->regw.size()) != hipSuccess ||
       d_x0.upload(tr.x0.data(), qq) != hipSuccess ||
       d_x1.upload(tr.x1.data(), qq) != hipSuccess ||
-      op->d_regpts.alloc(3 * (size_t)qq * s->nt) != hipSuccess) {
+      op->d_regpts.alloc(3 * (size_t)qq * s->nt) != hipSuccess ||
+      (layer != H2HIP_SLP &&
+       op->d_regn.alloc(4 * (size_t)s->nt) != hipSuccess)) {
     set_error("h2hip_op_create: device allocation failed");
     rc = H2HIP_ENOMEM;
   }
@@ -1269,6 +1288,10 @@ int h2hip_op_create(h2hip_op **out, const h2hip_surface *s, int kernel,
     hipLaunchKernelGGL(regpts_kernel, dim3((n + 255) / 256), dim3(256), 0, 0,
                        s->d_x.p, s->d_t.p, s->nt, d_x0.p, d_x1.p, qq,
                        op->d_regpts.p);
+    if (layer != H2HIP_SLP)
+      hipLaunchKernelGGL(regn_kernel, dim3((s->nt + 255) / 256), dim3(256), 0,
+                         0, s->d_n.p, op->d_regpts.p, s->nt, qq,
+                         op->d_regn.p);
     if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
       set_error("h2hip_op_create: point kernel failed");
       rc = H2HIP_EDEVICE;

@@ -246,7 +246,8 @@ __device__ __forceinline__ void kahan_add(float &s, float &c, float x) {
 // Element matrices of a pair of triangles without common vertices by the
 // tensor-product rule with points x_i on triangle tt and y_b on triangle ts,
 // d = x_i - y_b, over the local functions l of tt and k of ts (1 or 3 each).
-// nt, ns: the triangles' normals.
+// nt, ns: the triangles' normals and the means of their points' <p_i - p_0,
+// n> (KArgs::regn).
 //
 // The double layers' <d, n> of one order of the pair takes the normal of ts,
 // of the other that of tt: A = <d, ns> and B = <d, -nt> (the differences
@@ -256,7 +257,11 @@ __device__ __forceinline__ void kahan_add(float &s, float &c, float x) {
 // phase.  FP64 and a.plane (normals perpendicular to the triangles): A does
 // not depend on b nor B on i, so A is a factor of the row point and B of the
 // column point and no value takes a product of vectors (double layer, linear
-// basis, 32768 triangles: 1011 -> 945 us).
+// basis, 32768 triangles: 1011 -> 945 us).  Both are taken from the mean of
+// the other triangle's points, not from one of them, whose rounding would be
+// in every value: entries of touching clusters are then off by 0.97 to 1.01
+// times what a product per value gives, from one point by 1.6 times (sphere
+// of 8192 triangles, constant basis, against long double).
 // MP: 0 FP64; 1 mixed (FP32 kernel values and inner sums, FP64 outer sums);
 // 2 mixed with FP32 accumulation throughout, the outer sums compensated
 // (Kahan); TWO is for MP 0 and single layers with MP 1 (S2 is not set: the
@@ -265,8 +270,8 @@ __device__ __forceinline__ void kahan_add(float &s, float &c, float x) {
 // kernel with both ways takes the registers of the larger, up to 220).
 template <int KER, int BR, int BC, int Q, int MP, bool TWO, int PL_>
 __device__ __forceinline__ void pair_sums(
-    const KArgs &a, uint32_t tt, uint32_t ts, const double (&nt)[3],
-    const double (&ns)[3], bool wantB, double sg,
+    const KArgs &a, uint32_t tt, uint32_t ts, const double (&nt)[4],
+    const double (&ns)[4], bool wantB, double sg,
     double (&S1re)[BR ? 3 : 1][BC ? 3 : 1],
     double (&S1im)[BR ? 3 : 1][BC ? 3 : 1],
     double (&S2re)[BR ? 3 : 1][BC ? 3 : 1],
@@ -391,10 +396,12 @@ __device__ __forceinline__ void pair_sums(
         for (int i = 0; i < QQ; i++) {
           const double A =
               fma(ptx[i] - Ps[0], ns[0],
-                  fma(pty[i] - Ps[1], ns[1], (ptz[i] - Ps[2]) * ns[2]));
+                  fma(pty[i] - Ps[1], ns[1],
+                      fma(ptz[i] - Ps[2], ns[2], -ns[3])));
           const double B = -fma(ptx[0] - Ps[3 * i], nt[0],
                                 fma(pty[0] - Ps[3 * i + 1], nt[1],
-                                    (ptz[0] - Ps[3 * i + 2]) * nt[2]));
+                                    fma(ptz[0] - Ps[3 * i + 2], nt[2],
+                                        nt[3])));
           fi_[i] = TWO ? A : wantB ? 1.0 : sg * A;
           fb_[i] = TWO ? B : wantB ? sg * B : 1.0;
         }
@@ -536,11 +543,11 @@ __device__ __forceinline__ void entry_sums(
   // n_y belongs to the column triangle, the adjoint's -n_x to the row
   // triangle; d changes sign with the order except in the lc far rule
   const bool wantB = (a.adj != 0) != sw;
-  double nv[3] = {0.0, 0.0, 0.0};
+  double nv[4] = {0.0, 0.0, 0.0, 0.0};
   if constexpr (is_dlp(KER)) {
     const uint32_t t = a.adj ? rt : ct;
 #pragma unroll
-    for (int d = 0; d < 3; d++) nv[d] = a.n[3 * t + d];
+    for (int d = 0; d < 4; d++) nv[d] = a.regn[4 * (size_t)t + d];
   }
   double dre[BR ? 3 : 1][BC ? 3 : 1], dim[BR ? 3 : 1][BC ? 3 : 1];
   // (only the normal of the one order is read)
@@ -710,14 +717,19 @@ void nf_regular_kernel(KArgs a) {
 // per workgroup follow the LDS accumulators so that 4 to 5 waves per SIMD
 // are resident: 256 for 32 KB, 512 for 64 KB.  Against one workgroup per
 // tile (nf_regular_kernel): Laplace double layer, linear basis, 32768
-// triangles 1431 -> 1011 us; Helmholtz single layer, constant basis, 131072
-// triangles 2735 -> 1208 us (with the small phase; vertex pairs
-// 1291 -> 465 us, edge pairs, small phase alone, 1153 -> 799 us).
+// triangles 1431 -> 1011 us by this kernel alone and 822 with the points'
+// factors; Helmholtz single layer, constant basis, 131072 triangles, all
+// launches, 5230 -> 2490 us with it and the small phase (2050 to 2190 with
+// the tiny one).  Constant basis: 4 waves where 5 spill (Laplace double
+// layer, 12800 triangles 230 -> 177 us), 3 for the tiny-phase double layer
+// (260 -> 244 us).
 constexpr int pair_threads(int ker, int basis) {
   return pair_arrays(ker, basis) > 1 ? 512 : NTHREADS;
 }
 constexpr int pair_waves(int ker, int basis) {
-  return (basis ? pair_arrays(ker, basis) > 1 : ker >= K_HELM_SLP) ? 4 : 5;
+  return ker == K_HELM_DLP_TP && !basis ? 3
+         : (basis ? pair_arrays(ker, basis) > 1 : ker != K_LAP_SLP) ? 4
+                                                                    : 5;
 }
 
 template <int KER, int B, int Q, int MP>
@@ -795,12 +807,12 @@ __global__ __launch_bounds__(pair_threads(KER, B),
     if (!shared) {
       f2 = pair_factor<!B>(a, sr.tri, sc.tri);
       const uint32_t tt = sw ? sc.tri : sr.tri, ts = sw ? sr.tri : sc.tri;
-      double nt[3] = {0.0, 0.0, 0.0}, ns[3] = {0.0, 0.0, 0.0};
+      double nt[4] = {0.0, 0.0, 0.0, 0.0}, ns[4] = {0.0, 0.0, 0.0, 0.0};
       if constexpr (DLP) {
 #pragma unroll
-        for (int d = 0; d < 3; d++) {
-          nt[d] = a.n[3 * tt + d];
-          ns[d] = a.n[3 * ts + d];
+        for (int d = 0; d < 4; d++) {
+          nt[d] = a.regn[4 * (size_t)tt + d];
+          ns[d] = a.regn[4 * (size_t)ts + d];
         }
       }
       pair_sums<KER, B, B, Q, MP, DLP, 1>(a, tt, ts, nt, ns, false, 1.0, S1re,

@@ -301,3 +301,68 @@ def test_given_normals_are_exact(tilt, kern, k, layer, basis, sphere8):
         vals.append(run(h, plan, op, (0, 0, 0)))
     a, b, c = vals
     assert np.abs(c - (a + tilt * b)).max() < 16 * 2.0 ** -52 * np.abs(b).max()
+
+
+@pytest.mark.parametrize("layer", [1, 2])
+@pytest.mark.parametrize("k", [0.0, 2.0])
+def test_double_layer_entries_lose_no_digits(layer, k):
+    """Entries of touching clusters against long double: no further off than a
+    product <x - y, n> per value in FP64 (the regular rule of triangles
+    without common vertices; the kernels take <x - y, n> as a factor of one
+    triangle's point)."""
+    import h2lib_amd as h
+    from h2lib_amd import geometry as G
+    mesh = G.sphere(32)
+    gr = h.Surface3d(mesh.x, mesh.t, mesh.n, mesh.g)
+    op = h.Bem3d(gr, int(k != 0.0), layer, 2, 4, 0, 0, alpha=0.0, k=k)
+    rt = G.ClusterTree(mesh, 0, 64)
+    blocks = [b for b in G.BlockTree(rt, rt, 2.0, 0).near_block_list()
+              if b[0] != b[2]][::9]
+    gauss, wg = np.polynomial.legendre.leggauss(2)
+    gauss, wg = 0.5 * (gauss + 1.0), 0.5 * wg
+    u = np.repeat(gauss, 2)
+    v = np.outer(gauss, gauss).ravel()
+    w = (np.outer(wg, wg) * gauss[:, None]).ravel()
+    x, t = np.asarray(mesh.x), np.asarray(mesh.t).astype(np.int64)
+
+    def entries(ri, ci, real):
+        X = x.astype(real)
+        uu, vv, ww = u.astype(real), v.astype(real), w.astype(real)
+
+        def points(tri):
+            a, b, c = (X[t[tri, i]][:, None, :] for i in range(3))
+            return (a * (1 - uu)[None, :, None] + b * (uu - vv)[None, :, None]
+                    + c * vv[None, :, None])
+        p, q = points(ri), points(ci)
+        n = np.asarray(mesh.n).astype(real)
+        g = np.asarray(mesh.g).astype(real)
+        re = np.zeros((len(ri), len(ci)), real)
+        im = np.zeros_like(re)
+        for i in range(4):
+            for j in range(4):
+                d = p[:, None, i] - q[None, :, j]
+                r2 = (d * d).sum(-1)
+                r = np.sqrt(r2)
+                dn = (d * n[ci][None]).sum(-1) if layer == 1 else \
+                    -(d * n[ri][:, None]).sum(-1)
+                val = ww[i] * ww[j] * dn / (r * r2)
+                ph = real(k) * r
+                re += val * (np.cos(ph) + ph * np.sin(ph))
+                im += val * (np.sin(ph) - ph * np.cos(ph))
+        f = g[ri][:, None] * g[ci][None] / (4 * real(np.pi))
+        return (re * f, im * f) if k else (re * f,)
+
+    err = np.zeros(2)
+    for ro, r, co, c in blocks:
+        ri, ci = rt.idx[ro:ro + r], rt.idx[co:co + c]
+        got = op.nearfield(ri, ci)
+        apart = ~(t[ri][:, None, :, None] == t[ci][None, :, None, :]).any(
+            axis=(2, 3))
+        want = entries(ri, ci, np.longdouble)
+        plain = entries(ri, ci, np.float64)
+        for part, a, b in zip((got.real, got.imag), want, plain):
+            # (pi rounded in both references, the same factor)
+            err += [float((((z - a) ** 2)[apart]).sum()) for z in (part, b)]
+    print("error against a product per value: %.3f" % np.sqrt(
+        err[0] / err[1]))
+    assert err[0] <= 1.1 * err[1]
