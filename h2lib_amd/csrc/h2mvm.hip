@@ -1121,28 +1121,27 @@ __global__ __launch_bounds__(NT) void couple_trans_wg(CNArgs a) {
   }
 }
 
-// Couplings computed in the product at interpolation order M = 5 (order 4:
-// couple_pairs64), one vector, for a symmetric block structure (row and column trees with the
-// same points, every admissible block (r, c) with its mirror (c, r), whose
-// coupling matrix is S_rc^T: the squared distances, and so the values of
-// 1/r or e^{ikr}/r, are the same bit for bit).  One wave per pair r > c
-// evaluates each value once for both blocks: lane l keeps the sums of row
-// points l and l + 64 (rank M^3 <= 128) of block (r, c), yt_r[i] += sum_j
-// S_ij xt_c[j], with the arithmetic and order of the per-block kernel
-// (the general loop), and the products S_ij xt_r[i]
-// of W columns at a time, whose sums over the rows, yt_c[j] += sum_i S_ij
+// Couplings computed in the product at interpolation order 5 (order 4:
+// couple_pairs64), one vector, for a symmetric block structure (row and
+// column trees with the same points, every admissible block (r, c) with its
+// mirror (c, r), whose coupling matrix is S_rc^T: the squared distances, and
+// so the values of 1/r or e^{ikr}/r, are the same bit for bit).  One wave per
+// pair r > c evaluates each value once for both blocks: lane l keeps the sums
+// of row points l and l + 64 (rank 125) of block (r, c), yt_r[i] += sum_j
+// S_ij xt_c[j], with the arithmetic and order of the per-block kernel (the
+// general loop), and the products S_ij xt_r[i] of W columns at a time, whose sums over the rows, yt_c[j] += sum_i S_ij
 // xt_r[i] for the mirror block, a butterfly over the lanes forms.  Half the
 // evaluations of the two blocks' waves.  C: Helmholtz (complex).
-template <int C, int M>
+template <int C>
 __global__ __launch_bounds__(NT) void couple_mf_pairs(CNArgs a,
                                                       const PairD *pairs,
                                                       uint32_t npair) {
   constexpr double KCONST = 0.0795774715459476679;
-  constexpr int R = M * M * M, RH = (R + 63) / 64;
+  constexpr int M = 5, R = M * M * M, RH = (R + 63) / 64;
   // columns per butterfly: the products of a pass stay in registers until
   // then (fewer for the complex values, whose sine and cosine take the
   // registers)
-  constexpr int W = C ? (RH > 1 ? 2 : 4) : 16;
+  constexpr int W = C ? 2 : 16;
   constexpr int NP = (R + W - 1) / W;
   __shared__ double xs_all[WPB][2 * R];
   const uint32_t w = blockIdx.x * WPB + (threadIdx.x >> 6);
@@ -3007,7 +3006,7 @@ void launch(const VecSet &vs, const h2hip_h2matrix *H, double *xt, double *yt,
                  c.nnear == 0 && !ord;
       const dim3 gp((H->npair + WPB - 1) / WPB);
       if (paired)
-        hipLaunchKernelGGL((couple_mf_pairs<C, 5>), gp, dim3(NT), 0, st, c,
+        hipLaunchKernelGGL((couple_mf_pairs<C>), gp, dim3(NT), 0, st, c,
                            (const PairD *)H->d_pairs.p, H->npair);
       else if (ord)
         hipLaunchKernelGGL((couple_near<C, false, NV, true, true>), gc,

@@ -384,8 +384,9 @@ class H2Matrix:
         return int(hip().h2hip_h2matrix_coupling_pairs(self._h))
 
     def bytes(self):
-        """Bytes one product y += alpha H x reads in the current schedule
-        and coupling mode (couplings 0 when computed in the product)."""
+        """Bytes of one product y += alpha H x in the current schedule and
+        coupling mode (couplings 0 when computed in the product; those of
+        both blocks of a mirrored pair, though one is read)."""
         out = np.zeros(3, dtype=np.uint64)
         check(hip().h2hip_h2matrix_bytes(self._h, _ptr(out)),
               "h2hip_h2matrix_bytes")

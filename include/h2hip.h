@@ -159,7 +159,13 @@ int h2hip_nearfield_flush(const h2hip_op *op);
  * bem->nearfield for every inadmissible leaf block.  Where both sides have
  * one basis and equal index arrays and every block comes with its mirror
  * (cols x rows), the default schedule evaluates each pair of triangles once
- * for both entries. */
+ * for both entries.  Not the FP64 double layers on a surface that folds back
+ * on itself anywhere (two triangles with a common vertex and normals within
+ * 18 degrees of opposite) or whose normals are not perpendicular to the
+ * triangles to rounding: these keep a product <x - y, n> per value and one
+ * evaluation per entry.  Both hold for a surface as a whole, as does the
+ * choice of the Helmholtz kernels without argument reduction by its longest
+ * edge, also where it joins several meshes. */
 int h2hip_nfplan_create(h2hip_nfplan **out, const h2hip_surface *s,
                         int row_basis, int col_basis,
                         const uint32_t *ridx_all, uint32_t nridx,
@@ -185,8 +191,10 @@ int h2hip_nfplan_set_schedule(h2hip_nfplan *p, int sorted, int persistent);
  * its LDS accumulator before the tile is stored, so one launch (one
  * workgroup per tile, or the persistent grid when persistent = 1) assembles
  * every block, tiles taken by decreasing total work; no global atomics.
- * Applies to regular order 2 with singular order 4 (other orders keep the
- * launches per rule class).  Same entries up to the order of the sums. */
+ * Applies to regular order 2 with singular order 4; other orders, and FP64
+ * double layers on folded surfaces or with other normals (see
+ * h2hip_nfplan_create), keep the launches per rule class, which are the
+ * faster way there.  Same entries up to the order of the sums. */
 int h2hip_nfplan_set_fused(h2hip_nfplan *p, int fused);
 /* Tile edge of the plan (8..64 DOFs, default 64; no counterpart in the
  * reference): the blocks are cut again into tiles of at most tile x tile
@@ -267,8 +275,10 @@ int h2hip_h2matrix_set_mfma(h2hip_h2matrix *H, int on);
  * mesh: the products use each coupling value once for both blocks of a pair
  * (on = 1, the default; no counterpart in the reference): order 4, read
  * (h2hip_h2matrix_interp_couplings) or computed in the product (coupling
- * mode 1), forward and adjoint, of one or several vectors; order 5,
- * computed, forward, one vector.  Reproducible mode, the adjoint from kept
+ * mode 1), forward and adjoint, of one or several vectors, where there are
+ * enough pairs to fill the device (64 to 2048, by schedule and vectors;
+ * small matrices are faster block by block); order 5, computed, forward, one
+ * vector.  Reproducible mode, the adjoint from kept
  * transposes, products on matrix cores and forward products of more than
  * four complex vectors with read couplings keep one evaluation per block. */
 int h2hip_h2matrix_set_coupling_pairs(h2hip_h2matrix *H, int on);
@@ -309,14 +319,15 @@ int h2hip_addevalsymm_h2matrix(const double *alpha, const h2hip_h2matrix *H,
  * thread-safe against products in flight.  No counterpart in the
  * reference. */
 int h2hip_h2matrix_set_schedule(h2hip_h2matrix *H, int level_sync);
-/* Couplings of the products y += alpha H x (h2hip_addeval_h2matrix and
- * h2hip_addeval_h2matrix_batch, not transposed): recompute = 0 reads the
- * stored couplings, 1 computes each entry in the product from the
- * interpolation points kept by h2hip_h2matrix_interp_couplings (the same
- * arithmetic, so the same values), which trades the product's largest read
+/* Couplings of the products y += alpha H x and y += alpha H^* x
+ * (h2hip_addeval_h2matrix, h2hip_addevaltrans_h2matrix and
+ * h2hip_addeval_h2matrix_batch): recompute = 0 reads the stored couplings, 1
+ * computes each entry in the product from the interpolation points kept by
+ * h2hip_h2matrix_interp_couplings (the same arithmetic, up to where the
+ * constant 1/(4 pi) is applied), which trades the product's largest read
  * (k^2 doubles per admissible block) for k^2 kernel evaluations, shared by
- * all vectors of a batched product.  Transposed and self-adjoint products
- * keep reading the stored couplings.  Needs couplings set by
+ * all vectors of a batched product.  Self-adjoint products keep reading the
+ * stored couplings.  Needs couplings set by
  * h2hip_h2matrix_interp_couplings; h2hip_h2matrix_set_couplings switches
  * back to 0.  h2hip_h2matrix_bytes then counts no coupling bytes.  No
  * counterpart in the reference. */
