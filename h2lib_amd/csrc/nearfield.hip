@@ -767,6 +767,11 @@ int execute(const h2hip_op *op, const h2hip_nfplan *P, int far, void *d_out,
     return H2HIP_EINVAL;
   }
   if (P->tiles.empty()) return H2HIP_OK;
+  if (!P->d_lists.p) {
+    // a new tiling whose lists did not fit, nor the previous one's again
+    set_error("h2hip_nearfield_execute: the plan has no device lists");
+    return H2HIP_ENOMEM;
+  }
   const h2hip_surface *s = op->s;
   nf::KArgs a;
   a.tiles = P->sorted ? P->d_tiles_s.p : P->d_tiles;
@@ -1577,8 +1582,9 @@ int h2hip_nfplan_set_fused(h2hip_nfplan *p, int fused) {
     std::stable_sort(tf.begin(), tf.end(), [&](const Tile &x, const Tile &y) {
       return work(x) > work(y);
     });
-    H2HIP_CHECK(p->d_tiles_f.upload(tf.data(), tf.size()));
+    // (the tiles last: they mark the lists as made)
     H2HIP_CHECK(p->d_tpairs.upload(tpairs.data(), tpairs.size()));
+    H2HIP_CHECK(p->d_tiles_f.upload(tf.data(), tf.size()));
   }
   p->fused = fused;
   return H2HIP_OK;

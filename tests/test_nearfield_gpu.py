@@ -217,6 +217,41 @@ def test_deferred_blocks_across_pieces():
         assert np.all(big[wr:] == 7.0) and np.all(big[:, wc:] == 7.0)
 
 
+@pytest.mark.parametrize("layer", [0, 1])
+def test_vertex_of_many_triangles(layer):
+    # a tile whose 300 triangles all touch has 90000 pairs with common
+    # vertices, more than the 16-bit counts of the fused lists: the launches
+    # per rule class take them, the fused schedule refuses and leaves the plan
+    # as it was
+    import h2lib_amd as h
+    m = 300
+    ang = 2.0 * np.pi * np.arange(m) / m
+    x = np.concatenate([[[0.0, 0.0, 0.3]], np.stack(
+        [np.cos(ang), np.sin(ang), 0.1 * np.cos(5 * ang)], 1)])
+    t = np.array([(0, 1 + i, 1 + (i + 1) % m) for i in range(m)],
+                 dtype=np.uint32)
+    gr = h.Surface3d(x, t)
+    op = h.Bem3d(gr, 0, layer, 2, 4, 1, 1, alpha=0.5 if layer else 0.0)
+    orc = OracleBem(0, layer, 1, 1, x, t, q=2, q2=4,
+                    alpha=0.5 if layer else 0.0)
+    idx = np.arange(m + 1, dtype=np.uint32)
+    blocks = [(0, 40, 0, 40), (0, 40, 40, 70), (40, 70, 0, 40)]
+    plan = h.NearfieldPlan(gr, 1, 1, idx, idx, blocks)
+    stream = h.Stream()
+    for fused in (0, 1):
+        if fused:
+            with pytest.raises(h.H2HipError):
+                plan.set_schedule(0, 0, 1)
+        out = h.DeviceArray(plan.entries, op.dtype)
+        out.fill_nan()
+        plan.execute(op, out.ptr, stream.handle)
+        stream.sync()
+        flat = out.download()
+        for b, (ro, r, co, c) in enumerate(blocks):
+            ref = orc.nearfield(idx[ro:ro + r], idx[co:co + c])
+            assert rel_block_err(plan.block(flat, b), ref) < TOL, (fused, b)
+
+
 @pytest.mark.parametrize("q,q2", [(1, 3), (3, 5), (4, 6)])
 def test_other_orders(q, q2, sphere4):
     for name in ("lap_slp_cc", "helm_dlp_ll", "lap_dlp_cl", "lap_adlp_lc"):
