@@ -762,9 +762,10 @@ __device__ __forceinline__ void near_adjoint64(const CNArgs &a,
 // yt_r += S_rc xt_c and y|_r += alpha N_rc x|_c; TRANS: yt_c += S^* xt_r and
 // y|_c += alpha N^* x|_r.  One wave per block; the wave first gathers its
 // block's input entries into its own LDS slice.
-// MF (not transposed): the couplings are computed from the interpolation
-// points instead of read (cpl_value), lane i keeping row point i and
-// stepping through the column points j = (ja m + jb) m + jc; each value
+// MF: the couplings are computed from the interpolation points instead of
+// read (cpl_value; complex matrices: Helmholtz, real ones: Laplace, which
+// h2hip_h2matrix_interp_couplings makes sure of), lane i keeping row point i
+// and stepping through the column points j = (ja m + jb) m + jc; each value
 // serves all NV vectors.
 // Item w of the wave (w < nfar: far block w, else near block w - nfar);
 // xs: the wave's LDS slice of NV * 2 * XR doubles.  PF: near blocks of one
@@ -809,7 +810,7 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
         const uint32_t ia = i / (m * m), ib = (i / m) % m, ic = i % m;
         const double qx = pc[ia], qy = pc[m + ib], qz = pc[2 * m + ic];
         uint32_t j = 0;
-        if (m == 4 && !a.cs.helmholtz) {  // uniform over the grid
+        if (!C && m == 4) {  // uniform over the grid
           const double p3[3] = {qx, qy, qz};
           mf_laplace4<C, NV, XR>(p3, pr, -1.0, xs, ar, ai);
           m4 = true;
@@ -820,7 +821,7 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
             const double d1 = pr[m + jb] - qy;
             for (uint32_t jc = 0; jc < m; jc++, j++) {
               double sr, si;
-              cpl_value(d0, d1, pr[2 * m + jc] - qz, a.cs.helmholtz,
+              cpl_value(d0, d1, pr[2 * m + jc] - qz, C,
                         a.cs.kr, a.cs.kdamp, sr, si);
               si = -si;
 #pragma unroll
@@ -843,7 +844,7 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
         const uint32_t ia = i / (m * m), ib = (i / m) % m, ic = i % m;
         const double px = pr[ia], py = pr[m + ib], pz = pr[2 * m + ic];
         uint32_t j = 0;
-        if (m == 4 && !a.cs.helmholtz) {  // uniform over the grid
+        if (!C && m == 4) {  // uniform over the grid
           const double p3[3] = {px, py, pz};
           mf_laplace4<C, NV, XR>(p3, pc, 1.0, xs, ar, ai);
           m4 = true;
@@ -854,7 +855,7 @@ __device__ __forceinline__ void couple_near_dev(const CNArgs &a, uint32_t w,
             const double d1 = py - pc[m + jb];
             for (uint32_t jc = 0; jc < m; jc++, j++) {
               double sr, si;
-              cpl_value(d0, d1, pz - pc[2 * m + jc], a.cs.helmholtz, a.cs.kr,
+              cpl_value(d0, d1, pz - pc[2 * m + jc], C, a.cs.kr,
                         a.cs.kdamp, sr, si);
 #pragma unroll
               for (int v = 0; v < NV; v++) {
@@ -2750,12 +2751,16 @@ void launch(const VecSet &vs, const h2hip_h2matrix *H, double *xt, double *yt,
   // each value once for a block and its mirror, where there are enough of
   // them (several vectors keep the matrix cores where they are asked for; more
   // than four complex vectors with read couplings, forward, keep a wave per
-  // block: 259 us against 279 for eight at 12800 triangles)
+  // block: 259 us against 279 for eight at 12800 triangles; so do more than
+  // six with computed ones where there are many pairs: eight, 32768
+  // triangles, 568 us against 644, 4608 triangles 114 against 109; five 295
+  // against 285 at 20000)
   const bool pairs64 = !symm && !ord && !tv && H->pairs_on && H->npair &&
                        H->cpl_known && H->cpl.m == 4 &&
                        H->npair >= pairs_from<C, NV>(flat, trans, mf, twg) &&
                        (NV == 1 || C || mf || !H->cpl_mfma || trans) &&
-                       !(C && NV > 4 && !mf && !trans);
+                       !(C && NV > 4 && !mf && !trans) &&
+                       !(C && mf && vs.nv > 6 && H->npair >= 1536);
   // the near blocks of a flat, not symmetric product run with the computed
   // complex pairs or in the upward launch (not the workgroup adjoint blocks
   // of several vectors, fixed-order sums or few real blocks: 196 far blocks
