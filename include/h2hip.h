@@ -279,8 +279,9 @@ int h2hip_h2matrix_set_mfma(h2hip_h2matrix *H, int on);
  * enough pairs to fill the device (64 to 2048, by schedule and vectors;
  * small matrices are faster block by block); order 5, computed, forward, one
  * vector.  Reproducible mode, the adjoint from kept
- * transposes, products on matrix cores and forward products of more than
- * four complex vectors with read couplings keep one evaluation per block. */
+ * transposes, products on matrix cores, forward products of more than four
+ * complex vectors with read couplings and products of more than six with
+ * many computed ones keep one evaluation per block. */
 int h2hip_h2matrix_set_coupling_pairs(h2hip_h2matrix *H, int on);
 /* The number of mirrored pairs found by h2hip_h2matrix_interp_couplings
  * (0: the structure is not symmetric, or not order 4 or 5; -1: H null). */
